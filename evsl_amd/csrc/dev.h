@@ -87,7 +87,9 @@ enum Mode { kPlain = 0, kCheb = 1, kKpm = 2, kRes = 3 };
 //             yflush 3: y += s[c-2B]*xkm1, then += s[c-B]*xk, then += s[c]*w
 //             yflush 2: y += s[c-B]*xk, then += s[c]*w;  1: y += s[c]*w
 //             yflush 0: y untouched (neither read nor written)
-//   kKpm  : w as kCheb; xkp1 = w; part[blk*B + c] = sum_rows w*v0
+//   kKpm  : w as kCheb; xkp1 = w; the block's dots of W = kpm_dots values:
+//           FP64 part[blk*W + c] = sum_rows w*w, part[blk*W + B + c] =
+//           sum_rows w*xk (v0 unused); FP32 part[blk*W + c] = sum_rows w*v0
 //   kRes  : w = t*(acc - cc*xk) - xkm1 + s[c]*v0 (v0 = residual block R);
 //           xkp1 = w; y as kCheb with coefficients mu0[0] (this degree),
 //           mu0[-2], mu0[-4] (the two before) and mu0[1] for xk when first
@@ -205,11 +207,35 @@ int cheb_spmm_nblk(const Csr& A, int B, bool fp32, Mode mode);
 // instance (k_cheb_spmm<..., NT = true>)
 bool cheb_spmm_streaming(const Csr& A, int B, bool fp32, Mode mode);
 
+// KPM dots.  With T_a(x) T_b(x) = (T_{a+b}(x) + T_{|a-b|}(x)) / 2, the vectors
+// T_j v and T_{j-1} v give two moments at once,
+//   v.T_{2j} v = 2 T_j v.T_j v - v.v,  v.T_{2j-1} v = 2 T_j v.T_{j-1} v - v.T_1 v,
+// so an FP64 series of Mdeg moments runs (Mdeg + 1) / 2 steps, and both
+// factors are in registers where T_j v is formed (v itself is not read).
+// Measured, 300 moments: 40 vectors on the 100^3 Laplacian 104.0 -> 48.3 ms
+// (half the steps, three vector streams instead of four), 60 on a 100^2 grid
+// 12.4 -> 4.2 ms (with the sums of kKpmSumDegrees degrees in one launch).  The FP32
+// recurrence of the mixed form keeps v.T_k v at every step: its moments carry
+// the recurrence's FP32 rounding, which the products would change.
+constexpr int kpm_dots(int B, bool fp32) { return fp32 ? B : 2 * B; }
+// steps of a series of Mdeg moments
+inline int kpm_steps(int Mdeg, bool fp32) { return fp32 ? Mdeg : (Mdeg + 1) / 2; }
+// degrees whose block partials are kept and then summed by one launch: the
+// sums of one degree are a launch or two of 5-7 us beside a step of 5 us at
+// n = 10^4.  At most kKpmSumDegrees, fewer where the partials of one degree
+// (nblk * W values) are large.
+constexpr int kKpmSumDegrees = 16;
+inline int kpm_sum_degrees(size_t part_values) {
+  const size_t d = ((size_t)4 << 20) / (part_values ? part_values : 1);
+  return d < 1 ? 1 : d > kKpmSumDegrees ? kKpmSumDegrees : (int)d;
+}
+
 // One matrix of a grouped KPM launch (a device-resident table entry): its
 // CSR (int32 column indices), its row-block table for the launch's lane
 // layout ((row, ia[row]) pairs), the start block v0 and the ring of three
 // T_k blocks (n x B interleaved, element type of the launch), the block
-// partials of the moment dots, and the recurrence
+// partials of the moment dots (part_step values for each of the degrees that
+// are summed together), and the recurrence
 // T_{k+1} = t (A - cc I) T_k - T_{k-1} with factor t0 at k = 0.  A launch
 // at step k advances this matrix's recurrence at its own step k - k0.
 struct KpmGroupEntry {
@@ -222,7 +248,7 @@ struct KpmGroupEntry {
   double* part;
   double t0, t, cc;
   int n, blk0;  // rows; first global row block of this matrix
-  int k0, pad;
+  int k0, part_step;
 };
 // One column block of a grouped ChebAv launch (a device table entry): its
 // matrix's CSR (16-bit column offsets jd when the launch's instance reads
@@ -253,9 +279,10 @@ struct ChebGroupEntry {
 hipError_t cheb_group_step(bool fp32, int B, bool i16, const ChebGroupEntry* tab,
                            const int* owner, int total, int k, hipStream_t st);
 
-// The partial sums of one grouped matrix: nblk block partials (B per block)
-// summed as sum_block_partials does (G first-level blocks into scratch, then
-// one; or directly when G == 1) into dots + (k+1)*B.
+// The partial sums of one grouped matrix: nblk block partials (W = kpm_dots
+// per block) of each of nd degrees, summed as sum_block_partials does (G
+// first-level blocks into scratch, then one; or directly when G == 1) into
+// dots + (k+1)*W.
 struct KpmSumEntry {
   const double* part;
   double* scratch;
@@ -264,23 +291,27 @@ struct KpmSumEntry {
   int k0, pad;
 };
 // One grouped KPM step k over `total` row blocks (owner[gb] = entry of row
-// block gb) at block width B (lane layout of the kKpm policy), then its
-// partial sums: level 1 over nl1 blocks (owner1/first1), level 2 over the
-// two-level entries listed in owner2.
+// block gb) at block width B (lane layout of the kKpm policy), its partials
+// at place d of the degrees that are summed together
 hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int* owner,
-                          int total, int k, const KpmSumEntry* sums, const int* owner1,
-                          const int* first1, int nl1, const int* owner2, int nl2,
-                          hipStream_t st);
+                          int total, int k, int d, hipStream_t st);
+// the partial sums of the steps k .. k + nd - 1 (places 0 .. nd - 1): level 1
+// over nl1 blocks (owner1/first1), level 2 over the two-level entries listed
+// in owner2
+hipError_t kpm_group_sums(bool fp32, int B, const KpmSumEntry* sums, int k, int nd,
+                          const int* owner1, const int* first1, int nl1, const int* owner2,
+                          int nl2, hipStream_t st);
 
-// out[c] = sum_b part[b*B + c] over nblk row blocks, in a fixed order; uses
-// scratch (>= kSumScratch doubles) for a first level when nblk is large
-constexpr int kSumScratch = 256 * 32;
-// first-level blocks of sum_block_partials for (nblk, B): 1 when it sums
-// directly, else kSumScratch / 32
-inline int sum_levels_blocks(int nblk, int B) {
-  return ((size_t)nblk * B <= 16384) ? 1 : kSumScratch / 32;
+// out[d*W + c] = sum_b part[(d*nblk + b)*W + c] over nblk row blocks, in a
+// fixed order, for nd consecutive degrees d in one launch; uses scratch (nd *
+// kSumScratch doubles) for a first level when nblk is large
+constexpr int kSumScratch = 256 * 64;
+// first-level blocks of sum_block_partials for (nblk, W): 1 when it sums
+// directly, else 256
+inline int sum_levels_blocks(int nblk, int W) {
+  return ((size_t)nblk * W <= 16384) ? 1 : 256;
 }
-hipError_t sum_block_partials(const double* part, int nblk, int B, double* out,
+hipError_t sum_block_partials(const double* part, int nblk, int W, int nd, double* out,
                               double* scratch, hipStream_t st);
 
 // Fixed-grid reductions: partial buffers hold kRedBlocks entries.

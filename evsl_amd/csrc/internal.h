@@ -146,8 +146,6 @@ int apply_A(const double* x, double* y);
 // device scratch for reductions (>= kRedBlocks * 64 doubles, plus scalars)
 double* red_part();
 double* red_scalar(int i);
-// kSumScratch doubles at the end of the reduction scratch (two-level sums)
-double* red_scratch();
 // copy cnt doubles from device to the pinned host buffer and wait
 int read_scalars(const double* d, int cnt, double* out);
 
@@ -312,6 +310,10 @@ struct GroupedWork {
 // Each column gets the bits of its one-matrix filter.
 int grouped_filter(const std::vector<GroupedCols>& parts, GroupedWork& W);
 
+// raw[k] (k >= 1) += the B columns' v^T T_k v from the dots of a series in the
+// order sum_block_partials leaves them (row j: the W = kpm_dots values of
+// step j - 1)
+void kpm_add_dots(int Mdeg, bool f32, int B, const double* dots, double* raw);
 // KPM moments and eigenvalue count from raw[k] = sum over the nvec vectors of
 // v^T T_k(A~) v (k >= 1), as kpmdos finishes them
 void kpm_moments(int Mdeg, int damping, int nvec, const double* intv, int n, const double* raw,

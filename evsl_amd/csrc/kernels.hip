@@ -51,7 +51,7 @@ __device__ __forceinline__ double block_sum(double v, double* sh /*>=4*/) {
 template <typename VT, int B, int V>
 __global__ __launch_bounds__(kWG) void k_kpm_group(const KpmGroupEntry* __restrict__ tab,
                                                    const int* __restrict__ owner, int total,
-                                                   int k) {
+                                                   int k, int d) {
   const int gb = xcd_remap(blockIdx.x, total);
   const KpmGroupEntry& e = tab[owner[gb]];
   k -= e.k0;  // this matrix's own step
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kWG) void k_kpm_group(const KpmGroupEntry* __restri
   cheb_spmm_block<VT, B, V, kKpm, true, 0, false>(
       gb - e.blk0, e.ia, e.ja, nullptr, static_cast<const VT*>(e.a),
       reinterpret_cast<const int2*>(e.rbp), xk, xkm1, xkp1, nullptr, x0, nullptr, nullptr,
-      k == 0 ? e.t0 : e.t, e.cc, 0, 0, e.part);
+      k == 0 ? e.t0 : e.t, e.cc, 0, 0, e.part + (size_t)d * e.part_step);
 }
 
 // the y-flush schedule of evsl_dev::y_flush, for the grouped launch (each
@@ -125,32 +125,38 @@ __device__ __forceinline__ void sum_partials_block(const double* __restrict__ pa
   }
 }
 
+// blockIdx.y: the degree, whose partials and sums follow the previous one's
 __global__ __launch_bounds__(kWG) void k_sum_block_partials(const double* __restrict__ part,
                                                             int nblk, int B,
                                                             double* __restrict__ out) {
   __shared__ double s_red[kWG];
-  sum_partials_block(part, nblk, B, out, blockIdx.x, gridDim.x, s_red);
+  const size_t d = blockIdx.y;
+  sum_partials_block(part + d * nblk * B, nblk, B, out + d * gridDim.x * B, blockIdx.x,
+                     gridDim.x, s_red);
 }
 
-// The partial sums of a grouped KPM step, per matrix in the order of
-// sum_block_partials: level 1 runs entry owner[blockIdx] as block
-// blockIdx - first[owner] of its G; level 2 sums the G first-level values of
-// each two-level entry.
+// The partial sums of grouped KPM steps k + blockIdx.y, per matrix in the
+// order of sum_block_partials: level 1 runs entry owner[blockIdx.x] as block
+// blockIdx.x - first[owner] of its G; level 2 sums the G first-level values
+// of each two-level entry.
 __global__ __launch_bounds__(kWG) void k_kpm_group_sums(const KpmSumEntry* __restrict__ tab,
                                                         const int* __restrict__ owner,
                                                         const int* __restrict__ first, int B,
                                                         int k, int level) {
   __shared__ double s_red[kWG];
   const int r = owner[blockIdx.x];
+  const size_t d = blockIdx.y;
   const KpmSumEntry& e = tab[r];
-  double* out = e.dots + (size_t)(k - e.k0 + 1) * B;
+  const double* part = e.part + d * e.nblk * B;
+  double* scratch = e.scratch + d * e.G * B;
+  double* out = e.dots + (size_t)(k + (int)d - e.k0 + 1) * B;
   if (level == 1) {
     if (e.G == 1)
-      sum_partials_block(e.part, e.nblk, B, out, 0, 1, s_red);
+      sum_partials_block(part, e.nblk, B, out, 0, 1, s_red);
     else
-      sum_partials_block(e.part, e.nblk, B, e.scratch, blockIdx.x - first[r], e.G, s_red);
+      sum_partials_block(part, e.nblk, B, scratch, blockIdx.x - first[r], e.G, s_red);
   } else {
-    sum_partials_block(e.scratch, e.G, B, out, 0, 1, s_red);
+    sum_partials_block(scratch, e.G, B, out, 0, 1, s_red);
   }
 }
 
@@ -1146,13 +1152,11 @@ hipError_t cheb_spmm(const Csr& A, int B, bool fp32, Mode mode, const void* xk,
 }
 
 hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int* owner,
-                          int total, int k, const KpmSumEntry* sums, const int* owner1,
-                          const int* first1, int nl1, const int* owner2, int nl2,
-                          hipStream_t st) {
-  if (total <= 0 || nl1 <= 0) return hipErrorInvalidValue;
+                          int total, int k, int d, hipStream_t st) {
+  if (total <= 0 || d < 0) return hipErrorInvalidValue;
 #define EVSL_KPM_GROUP(VT_, B_)                                                           \
   hipLaunchKernelGGL((k_kpm_group<VT_, B_, SpmmPolicy<VT_, B_, kKpm>::V>), dim3(total),   \
-                     dim3(kWG), 0, st, tab, owner, total, k)
+                     dim3(kWG), 0, st, tab, owner, total, k, d)
 #define EVSL_KPM_GROUP_B(VT_)                  \
   switch (B) {                                 \
     case 1: EVSL_KPM_GROUP(VT_, 1); break;     \
@@ -1170,25 +1174,32 @@ hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int*
   }
 #undef EVSL_KPM_GROUP_B
 #undef EVSL_KPM_GROUP
-  hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl1), dim3(kWG), 0, st, sums, owner1, first1, B, k,
-                     1);
-  if (nl2 > 0)
-    hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl2), dim3(kWG), 0, st, sums, owner2,
-                       (const int*)nullptr, B, k, 2);
   return hipGetLastError();
 }
 
-hipError_t sum_block_partials(const double* part, int nblk, int B, double* out,
+hipError_t kpm_group_sums(bool fp32, int B, const KpmSumEntry* sums, int k, int nd,
+                          const int* owner1, const int* first1, int nl1, const int* owner2,
+                          int nl2, hipStream_t st) {
+  if (nl1 <= 0 || nd <= 0) return hipErrorInvalidValue;
+  const int W = kpm_dots(B, fp32);
+  hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl1, nd), dim3(kWG), 0, st, sums, owner1, first1, W,
+                     k, 1);
+  if (nl2 > 0)
+    hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl2, nd), dim3(kWG), 0, st, sums, owner2,
+                       (const int*)nullptr, W, k, 2);
+  return hipGetLastError();
+}
+
+hipError_t sum_block_partials(const double* part, int nblk, int W, int nd, double* out,
                               double* scratch, hipStream_t st) {
-  if (B < 1 || B > 32) return hipErrorInvalidValue;
-  const int G = kSumScratch / 32;  // first-level blocks (<= 256)
-  if (sum_levels_blocks(nblk, B) == 1 || !scratch) {
-    hipLaunchKernelGGL(k_sum_block_partials, dim3(1), dim3(kWG), 0, st, part, nblk, B, out);
-  } else {
-    hipLaunchKernelGGL(k_sum_block_partials, dim3(G), dim3(kWG), 0, st, part, nblk, B, scratch);
-    hipLaunchKernelGGL(k_sum_block_partials, dim3(1), dim3(kWG), 0, st,
-                       (const double*)scratch, G, B, out);
-  }
+  if (W < 1 || W > 64 || nd < 1) return hipErrorInvalidValue;
+  const int G = sum_levels_blocks(nblk, W);
+  if (G > 1 && !scratch) return hipErrorInvalidValue;
+  double* first = G > 1 ? scratch : out;
+  hipLaunchKernelGGL(k_sum_block_partials, dim3(G, nd), dim3(kWG), 0, st, part, nblk, W, first);
+  if (G > 1)
+    hipLaunchKernelGGL(k_sum_block_partials, dim3(1, nd), dim3(kWG), 0, st,
+                       (const double*)first, G, W, out);
   return hipGetLastError();
 }
 

@@ -187,18 +187,25 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
     std::vector<evsl_dev::KpmSumEntry> sums(nreq);
     std::vector<int> owner, owner1, first1(nreq), owner2;
     int total = 0;
+    // values per block partial, steps, and the degrees summed by one launch
+    const int W = evsl_dev::kpm_dots(B, f32), steps = evsl_dev::kpm_steps(Mdeg, f32);
+    size_t pv = 0;
+    for (int r = 0; r < nreq; ++r) {
+      if (int e = req[r].mat->ensure_table(lanes)) return e;
+      pv = std::max(pv, (size_t)req[r].mat->nblk[lanes] * W);
+    }
+    const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
     for (int r = 0; r < nreq; ++r) {
       BatchRequest& q = req[r];
       BatchMatrix& m = *q.mat;
-      if (int e = m.ensure_table(lanes)) return e;
       const int nblk = m.nblk[lanes];
       const size_t nb = (size_t)m.n * B;
       EVSL_HIP(q.x0.alloc(nb * vs));
       EVSL_HIP(q.ring.alloc(3 * nb * vs));
-      EVSL_HIP(q.part.alloc((size_t)std::max(nblk, 1) * B * sizeof(double)));
-      EVSL_HIP(q.dots.alloc((size_t)(Mdeg + 1) * B * sizeof(double)));
-      const int G = evsl_dev::sum_levels_blocks(nblk, B);
-      if (G > 1) EVSL_HIP(q.scratch.alloc((size_t)G * B * sizeof(double)));
+      EVSL_HIP(q.part.alloc((size_t)nd * std::max(nblk, 1) * W * sizeof(double)));
+      EVSL_HIP(q.dots.alloc((size_t)(steps + 1) * W * sizeof(double)));
+      const int G = evsl_dev::sum_levels_blocks(nblk, W);
+      if (G > 1) EVSL_HIP(q.scratch.alloc((size_t)nd * G * W * sizeof(double)));
       // start block: the kpmdos_ex vectors of this request's seed, unit columns
       double* xd = f32 ? x64.as<double>() : q.x0.as<double>();
       EVSL_HIP(evsl_dev::rm_random(m.n, B, vec_kind == EVSL_VEC_RADEMACHER ? 0 : 1, q.seed, done,
@@ -221,7 +228,7 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       e.n = m.n;
       e.blk0 = total;
       e.k0 = 0;
-      e.pad = 0;
+      e.part_step = nblk * W;
       owner.insert(owner.end(), nblk, r);
       total += nblk;
       evsl_dev::KpmSumEntry& s = sums[r];
@@ -245,22 +252,26 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
     double step_bytes = 0.0;
     for (int r = 0; r < nreq; ++r)
       step_bytes += (double)req[r].mat->nnz * (vs + 4) + 4.0 * (req[r].mat->n + 1) +
-                    4.0 * req[r].mat->n * B * vs;
-    for (int k = 0; k < Mdeg; ++k) {
-      EVSL_HIP(evsl_dev::kpm_group_step(
-          f32, B, d_tab.as<evsl_dev::KpmGroupEntry>(), d_owner.as<int>(), total, k,
-          d_sums.as<evsl_dev::KpmSumEntry>(), d_owner1.as<int>(), d_first1.as<int>(),
-          (int)owner1.size(), d_owner2.as<int>(), (int)owner2.size(), c.stream));
+                    (f32 ? 4.0 : 3.0) * req[r].mat->n * B * vs;
+    for (int k = 0; k < steps; ++k) {
+      EVSL_HIP(evsl_dev::kpm_group_step(f32, B, d_tab.as<evsl_dev::KpmGroupEntry>(),
+                                        d_owner.as<int>(), total, k, k % nd, c.stream));
+      if ((k + 1) % nd == 0 || k + 1 == steps) {
+        const int have = k % nd + 1;
+        EVSL_HIP(evsl_dev::kpm_group_sums(f32, B, d_sums.as<evsl_dev::KpmSumEntry>(),
+                                          k + 1 - have, have, d_owner1.as<int>(),
+                                          d_first1.as<int>(), (int)owner1.size(),
+                                          d_owner2.as<int>(), (int)owner2.size(), c.stream));
+      }
       c.astats.filter_bytes += step_bytes;
     }
-    c.astats.n_filter_steps += Mdeg;
-    c.astats.n_filter_cols += (size_t)Mdeg * B * nreq;
-    hdots.resize((size_t)(Mdeg + 1) * B);
+    c.astats.n_filter_steps += steps;
+    c.astats.n_filter_cols += (size_t)steps * B * nreq;
+    hdots.resize((size_t)(steps + 1) * W);
     for (int r = 0; r < nreq; ++r) {
       EVSL_HIP(hipMemcpy(hdots.data(), req[r].dots.p, hdots.size() * sizeof(double),
                          hipMemcpyDeviceToHost));
-      for (int k = 1; k <= Mdeg; ++k)
-        for (int col = 0; col < B; ++col) req[r].raw[k] += hdots[(size_t)k * B + col];
+      kpm_add_dots(Mdeg, f32, B, hdots.data(), req[r].raw.data());
     }
     done += B;
   }

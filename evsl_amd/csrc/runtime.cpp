@@ -332,19 +332,18 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
     }
     EVSL_HIP(hipMalloc((void**)&M.rb[w], rbp.size() * sizeof(int)));
     EVSL_HIP(hipMemcpy(M.rb[w], rbp.data(), rbp.size() * sizeof(int), hipMemcpyHostToDevice));
-    need = std::max(need, (size_t)(M.nblk[w] + 1) * B);
+    need = std::max(need, (size_t)(M.nblk[w] + 1) * 2 * B);  // kpm_dots in FP64
   }
-  // reduction scratch: the largest per-row-block partial buffer, the
-  // first-level sums behind it, and one partial per 256 rows
+  // reduction scratch: the largest per-row-block partial buffer and one
+  // partial per 256 rows
   *red_need = std::max(need, (size_t)n / evsl_dev::kWG + 1);
   return 0;
 }
 
-// the context's reduction scratch holds at least `need` doubles (plus the
-// first-level sums behind them)
+// the context's reduction scratch holds at least `need` doubles
 int ensure_red_part(size_t need) {
   Context& c = g_ctx;
-  const size_t bytes = (need + evsl_dev::kSumScratch) * sizeof(double);
+  const size_t bytes = need * sizeof(double);
   if (c.red_part.bytes >= bytes) return 0;
   EVSL_HIP(c.red_part.alloc(bytes));
   return 0;
@@ -425,10 +424,6 @@ int make_filter_op(double cc, double dd, bool f32, FilterOp* op) {
   op->A.pval32 = c.A.pval32;  // made with a32 (the view above predates them)
   op->A.dg32 = c.A.dg32;
   return 0;
-}
-
-double* red_scratch() {
-  return g_ctx.red_part.as<double>() + (g_ctx.red_part.bytes / sizeof(double) - evsl_dev::kSumScratch);
 }
 
 }  // namespace evsl
@@ -594,8 +589,8 @@ int SetAMatvec(int n, MVFunc func, void* data) {
   c.A.release();
   c.n = n;
   c.op = 2;
-  EVSL_HIP(c.red_part.alloc(((size_t)evsl_dev::kRedBlocks * 64 + (size_t)n / evsl_dev::kWG + 1 +
-                             evsl_dev::kSumScratch) * sizeof(double)));
+  EVSL_HIP(c.red_part.alloc(((size_t)evsl_dev::kRedBlocks * 64 + (size_t)n / evsl_dev::kWG + 1) *
+                            sizeof(double)));
   c.func = func;
   c.func_data = data;
   return 0;

@@ -44,6 +44,9 @@ struct alignas(sizeof(VT) * V) VecT {
 // out of L2; it pays when the launch's working set exceeds the Infinity
 // Cache (chosen per launch, streaming_launch below) and leaves the
 // arithmetic unchanged.
+// a KPM step of this vector type sums the pair (w.w, w.xk) per column
+template <typename VT>
+constexpr bool kKpmPairs = kpm_dots(1, sizeof(VT) == 4) == 2;
 template <typename T, int V>
 struct ExtVec {
   typedef T type __attribute__((ext_vector_type(V)));
@@ -172,9 +175,12 @@ __device__ __forceinline__ void cheb_spmm_block(
   }
   const bool ymode = MODE == kCheb || MODE == kRes;
   const bool need_xr = first || MODE == kKpm || cc_ != 0.0 || (ymode && yflush >= 2);
-  double dacc[V];
+  // kKpm dots of this lane's columns: in FP64 dacc = w.w and dacc1 = w.xk
+  // (two moments a degree, see dev.h), in FP32 dacc = w.v0
+  constexpr bool kPairs = MODE == kKpm && kKpmPairs<VT>;
+  double dacc[V], dacc1[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) dacc[j] = 0.0;
+  for (int j = 0; j < V; ++j) dacc[j] = dacc1[j] = 0.0;
 
   // epilogue operands of a row, loaded ahead of the gathers
   struct Ops {
@@ -217,7 +223,7 @@ __device__ __forceinline__ void cheb_spmm_block(
     if (xkm1) o.km1 = ld_last(xkm1, i);
     if (ymode && yflush > 0 && !first) o.yo = ld_last(y, i);
     if (MODE == kRes) o.rr = ld(v0, i);
-    if (MODE == kKpm) o.v = ld(v0, i);
+    if (MODE == kKpm && !kPairs) o.v = ld(v0, i);
     return o;
   };
   auto epilogue = [&](int r, const VT* acc, const Ops& o) {
@@ -256,7 +262,14 @@ __device__ __forceinline__ void cheb_spmm_block(
       }
     } else if (MODE == kKpm) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) dacc[j] += (double)w.v[j] * (double)o.v.v[j];
+      for (int j = 0; j < V; ++j) {
+        if (kPairs) {
+          dacc[j] += (double)w.v[j] * (double)w.v[j];
+          dacc1[j] += (double)w.v[j] * (double)o.xr.v[j];
+        } else {
+          dacc[j] += (double)w.v[j] * (double)o.v.v[j];
+        }
+      }
     }
   };
 
@@ -459,19 +472,24 @@ __device__ __forceinline__ void cheb_spmm_block(
 
   if (MODE == kKpm) {  // L is a power of two here (NG*L == kWG)
     static_assert(MODE != kKpm || (kWG % L) == 0, "KPM blocks need B/V | 256");
+    constexpr int W = kpm_dots(B, sizeof(VT) == 4);
 #pragma unroll
-    for (int j = 0; j < V; ++j) s_red[tid * V + j] = dacc[j];
-    __syncthreads();
-    for (int st = NG / 2; st > 0; st >>= 1) {
-      if (grp < st) {
+    for (int h = 0; h < W / B; ++h) {
+      if (h) __syncthreads();
 #pragma unroll
-        for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
-      }
+      for (int j = 0; j < V; ++j) s_red[tid * V + j] = h ? dacc1[j] : dacc[j];
       __syncthreads();
-    }
-    if (grp == 0) {
+      for (int st = NG / 2; st > 0; st >>= 1) {
+        if (grp < st) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) part[(size_t)blk * B + c0 + j] = s_red[tid * V + j];
+          for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
+        }
+        __syncthreads();
+      }
+      if (grp == 0) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) part[(size_t)blk * W + h * B + c0 + j] = s_red[tid * V + j];
+      }
     }
   }
 }
