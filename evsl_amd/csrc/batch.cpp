@@ -43,6 +43,23 @@ int pow2_at_least(int b) {
 // block widths the kCheb kernel is instantiated for
 int kernel_width(int b) { return b <= 8 ? b : pow2_at_least(b); }
 
+// Columns of one filter block on A: kBmaxPow, or fewer for the row-mask kernel,
+// whose matrix is a small part of a step's bytes, where the block's vectors
+// (three of the vector type, y in FP64, and the residual block of kRes) outgrow
+// 200 MB: they then stay in the 256 MB Infinity Cache from step to step
+// (100^3, us per column and step at 4 / 8 / 16 / 32 columns: FP32 3.4 / 2.8 /
+// 4.2 / 4.1, FP64 5.1 / 6.8 / 6.7 / 6.9, FP32 residual step - / 3.1 / - / 4.4;
+// 80^3 lattice FP32 2.2 / 2.0 / 1.6 / 2.3).  At least one 16-byte vector a lane
+// and two lanes a row.  A column's bits do not depend on its block.
+int filter_block_cap(const evsl_dev::Csr& A, bool f32, evsl_dev::Mode mode) {
+  int B = kBmaxPow;
+  if (!evsl_dev::mask_launch(A, B, f32, mode)) return B;
+  const double vs = f32 ? 4 : 8;
+  const double col = ((mode == evsl_dev::kRes ? 4.0 : 3.0) * vs + 8.0) * A.n;
+  while (B > (f32 ? 8 : 4) && B * col > 200e6) B >>= 1;
+  return B;
+}
+
 // Launches k = k0..k1 of the Chebyshev filter of per-column coefficient
 // table mus (row d holds degree d, B entries per row) over the row-major
 // block X0 of B columns, accumulating into Y.  The y flushes are scheduled
@@ -60,7 +77,7 @@ int block_filter_seg(int B, const FilterOp& op, const double* mus_d, int k0, int
     EVSL_HIP(evsl_dev::cheb_spmm(op.A, B, op.f32, evsl_dev::kCheb, xk, xkm1, xkp1, Y, nullptr,
                                  mus_d + (size_t)k * B, mus_d, k == 1 ? op.t1 : op.t2, op.cc,
                                  k == 1, yf, nullptr, c.stream));
-    c.astats.filter_bytes += c.A.mat_bytes((int)vs, B) + 4.0 * (c.n + 1) +
+    c.astats.filter_bytes += c.A.mat_bytes((int)vs, B) +
                              evsl_dev::cheb_vec_bytes(yf, k == 1, (int)vs) * B * c.n;
   }
   c.astats.n_filter_steps += k1 - k0 + 1;
@@ -80,12 +97,20 @@ int block_filter(int B, const FilterOp& op, const double* mus_d, int maxdeg, con
 // (the batched solver filters the same slices step after step), so a filter
 // pass issues no host-device copy and no synchronisation.
 struct BlockWork {
-  DevBuf X0, bufs, Y, Y2, zero, junk, mus;
+  DevBuf X0, bufs, Y, Y2, zero, junk;
   int Bcap = 0;
   bool f32 = false;
-  std::vector<const polparams*> mus_key;  // filters (in column order) of `mus`
-  int mus_kind = -1;                      // layout of `mus`: B, or 0 for phased
-  std::vector<size_t> mus_off;            // phased: offset of each phase's table
+  struct CoefTab {
+    DevBuf mus;
+    std::vector<const polparams*> key;  // filters (in column order) of `mus`
+    int kind = -1;                      // layout of `mus`: B, or 0 for phased
+    std::vector<size_t> off;            // phased: offset of each phase's table
+  };
+  // the tables of a pass's blocks, at most kCoefTabs (a further block takes
+  // over the oldest)
+  static constexpr size_t kCoefTabs = 8;
+  std::vector<std::unique_ptr<CoefTab>> tabs;
+  size_t next_tab = 0;
   int ensure(int n, int B, bool fp32, int maxdeg) {
     const size_t vs = fp32 ? 4 : 8;
     const size_t nb = (size_t)n * B * vs;
@@ -107,16 +132,28 @@ struct BlockWork {
   }
   // uploads `tab` as the coefficient table of (key, kind) unless it is there
   template <typename Build>
-  int coef_table(const std::vector<const polparams*>& key, int kind, Build build) {
-    if (kind == mus_kind && key == mus_key) return 0;
+  int coef_table(const std::vector<const polparams*>& key, int kind, Build build, CoefTab** out) {
+    for (auto& t : tabs)
+      if (t->kind == kind && t->key == key) {
+        *out = t.get();
+        return 0;
+      }
+    if (tabs.size() < kCoefTabs) {
+      next_tab = tabs.size();
+      tabs.push_back(std::make_unique<CoefTab>());
+    }
+    CoefTab& t = *tabs[next_tab];
+    next_tab = (next_tab + 1) % kCoefTabs;
     std::vector<double> tab;
-    mus_off.clear();
-    build(tab, mus_off);
+    t.off.clear();
+    t.kind = -1;
+    build(tab, t.off);
     // the copy below is ordered after the launches that read the old table
-    EVSL_HIP(mus.alloc(tab.size() * sizeof(double)));
-    EVSL_HIP(hipMemcpy(mus.p, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
-    mus_key = key;
-    mus_kind = kind;
+    EVSL_HIP(t.mus.alloc(tab.size() * sizeof(double)));
+    EVSL_HIP(hipMemcpy(t.mus.p, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
+    t.key = key;
+    t.kind = kind;
+    *out = &t;
     return 0;
   }
 };
@@ -174,6 +211,7 @@ int filter_columns_phased(int b, const double* const* xin, double* const* yout,
       k0 = kend + 1;
     }
   };
+  BlockWork::CoefTab* ct = nullptr;
   if (int e = W.coef_table(key, 0, [&](std::vector<double>& tab, std::vector<size_t>& off) {
         phases([&](int active, int, int, int kend, int, int) {
           off.push_back(tab.size());
@@ -183,7 +221,7 @@ int filter_columns_phased(int b, const double* const* xin, double* const* yout,
             for (int d = 0; d <= kend && d <= key[i]->deg; ++d)
               t[(size_t)d * active + i] = key[i]->mu[d];
         });
-      }))
+      }, &ct))
     return e;
   EVSL_HIP(evsl_dev::pack_cols(n, b, col_ptrs(in.data(), b), W.X0.p, f32, c.stream));
   FilterOp op;
@@ -195,7 +233,7 @@ int filter_columns_phased(int b, const double* const* xin, double* const* yout,
   int phase = 0, err = 0;
   phases([&](int active, int live, int k0, int kend, int keep, int next) {
     if (err) return;
-    const double* mus_d = W.mus.as<double>() + W.mus_off[phase++];
+    const double* mus_d = ct->mus.as<double>() + ct->off[phase++];
     if ((err = block_filter_seg(active, op, mus_d, k0, kend, W.X0.p, slot, Y))) return;
     hipError_t he = evsl_dev::unpack_range(n, active, keep, live, Y, false,
                                            col_ptrs(out.data() + keep, live - keep), c.stream);
@@ -240,8 +278,9 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
   }
   int maxdeg = 0;
   for (int j = 0; j < ncols; ++j) maxdeg = std::max(maxdeg, pols[j]->deg);
-  for (int j0 = 0; j0 < ncols; j0 += kBmaxPow) {
-    const int b = std::min(kBmaxPow, ncols - j0);
+  const int cap = filter_block_cap(c.A.view(), f32, evsl_dev::kCheb);
+  for (int j0 = 0; j0 < ncols; j0 += cap) {
+    const int b = std::min(cap, ncols - j0);
     const int B = kernel_width(b);
     if (int e = W.ensure(n, B, f32, maxdeg)) return e;
     std::vector<const double*> in(B);
@@ -273,17 +312,18 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
       if (int e = filter_columns_phased(b, xin + j0, yout + j0, pols + j0, f32, W)) return e;
       continue;
     }
+    BlockWork::CoefTab* ct = nullptr;
     if (int e = W.coef_table(key, B, [&](std::vector<double>& tab, std::vector<size_t>&) {
           tab.assign((size_t)(md + 1) * B, 0.0);
           for (int cc = 0; cc < b; ++cc)
             for (int d = 0; d <= key[cc]->deg; ++d) tab[(size_t)d * B + cc] = key[cc]->mu[d];
-        }))
+        }, &ct))
       return e;
     EVSL_HIP(evsl_dev::pack_cols(n, B, col_ptrs(in.data(), B), W.X0.p, f32, c.stream));
     void* bufs[3] = {W.buf(0, n, B), W.buf(1, n, B), W.buf(2, n, B)};
     FilterOp op;
     if (int e = make_filter_op(pols[j0]->cc, pols[j0]->dd, f32, &op)) return e;
-    if (int e = block_filter(B, op, W.mus.as<double>(), md, W.X0.p, bufs, W.Y.p)) return e;
+    if (int e = block_filter(B, op, ct->mus.as<double>(), md, W.X0.p, bufs, W.Y.p)) return e;
     EVSL_HIP(evsl_dev::unpack_cols(n, B, W.Y.p, false, col_ptrs(out.data(), B), c.stream));
   }
   return 0;
@@ -441,11 +481,12 @@ int residual_filter(int n, int m, double* U, double* W, const polparams* pol, Bl
     if (int e = make_filter_op(pol->cc, pol->dd, true, &op)) return e;
     // per-launch coefficient tables of every chunk, uploaded once:
     // g[chunk][k][c] = 2 T_k(theta~_c), k = 1..deg-1; pairs (mu_{k+1}, mu_1)
-    const int nchunk = (ms + kBmaxPow - 1) / kBmaxPow;
-    const size_t gstride = (size_t)(deg + 1) * kBmaxPow;
+    const int cap = filter_block_cap(op.A, true, evsl_dev::kRes);
+    const int nchunk = (ms + cap - 1) / cap;
+    const size_t gstride = (size_t)(deg + 1) * cap;
     std::vector<double> g(gstride * nchunk, 0.0), mp((size_t)2 * (deg + 1), 0.0);
-    for (int j0 = 0, ch = 0; j0 < ms; j0 += kBmaxPow, ++ch) {
-      const int b = std::min(kBmaxPow, ms - j0);
+    for (int j0 = 0, ch = 0; j0 < ms; j0 += cap, ++ch) {
+      const int b = std::min(cap, ms - j0);
       const int B = kernel_width(b);
       for (int cc = 0; cc < b; ++cc) {
         const double x = ths[small[j0 + cc]];
@@ -467,8 +508,8 @@ int residual_filter(int n, int m, double* U, double* W, const polparams* pol, Bl
     EVSL_HIP(mp_d.alloc(mp.size() * sizeof(double)));
     EVSL_HIP(hipMemcpy(g_d.p, g.data(), g.size() * sizeof(double), hipMemcpyHostToDevice));
     EVSL_HIP(hipMemcpy(mp_d.p, mp.data(), mp.size() * sizeof(double), hipMemcpyHostToDevice));
-    for (int j0 = 0, ch = 0; j0 < ms; j0 += kBmaxPow, ++ch) {
-      const int b = std::min(kBmaxPow, ms - j0);
+    for (int j0 = 0, ch = 0; j0 < ms; j0 += cap, ++ch) {
+      const int b = std::min(cap, ms - j0);
       const int B = kernel_width(b);
       if (int e = bw.ensure(n, B, true, deg)) return e;
       // R columns -> FP32 block (xk of the first launch = D_1 = R); the same
@@ -498,7 +539,7 @@ int residual_filter(int n, int m, double* U, double* W, const polparams* pol, Bl
                                        gch + (size_t)k * B, mp_d.as<double>() + 2 * k, op.t2,
                                        op.cc, k == 1, yf, nullptr, c.stream));
           // the kCheb streams plus the residual block R
-          c.astats.refine_bytes += c.A.mat_bytes(4, B) + 4.0 * (n + 1) +
+          c.astats.refine_bytes += c.A.mat_bytes(4, B) +
                                    (evsl_dev::cheb_vec_bytes(yf, k == 1, 4) + 4.0) * B * n;
         }
         EVSL_HIP(evsl_dev::unpack_cols(n, B, Yb, false, col_ptrs(out.data(), B), c.stream));

@@ -31,6 +31,9 @@ struct SpmmTuner;
 constexpr int kPatCodes = 255;
 constexpr unsigned char kPatDiag = 255;
 
+// pairs a row-mask code holds (spmm_mask.h)
+constexpr int kMaskPairs = 18;  // 16 in use; the kernel reads whole groups of 6
+
 struct Csr {
   int n = 0, nnz = 0;
   const int* ia = nullptr;
@@ -56,6 +59,16 @@ struct Csr {
   const double* dg64 = nullptr;
   const float* pval32 = nullptr;
   const float* dg32 = nullptr;
+  // Row masks (spmm_mask.h), when the pattern codes name at most 16 pairs,
+  // every row's columns ascend and every diagonal is stored: rmask[row] (mbytes
+  // bytes) has bit p set where the row holds pair p = (moff[p], mval[p]), pairs
+  // in order of their offsets, the first nneg of them below the diagonal,
+  // whose value is dg64 / dg32.
+  const void* rmask = nullptr;
+  int mbytes = 0, npair = 0, nneg = 0;
+  int moff[kMaskPairs] = {};
+  double mval64[kMaskPairs] = {};
+  float mval32[kMaskPairs] = {};
   // per block width: nblk+1 pairs (first row of the block, its row pointer)
   const int* rb[kNumWidths] = {};
   int nblk[kNumWidths] = {};
@@ -75,6 +88,25 @@ inline bool pattern_launch(const Csr& A, int B, int vsize) {
 }
 
 enum Mode { kPlain = 0, kCheb = 1, kKpm = 2, kRes = 3 };
+
+// Lane layout of the row-mask kernel, 10 * (columns per lane) + rows per lane
+// group.  KPM steps keep the CSR kernel's layout, whose block tree their bits
+// come from.
+int mask_layout_of(int B, bool fp32, Mode mode);
+// Whether a launch on A runs the row-mask kernel.  Every coded matrix does, at
+// every width of a path's blocks (figures in spmm_mask.h); a KPM step only where the CSR kernel's row blocks
+// are full (rows per block times the longest row within kNnzCap), so that
+// both kernels sum the same blocks, and the FP32 plain and KPM modes, which no
+// one-matrix path runs, have no instance.
+bool mask_launch(const Csr& A, int B, bool fp32, Mode mode);
+hipError_t cheb_spmm_mask_f32(const Csr& A, int B, Mode mode, const void* xk, const void* xkm1,
+                              void* xkp1, void* y, const void* v0, const double* s,
+                              const double* mu0, double t, double cc, bool first, int yflush,
+                              double* part, hipStream_t st);
+hipError_t cheb_spmm_mask_f64(const Csr& A, int B, Mode mode, const void* xk, const void* xkm1,
+                              void* xkp1, void* y, const void* v0, const double* s,
+                              const double* mu0, double t, double cc, bool first, int yflush,
+                              double* part, hipStream_t st);
 
 // One Chebyshev degree step over a B-column block (B in {1..8,16,32}; the
 // KPM mode needs B in {1,2,4,8,16,32}):
@@ -154,6 +186,8 @@ void spmm_tuner_destroy(SpmmTuner* t);
 // policy of a key: layout > 0 forces that candidate, 0 the fixed table,
 // -1 tunes (the default); resets what was learned.  -1 on a bad key/layout.
 int spmm_tuner_set(SpmmTuner* t, int B, bool fp32, Mode mode, int layout);
+// the layout a key is forced to, 0 when it is not
+int spmm_tuner_forced(SpmmTuner* t, int B, bool fp32, Mode mode);
 // layout the key launches now: the forced or chosen one, or the table's
 // while undecided
 int spmm_tuner_layout(SpmmTuner* t, int B, bool fp32, Mode mode);
@@ -218,6 +252,19 @@ bool cheb_spmm_streaming(const Csr& A, int B, bool fp32, Mode mode);
 // recurrence of the mixed form keeps v.T_k v at every step: its moments carry
 // the recurrence's FP32 rounding, which the products would change.
 constexpr int kpm_dots(int B, bool fp32) { return fp32 ? B : 2 * B; }
+// Columns of a KPM block: 32, or fewer where the three FP64 vector blocks of
+// 32 columns outgrow 200 MB (n > 260,000) and the rows are regular (a row has
+// its neighbour's column offsets, so a gather reads contiguous segments and
+// the matrix is a small part of a step): 16 while that keeps them under it,
+// else 8.  The blocks then stay in the 256 MB Infinity Cache from step to
+// step (100^3, us per column and step at 32 / 16 / 8 columns: row-mask kernel
+// 6.5 / 6.5 / 4.1, CSR kernel 7.1 / 7.5 / 5.9); irregular rows pay for their
+// gathers by the segment, so wider is better (300,000 random rows of 3-9: 2.6
+// / 3.0 / 4.6).  One rule for every KPM path: moments depend on the width.
+inline int kpm_max_width(int n, bool regular) {
+  if (!regular || 24.0 * n * 32 <= 200e6) return 32;
+  return 24.0 * n * 16 <= 200e6 ? 16 : 8;
+}
 // steps of a series of Mdeg moments
 inline int kpm_steps(int Mdeg, bool fp32) { return fp32 ? Mdeg : (Mdeg + 1) / 2; }
 // degrees whose block partials are kept and then summed by one launch: the

@@ -57,6 +57,7 @@ struct DevMatrix {
   float* a32s = nullptr;           // FP32 copy of (A - shift_cc I) * shift_scale
   double shift_cc = 0.0, shift_scale = 0.0;
   bool full_diag = false;          // every row stores its diagonal entry
+  bool regular = false;            // regular_rows
   int* rb[evsl_dev::kNumWidths] = {};
   int nblk[evsl_dev::kNumWidths] = {};
   evsl_dev::SpmmTuner* tune = nullptr;  // the filter kernel's layout tuner
@@ -76,14 +77,21 @@ struct DevMatrix {
   float* dg32 = nullptr;
   float* pval32s = nullptr;
   float* dg32s = nullptr;
+  // row masks (evsl_dev::Csr::rmask): pair p is table entry mcode[p]
+  void* rmask = nullptr;
+  int mbytes = 0, nneg = 0;
+  std::vector<int> mcode, moff;
   // bytes per nonzero of the column index the filter kernels read
   int idx_bytes() const { return pc ? 1 : (jd ? 2 : 4); }
   // matrix bytes one filter launch of B columns streams with values of vs
-  // bytes: the codes, the diagonal and its position, or the indices and the
-  // values (evsl_dev::pattern_launch)
+  // bytes: the row masks and the diagonal, or the row pointers and either the
+  // codes, the diagonal and its position (evsl_dev::pattern_launch) or the
+  // indices and the values
   double mat_bytes(int vs, int B) const {
-    return (pc && B * vs <= evsl_dev::kPatMaxRowBytes) ? (double)nnz + (double)n * (vs + 1)
-                                                       : (double)nnz * (vs + (jd ? 2 : 4));
+    if (rmask) return (double)n * (mbytes + vs);
+    return 4.0 * (n + 1.0) + (pc && B * vs <= evsl_dev::kPatMaxRowBytes
+                                  ? (double)nnz + (double)n * (vs + 1)
+                                  : (double)nnz * (vs + (jd ? 2 : 4)));
   }
   evsl_dev::Csr view() const;
   void release();
@@ -91,12 +99,17 @@ struct DevMatrix {
 
 // Build the LDS row-block partition (at most rows_cap rows and kNnzCap
 // nonzeros per block) from host row pointers.
+// whether most of 64 rows spread over the matrix have the column offsets of the
+// row after them (stencils and lattices)
+bool regular_rows(int n, const int* ia_h, const int* ja_h);
 std::vector<int> make_row_blocks(const int* ia_h, int n, int rows_cap);
-// A device operator M from a device CSR: row-block tables of every width,
+// A device operator M from a device CSR (ia_h, ja_h, a_h: its host arrays, or
+// null to read them back): row-block tables of every width,
 // 16-bit column offsets when they fit, the stored-diagonal flag; *red_need =
 // reduction scratch (doubles) its launches need (see ensure_red_part)
 int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const int* ia_h,
-                        const int* ja_h, bool owns, DevMatrix& M, size_t* red_need);
+                        const int* ja_h, const double* a_h, bool owns, DevMatrix& M,
+                        size_t* red_need);
 int ensure_red_part(size_t need);
 // make sure the shifted FP32 copy for (cc, scale) exists; false if the
 // matrix lacks stored diagonal entries

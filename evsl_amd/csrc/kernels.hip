@@ -1095,6 +1095,19 @@ int cheb_spmm_nblk(const Csr& A, int B, bool fp32, Mode mode) {
   return slot < 0 ? -1 : A.nblk[slot];
 }
 
+int mask_layout_of(int B, bool fp32, Mode mode) {
+  return width_slot(B) < 0 ? -1 : mask_layout(fp32 ? 4 : 8, B, mode);
+}
+
+bool mask_launch(const Csr& A, int B, bool fp32, Mode mode) {
+  if (!A.rmask || width_slot(B) < 0) return false;
+  if (fp32) return mode == kCheb || mode == kRes;
+  if (mode != kKpm) return true;
+  const int lay = mask_layout(8, B, kKpm);
+  const int lanes = B / (lay / 10) / (lay % 10);
+  return (B & (B - 1)) == 0 && rows_cap_for(lanes) * (A.npair + 1) <= kNnzCap;
+}
+
 int spmm_table_layout(int B, bool fp32, Mode mode) {
   const int v = policy_factor(B, fp32, mode, true), vr = policy_factor(B, fp32, mode, false);
   return v > 0 ? 10 * v + vr / v : -1;
@@ -1120,6 +1133,12 @@ hipError_t cheb_spmm(const Csr& A, int B, bool fp32, Mode mode, const void* xk,
   if (A.n <= 0) return hipSuccess;
   if (yflush < 0 || yflush > 3 || (first && yflush != 1) || (yflush == 3 && !xkm1))
     return hipErrorInvalidValue;
+  // matrices coded by row masks run their own kernel, unless the caller has
+  // forced a lane layout of the CSR kernel
+  if (mask_launch(A, B, fp32, mode) &&
+      !(A.tune && (mode == kCheb || mode == kRes) && spmm_tuner_forced(A.tune, B, fp32, mode)))
+    return (fp32 ? cheb_spmm_mask_f32 : cheb_spmm_mask_f64)(A, B, mode, xk, xkm1, xkp1, y, v0, s,
+                                                            mu0, t, cc, first, yflush, part, st);
   // ChebAv and residual steps of the tuned widths go through the matrix's
   // layout tuner (same bits, the fastest layout once it has measured)
   if (A.tune && (mode == kCheb || mode == kRes) && tune_width_index(B) >= 0)

@@ -74,7 +74,7 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
   const int n = c.n;
   const double ctr = (intv[3] + intv[2]) / 2.0, wid = (intv[3] - intv[2]) / 2.0;
   std::vector<double> raw(Mdeg + 1, 0.0);  // raw[k] = sum_m v_m . T_k v_m
-  const int Bmax = 32;
+  const int Bmax = c.op == 1 ? evsl_dev::kpm_max_width(n, c.A.regular) : 32;
   // FP64 on a CSR matrix: two moments a step (kpm_dots); a user operator's
   // series takes v.T_k v at every step
   const bool pairs = c.op == 1;
@@ -131,7 +131,7 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
                                                 dots.as<double>() + (size_t)(k + 2 - have) * W,
                                                 scratch.as<double>(), c.stream));
         }
-        c.astats.filter_bytes += c.A.mat_bytes(8, B) + 4.0 * (n + 1) +
+        c.astats.filter_bytes += c.A.mat_bytes(8, B) +
                                  (double)(k == 0 ? 2 : 3) * nb * sizeof(double);
       }
       c.astats.n_filter_steps += steps;
@@ -352,7 +352,10 @@ int evsl_amd_bench_filter(int B, int prec, int mode, int nsteps, double cc, doub
   nsteps = (nsteps + 2) / 3 * 3;
   // the layout tuner settles first (its measuring launches run candidate
   // layouts), so the timed launches run the layout the solvers will use
-  if (md != evsl_dev::kKpm && op.A.tune) {
+  const bool forced = md != evsl_dev::kKpm && op.A.tune &&
+                      evsl_dev::spmm_tuner_forced(op.A.tune, B, f32, md) > 0;
+  const bool mask = evsl_dev::mask_launch(op.A, B, f32, md) && !forced;
+  if (md != evsl_dev::kKpm && op.A.tune && !mask) {
     for (int it = 0; it < 4096 && !evsl_dev::spmm_tuner_decided(op.A.tune, B, f32, md); ++it) {
       EVSL_HIP(evsl_dev::cheb_spmm(op.A, B, f32, md, buf[it % 3], buf[(it + 1) % 3],
                                    buf[(it + 2) % 3], buf[3], buf[4], scol, mu0col, op.t2, op.cc,
@@ -387,7 +390,7 @@ int evsl_amd_bench_filter(int B, int prec, int mode, int nsteps, double cc, doub
     vbytes = 3.0 * vs;
   else
     vbytes = 3.0 * vs + 16.0 * flushes / nsteps + (mode == 3 ? vs : 0.0);
-  *bytes_per_step = c.A.mat_bytes((int)vs, B) + 4.0 * (n + 1) + vbytes * nb;
+  *bytes_per_step = c.A.mat_bytes((int)vs, B) + vbytes * nb;
   return 0;
 }
 
@@ -506,6 +509,18 @@ int evsl_amd_pattern_codes(void) {
   return c.op == 1 && c.A.pc ? c.A.npat : 0;
 }
 
+int evsl_amd_spmm_row_masks(int B, int prec, int mode) {
+  const Context& c = ctx();
+  if (c.op != 1 || mode < 1 || mode > 3) return 0;
+  const evsl_dev::Mode md =
+      mode == 2 ? evsl_dev::kKpm : (mode == 3 ? evsl_dev::kRes : evsl_dev::kCheb);
+  const bool f32 = prec == EVSL_PREC_MIXED && mode != 2;
+  const evsl_dev::Csr A = c.A.view();
+  if (!evsl_dev::mask_launch(A, B, f32, md)) return 0;
+  if (mode != 2 && A.tune && evsl_dev::spmm_tuner_forced(A.tune, B, f32, md)) return 0;
+  return A.mbytes;
+}
+
 int evsl_amd_spmm_layout(int B, int prec, int mode, int* decided) {
   const Context& c = ctx();
   const evsl_dev::Mode md =
@@ -513,6 +528,7 @@ int evsl_amd_spmm_layout(int B, int prec, int mode, int* decided) {
   const bool f32 = prec == EVSL_PREC_MIXED && mode != 2;
   if (decided) *decided = 1;
   if (mode < 1 || mode > 3) return -1;
+  if (evsl_amd_spmm_row_masks(B, prec, mode) > 0) return evsl_dev::mask_layout_of(B, f32, md);
   if (c.op != 1 || !c.A.tune || !c.spmm_tuning) return evsl_dev::spmm_table_layout(B, f32, md);
   if (decided) *decided = evsl_dev::spmm_tuner_decided(c.A.tune, B, f32, md);
   return evsl_dev::spmm_tuner_layout(c.A.tune, B, f32, md);

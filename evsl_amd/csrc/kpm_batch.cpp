@@ -32,6 +32,7 @@ struct BatchMatrix {
   const csrMat* host = nullptr;
   int n = 0, nnz = 0;
   bool full_diag = false;
+  bool regular = false;
   DevBuf ia, ja, a64;
   std::map<int, DevBuf> table;  // row-block table by lanes per row
   std::map<int, int> nblk;
@@ -138,6 +139,7 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
         full = has;
       }
       m->full_diag = full;
+      m->regular = regular_rows(m->n, A->ia, A->ja);
       it = by_ptr.emplace(A, m.get()).first;
       mat.push_back(std::move(m));
     }
@@ -175,105 +177,112 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
   EVSL_HIP(nrm2.alloc(32 * sizeof(double)));
   DevBuf d_tab, d_owner, d_sums, d_owner1, d_first1, d_owner2;
   std::vector<double> hdots;
-  int done = 0;
-  while (done < nvec) {
-    int B = 32;
-    while (B > nvec - done) B >>= 1;
-    const int V = evsl_dev::cheb_spmm_vec(B, f32, evsl_dev::kKpm);
-    const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
-    if (V <= 0 || R <= 0) return EVSL_ERR_ARG;
-    const int lanes = B / V / R;
-    std::vector<evsl_dev::KpmGroupEntry> tab(nreq);
-    std::vector<evsl_dev::KpmSumEntry> sums(nreq);
-    std::vector<int> owner, owner1, first1(nreq), owner2;
-    int total = 0;
-    // values per block partial, steps, and the degrees summed by one launch
-    const int W = evsl_dev::kpm_dots(B, f32), steps = evsl_dev::kpm_steps(Mdeg, f32);
-    size_t pv = 0;
-    for (int r = 0; r < nreq; ++r) {
-      if (int e = req[r].mat->ensure_table(lanes)) return e;
-      pv = std::max(pv, (size_t)req[r].mat->nblk[lanes] * W);
-    }
-    const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
-    for (int r = 0; r < nreq; ++r) {
-      BatchRequest& q = req[r];
-      BatchMatrix& m = *q.mat;
-      const int nblk = m.nblk[lanes];
-      const size_t nb = (size_t)m.n * B;
-      EVSL_HIP(q.x0.alloc(nb * vs));
-      EVSL_HIP(q.ring.alloc(3 * nb * vs));
-      EVSL_HIP(q.part.alloc((size_t)nd * std::max(nblk, 1) * W * sizeof(double)));
-      EVSL_HIP(q.dots.alloc((size_t)(steps + 1) * W * sizeof(double)));
-      const int G = evsl_dev::sum_levels_blocks(nblk, W);
-      if (G > 1) EVSL_HIP(q.scratch.alloc((size_t)nd * G * W * sizeof(double)));
-      // start block: the kpmdos_ex vectors of this request's seed, unit columns
-      double* xd = f32 ? x64.as<double>() : q.x0.as<double>();
-      EVSL_HIP(evsl_dev::rm_random(m.n, B, vec_kind == EVSL_VEC_RADEMACHER ? 0 : 1, q.seed, done,
-                                   B, xd, c.stream));
-      EVSL_HIP(evsl_dev::rm_col_nrm2(m.n, B, xd, nrm_part.as<double>(), nrm2.as<double>(),
-                                     c.stream));
-      EVSL_HIP(evsl_dev::rm_col_scale_rsqrt(m.n, B, xd, nrm2.as<double>(), c.stream));
-      if (f32) EVSL_HIP(evsl_dev::f64_to_f32(nb, xd, q.x0.as<float>(), c.stream));
-      evsl_dev::KpmGroupEntry& e = tab[r];
-      e.ia = m.ia.as<int>();
-      e.ja = m.ja.as<int>();
-      e.a = f32 ? (const void*)q.a32.p : (const void*)m.a64.p;
-      e.rbp = m.table[lanes].as<int>();
-      e.x0 = q.x0.p;
-      e.ring = q.ring.p;
-      e.part = q.part.as<double>();
-      e.t0 = q.t0;
-      e.t = q.t;
-      e.cc = q.cc;
-      e.n = m.n;
-      e.blk0 = total;
-      e.k0 = 0;
-      e.part_step = nblk * W;
-      owner.insert(owner.end(), nblk, r);
-      total += nblk;
-      evsl_dev::KpmSumEntry& s = sums[r];
-      s.part = q.part.as<double>();
-      s.scratch = q.scratch.as<double>();
-      s.dots = q.dots.as<double>();
-      s.nblk = nblk;
-      s.G = G;
-      s.k0 = 0;
-      s.pad = 0;
-      first1[r] = (int)owner1.size();
-      owner1.insert(owner1.end(), G, r);
-      if (G > 1) owner2.push_back(r);
-    }
-    if (int e = upload(d_tab, tab.data(), tab.size() * sizeof(tab[0]))) return e;
-    if (int e = upload(d_owner, owner.data(), owner.size() * sizeof(int))) return e;
-    if (int e = upload(d_sums, sums.data(), sums.size() * sizeof(sums[0]))) return e;
-    if (int e = upload(d_owner1, owner1.data(), owner1.size() * sizeof(int))) return e;
-    if (int e = upload(d_first1, first1.data(), first1.size() * sizeof(int))) return e;
-    if (int e = upload(d_owner2, owner2.data(), owner2.size() * sizeof(int))) return e;
-    double step_bytes = 0.0;
-    for (int r = 0; r < nreq; ++r)
-      step_bytes += (double)req[r].mat->nnz * (vs + 4) + 4.0 * (req[r].mat->n + 1) +
-                    (f32 ? 4.0 : 3.0) * req[r].mat->n * B * vs;
-    for (int k = 0; k < steps; ++k) {
-      EVSL_HIP(evsl_dev::kpm_group_step(f32, B, d_tab.as<evsl_dev::KpmGroupEntry>(),
-                                        d_owner.as<int>(), total, k, k % nd, c.stream));
-      if ((k + 1) % nd == 0 || k + 1 == steps) {
-        const int have = k % nd + 1;
-        EVSL_HIP(evsl_dev::kpm_group_sums(f32, B, d_sums.as<evsl_dev::KpmSumEntry>(),
-                                          k + 1 - have, have, d_owner1.as<int>(),
-                                          d_first1.as<int>(), (int)owner1.size(),
-                                          d_owner2.as<int>(), (int)owner2.size(), c.stream));
+  // the requests whose column blocks start at one width share their launches
+  for (int width : {32, 16, 8}) {
+    std::vector<BatchRequest*> reqs;
+    for (auto& q : req)
+      if (evsl_dev::kpm_max_width(q.mat->n, !f32 && q.mat->regular) == width) reqs.push_back(&q);
+    const int nr = (int)reqs.size();
+    int done = nr ? 0 : nvec;
+    while (done < nvec) {
+      int B = width;
+      while (B > nvec - done) B >>= 1;
+      const int V = evsl_dev::cheb_spmm_vec(B, f32, evsl_dev::kKpm);
+      const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
+      if (V <= 0 || R <= 0) return EVSL_ERR_ARG;
+      const int lanes = B / V / R;
+      std::vector<evsl_dev::KpmGroupEntry> tab(nr);
+      std::vector<evsl_dev::KpmSumEntry> sums(nr);
+      std::vector<int> owner, owner1, first1(nr), owner2;
+      int total = 0;
+      // values per block partial, steps, and the degrees summed by one launch
+      const int W = evsl_dev::kpm_dots(B, f32), steps = evsl_dev::kpm_steps(Mdeg, f32);
+      size_t pv = 0;
+      for (int r = 0; r < nr; ++r) {
+        if (int e = reqs[r]->mat->ensure_table(lanes)) return e;
+        pv = std::max(pv, (size_t)reqs[r]->mat->nblk[lanes] * W);
       }
-      c.astats.filter_bytes += step_bytes;
+      const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
+      for (int r = 0; r < nr; ++r) {
+        BatchRequest& q = *reqs[r];
+        BatchMatrix& m = *q.mat;
+        const int nblk = m.nblk[lanes];
+        const size_t nb = (size_t)m.n * B;
+        EVSL_HIP(q.x0.alloc(nb * vs));
+        EVSL_HIP(q.ring.alloc(3 * nb * vs));
+        EVSL_HIP(q.part.alloc((size_t)nd * std::max(nblk, 1) * W * sizeof(double)));
+        EVSL_HIP(q.dots.alloc((size_t)(steps + 1) * W * sizeof(double)));
+        const int G = evsl_dev::sum_levels_blocks(nblk, W);
+        if (G > 1) EVSL_HIP(q.scratch.alloc((size_t)nd * G * W * sizeof(double)));
+        // start block: the kpmdos_ex vectors of this request's seed, unit columns
+        double* xd = f32 ? x64.as<double>() : q.x0.as<double>();
+        EVSL_HIP(evsl_dev::rm_random(m.n, B, vec_kind == EVSL_VEC_RADEMACHER ? 0 : 1, q.seed, done,
+                                     B, xd, c.stream));
+        EVSL_HIP(evsl_dev::rm_col_nrm2(m.n, B, xd, nrm_part.as<double>(), nrm2.as<double>(),
+                                       c.stream));
+        EVSL_HIP(evsl_dev::rm_col_scale_rsqrt(m.n, B, xd, nrm2.as<double>(), c.stream));
+        if (f32) EVSL_HIP(evsl_dev::f64_to_f32(nb, xd, q.x0.as<float>(), c.stream));
+        evsl_dev::KpmGroupEntry& e = tab[r];
+        e.ia = m.ia.as<int>();
+        e.ja = m.ja.as<int>();
+        e.a = f32 ? (const void*)q.a32.p : (const void*)m.a64.p;
+        e.rbp = m.table[lanes].as<int>();
+        e.x0 = q.x0.p;
+        e.ring = q.ring.p;
+        e.part = q.part.as<double>();
+        e.t0 = q.t0;
+        e.t = q.t;
+        e.cc = q.cc;
+        e.n = m.n;
+        e.blk0 = total;
+        e.k0 = 0;
+        e.part_step = nblk * W;
+        owner.insert(owner.end(), nblk, r);
+        total += nblk;
+        evsl_dev::KpmSumEntry& s = sums[r];
+        s.part = q.part.as<double>();
+        s.scratch = q.scratch.as<double>();
+        s.dots = q.dots.as<double>();
+        s.nblk = nblk;
+        s.G = G;
+        s.k0 = 0;
+        s.pad = 0;
+        first1[r] = (int)owner1.size();
+        owner1.insert(owner1.end(), G, r);
+        if (G > 1) owner2.push_back(r);
+      }
+      if (int e = upload(d_tab, tab.data(), tab.size() * sizeof(tab[0]))) return e;
+      if (int e = upload(d_owner, owner.data(), owner.size() * sizeof(int))) return e;
+      if (int e = upload(d_sums, sums.data(), sums.size() * sizeof(sums[0]))) return e;
+      if (int e = upload(d_owner1, owner1.data(), owner1.size() * sizeof(int))) return e;
+      if (int e = upload(d_first1, first1.data(), first1.size() * sizeof(int))) return e;
+      if (int e = upload(d_owner2, owner2.data(), owner2.size() * sizeof(int))) return e;
+      double step_bytes = 0.0;
+      for (int r = 0; r < nr; ++r)
+        step_bytes += (double)reqs[r]->mat->nnz * (vs + 4) + 4.0 * (reqs[r]->mat->n + 1) +
+                      (f32 ? 4.0 : 3.0) * reqs[r]->mat->n * B * vs;
+      for (int k = 0; k < steps; ++k) {
+        EVSL_HIP(evsl_dev::kpm_group_step(f32, B, d_tab.as<evsl_dev::KpmGroupEntry>(),
+                                          d_owner.as<int>(), total, k, k % nd, c.stream));
+        if ((k + 1) % nd == 0 || k + 1 == steps) {
+          const int have = k % nd + 1;
+          EVSL_HIP(evsl_dev::kpm_group_sums(f32, B, d_sums.as<evsl_dev::KpmSumEntry>(),
+                                            k + 1 - have, have, d_owner1.as<int>(),
+                                            d_first1.as<int>(), (int)owner1.size(),
+                                            d_owner2.as<int>(), (int)owner2.size(), c.stream));
+        }
+        c.astats.filter_bytes += step_bytes;
+      }
+      c.astats.n_filter_steps += steps;
+      c.astats.n_filter_cols += (size_t)steps * B * nr;
+      hdots.resize((size_t)(steps + 1) * W);
+      for (int r = 0; r < nr; ++r) {
+        EVSL_HIP(hipMemcpy(hdots.data(), reqs[r]->dots.p, hdots.size() * sizeof(double),
+                           hipMemcpyDeviceToHost));
+        kpm_add_dots(Mdeg, f32, B, hdots.data(), reqs[r]->raw.data());
+      }
+      done += B;
     }
-    c.astats.n_filter_steps += steps;
-    c.astats.n_filter_cols += (size_t)steps * B * nreq;
-    hdots.resize((size_t)(steps + 1) * W);
-    for (int r = 0; r < nreq; ++r) {
-      EVSL_HIP(hipMemcpy(hdots.data(), req[r].dots.p, hdots.size() * sizeof(double),
-                         hipMemcpyDeviceToHost));
-      kpm_add_dots(Mdeg, f32, B, hdots.data(), req[r].raw.data());
-    }
-    done += B;
   }
   for (int r = 0; r < nreq; ++r)
     kpm_moments(Mdeg, damping, nvec, req[r].intv, req[r].mat->n, req[r].raw.data(),

@@ -66,6 +66,17 @@ evsl_dev::Csr DevMatrix::view() const {
     c.pval32 = pval32;
     c.dg32 = dg32;
   }
+  if (rmask) {
+    c.rmask = rmask;
+    c.mbytes = mbytes;
+    c.npair = (int)mcode.size();
+    c.nneg = nneg;
+    for (int p = 0; p < c.npair; ++p) {
+      c.moff[p] = moff[p];
+      c.mval64[p] = pval_h[mcode[p]];
+      c.mval32[p] = (float)pval_h[mcode[p]];
+    }
+  }
   for (int w = 0; w < evsl_dev::kNumWidths; ++w) {
     c.rb[w] = rb[w];
     c.nblk[w] = nblk[w];
@@ -86,10 +97,23 @@ void DevMatrix::release() {
   if (a32) (void)hipFree(a32);
   if (a32s) (void)hipFree(a32s);
   for (void* p : {(void*)pc, (void*)pdpos, (void*)poff, (void*)pval64, (void*)dg64, (void*)pval32,
-                  (void*)dg32, (void*)pval32s, (void*)dg32s})
+                  (void*)dg32, (void*)pval32s, (void*)dg32s, rmask})
     if (p) (void)hipFree(p);
   evsl_dev::spmm_tuner_destroy(tune);
   *this = DevMatrix();
+}
+
+bool regular_rows(int n, const int* ia, const int* ja) {
+  const int samples = std::min(64, n - 1);
+  int same = 0;
+  for (int s = 0; s < samples; ++s) {
+    const int r = (int)((long long)(n - 1) * s / samples);
+    const int len = ia[r + 1] - ia[r];
+    bool eq = ia[r + 2] - ia[r + 1] == len;
+    for (int k = 0; k < len && eq; ++k) eq = ja[ia[r + 1] + k] == ja[ia[r] + k] + 1;
+    same += eq;
+  }
+  return 2 * same > samples;
 }
 
 std::vector<int> make_row_blocks(const int* ia, int n, int rows_cap) {
@@ -234,10 +258,39 @@ bool encode_pattern(int n, const int* ia, const int* ja, const double* a,
   return true;
 }
 
+// Row masks from pattern codes: at most 16 pairs of finite value, numbered in
+// order of their offsets, in rows of ascending columns that all store their
+// diagonal.  False where that does not hold.
+bool encode_masks(int n, const int* ia, const int* ja, const std::vector<unsigned char>& code,
+                  const std::vector<int>& off, const std::vector<double>& val,
+                  std::vector<int>& order, std::vector<unsigned short>& mask) {
+  const int np = (int)off.size();
+  if (np > 16) return false;
+  for (double v : val)
+    if (!std::isfinite(v)) return false;
+  order.resize(np);
+  for (int p = 0; p < np; ++p) order[p] = p;
+  std::sort(order.begin(), order.end(), [&](int x, int y) { return off[x] < off[y]; });
+  std::vector<unsigned short> bit(evsl_dev::kPatCodes + 1, 0);
+  for (int p = 0; p < np; ++p) bit[order[p]] = (unsigned short)(1u << p);
+  mask.assign((size_t)n, 0);
+  for (int r = 0; r < n; ++r) {
+    bool diag = false;
+    for (int k = ia[r]; k < ia[r + 1]; ++k) {
+      if (k > ia[r] && ja[k] <= ja[k - 1]) return false;
+      diag = diag || ja[k] == r;
+      mask[r] |= bit[code[k]];  // 0 for the diagonal's code
+    }
+    if (!diag) return false;
+  }
+  return true;
+}
+
 }  // namespace
 
 int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const int* ia_h,
-                        const int* ja_h, bool owns, DevMatrix& M, size_t* red_need) {
+                        const int* ja_h, const double* a_h, bool owns, DevMatrix& M,
+                        size_t* red_need) {
   M.release();
   M.n = n;
   M.nnz = nnz;
@@ -256,55 +309,63 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
     EVSL_HIP(hipMemcpy(ja_tmp.data(), ja_d, (size_t)nnz * sizeof(int), hipMemcpyDeviceToHost));
     ja_h = ja_tmp.data();
   }
-  bool full = true;
-  for (int r = 0; r < n && full; ++r) {
+  // 16-bit column offsets when every |ja - row| fits (banded and stencil
+  // matrices in a local ordering): 2 bytes less per nonzero and filter step
+  bool full = true, fits = nnz > 0;
+  for (int r = 0; r < n && (full || fits); ++r) {
     bool has = false;
-    for (int k = ia_h[r]; k < ia_h[r + 1]; ++k)
-      if (ja_h[k] == r) {
-        has = true;
-        break;
-      }
-    full = has;
+    for (int k = ia_h[r]; k < ia_h[r + 1]; ++k) {
+      const int d = ja_h[k] - r;
+      has = has || d == 0;
+      fits = fits && d >= -32768 && d <= 32767;
+    }
+    full = full && has;
   }
   M.full_diag = full;
+  M.regular = regular_rows(n, ia_h, ja_h);
   M.tune = evsl_dev::spmm_tuner_create();
   if (!M.tune) {
     set_error_msg("out of host memory for the layout tuner");
     return EVSL_ERR_DEVICE;
   }
-  // 16-bit column offsets when every |ja - row| fits (banded and stencil
-  // matrices in a local ordering): 2 bytes less per nonzero and filter step
-  {
-    bool fits = true;
-    for (int r = 0; r < n && fits; ++r)
-      for (int k = ia_h[r]; k < ia_h[r + 1]; ++k) {
-        const long d = (long)ja_h[k] - r;
-        if (d < -32768 || d > 32767) {
-          fits = false;
-          break;
-        }
-      }
-    if (fits && nnz > 0) {
-      std::vector<short> jd((size_t)nnz);
-      for (int r = 0; r < n; ++r)
-        for (int k = ia_h[r]; k < ia_h[r + 1]; ++k) jd[k] = (short)(ja_h[k] - r);
-      EVSL_HIP(hipMalloc((void**)&M.jd, (size_t)nnz * sizeof(short)));
-      EVSL_HIP(hipMemcpy(M.jd, jd.data(), (size_t)nnz * sizeof(short), hipMemcpyHostToDevice));
-    }
+  if (fits) {
+    std::vector<short> jd((size_t)nnz);
+    for (int r = 0; r < n; ++r)
+      for (int k = ia_h[r]; k < ia_h[r + 1]; ++k) jd[k] = (short)(ja_h[k] - r);
+    EVSL_HIP(hipMalloc((void**)&M.jd, (size_t)nnz * sizeof(short)));
+    EVSL_HIP(hipMemcpy(M.jd, jd.data(), (size_t)nnz * sizeof(short), hipMemcpyHostToDevice));
   }
   // pattern codes when the off-diagonal entries take few distinct
   // (offset, value) pairs: 1 byte per nonzero for the filter kernels
   if (ctx().pattern_codes && nnz > 0) {
-    std::vector<double> a_h((size_t)nnz);
-    EVSL_HIP(hipMemcpy(a_h.data(), a_d, (size_t)nnz * sizeof(double), hipMemcpyDeviceToHost));
+    std::vector<double> a_tmp;
+    if (!a_h) {
+      a_tmp.resize((size_t)nnz);
+      EVSL_HIP(hipMemcpy(a_tmp.data(), a_d, (size_t)nnz * sizeof(double), hipMemcpyDeviceToHost));
+      a_h = a_tmp.data();
+    }
     std::vector<unsigned char> code, dpos;
     std::vector<int> off;
     std::vector<double> val, dg;
-    if (encode_pattern(n, ia_h, ja_h, a_h.data(), code, off, val, dg, dpos)) {
+    if (encode_pattern(n, ia_h, ja_h, a_h, code, off, val, dg, dpos)) {
       M.npat = (int)off.size();
       M.pshort = true;
       for (int o : off) M.pshort = M.pshort && o >= -32768 && o <= 32767;
       M.pval_h = val;
+      std::vector<unsigned short> mask;
+      if (encode_masks(n, ia_h, ja_h, code, off, val, M.mcode, mask)) {
+        M.mbytes = M.npat <= 8 ? 1 : 2;
+        M.nneg = 0;
+        for (int c : M.mcode) {
+          M.moff.push_back(off[c]);
+          M.nneg += off[c] < 0;
+        }
+        EVSL_HIP(hipMalloc(&M.rmask, (size_t)n * M.mbytes));
+        std::vector<unsigned char> m8;
+        if (M.mbytes == 1) m8.assign(mask.begin(), mask.end());
+        EVSL_HIP(hipMemcpy(M.rmask, M.mbytes == 1 ? (const void*)m8.data() : mask.data(),
+                           (size_t)n * M.mbytes, hipMemcpyHostToDevice));
+      }
       off.resize(evsl_dev::kPatCodes + 1, 0);
       val.resize(evsl_dev::kPatCodes + 1, 0.0);
       EVSL_HIP(hipMalloc((void**)&M.pc, (size_t)nnz));
@@ -350,10 +411,11 @@ int ensure_red_part(size_t need) {
 }
 
 static int register_device_csr(int n, int nnz, int* ia_d, int* ja_d, double* a_d,
-                               const int* ia_h, const int* ja_h, bool owns) {
+                               const int* ia_h, const int* ja_h, const double* a_h, bool owns) {
   Context& c = g_ctx;
   size_t need = 0;
-  if (int e = build_device_matrix(n, nnz, ia_d, ja_d, a_d, ia_h, ja_h, owns, c.A, &need)) {
+  if (int e = build_device_matrix(n, nnz, ia_d, ja_d, a_d, ia_h, ja_h, a_h, owns, c.A,
+                                  &need)) {
     c.n = 0;
     c.op = 0;
     return e;
@@ -414,6 +476,7 @@ int make_filter_op(double cc, double dd, bool f32, FilterOp* op) {
     op->A.a32 = c.A.a32s;
     op->A.pval32 = c.A.pval32s;
     op->A.dg32 = c.A.dg32s;
+    for (int p = 0; p < op->A.npair; ++p) op->A.mval32[p] = (float)(op->A.mval64[p] * scale);
     op->t1 /= scale;
     op->t2 /= scale;
     op->cc = 0.0;
@@ -542,7 +605,7 @@ int SetAMatrix(csrMat* A) {
   EVSL_HIP(hipMemcpy(ia, A->ia, (n + 1) * sizeof(int), hipMemcpyHostToDevice));
   EVSL_HIP(hipMemcpy(ja, A->ja, (size_t)nnz * sizeof(int), hipMemcpyHostToDevice));
   EVSL_HIP(hipMemcpy(a, A->a, (size_t)nnz * sizeof(double), hipMemcpyHostToDevice));
-  return register_device_csr(n, nnz, ia, ja, a, A->ia, A->ja, true);
+  return register_device_csr(n, nnz, ia, ja, a, A->ia, A->ja, A->a, true);
 }
 
 // A->ia/ja/a are device pointers (as produced by evsl_create_csr_gpu)
@@ -551,7 +614,7 @@ int SetAMatrix_device_csr(csrMat* A) {
   if (!A || A->nrows != A->ncols || A->nrows <= 0) return EVSL_ERR_ARG;
   int nnz = 0;
   EVSL_HIP(hipMemcpy(&nnz, A->ia + A->nrows, sizeof(int), hipMemcpyDeviceToHost));
-  return register_device_csr(A->nrows, nnz, A->ia, A->ja, A->a, nullptr, nullptr, false);
+  return register_device_csr(A->nrows, nnz, A->ia, A->ja, A->a, nullptr, nullptr, nullptr, false);
 }
 
 void evsl_create_csr_gpu(csrMat* Acpu, csrMat* Agpu) {

@@ -135,7 +135,7 @@ int dos_round(evslAmdServer* s, SrvRequest& q) {
   SrvMatrix& m = *s->mats[q.mat];
   const bool f32 = s->mixed;
   const size_t vs = f32 ? 4 : 8;
-  int B = 32;
+  int B = evsl_dev::kpm_max_width(m.M.n, !f32 && m.M.regular);
   while (B > q.nvec - q.done_vec) B >>= 1;
   q.B = B;
   q.k = 0;
@@ -430,7 +430,7 @@ int evsl_amd_server_add_matrix(evslAmdServer* s, csrMat* A, double lmin, double 
   EVSL_HIP(hipMemcpy(a, A->a, (size_t)nnz * sizeof(double), hipMemcpyHostToDevice));
   auto m = std::make_unique<SrvMatrix>();
   size_t need = 0;
-  if (int e = build_device_matrix(n, nnz, ia, ja, a, A->ia, A->ja, true, m->M, &need)) return e;
+  if (int e = build_device_matrix(n, nnz, ia, ja, a, A->ia, A->ja, A->a, true, m->M, &need)) return e;
   if (int e = ensure_red_part(need)) return e;
   m->lmin = lmin;
   m->lmax = lmax;

@@ -616,13 +616,17 @@ hipError_t launch_variant(const Csr& A, const void* xk, const void* xkm1, void* 
 // R = 1 layout: FP32 ChebAv 7% at 4 columns, 9% at 8, 15% at 16, 19% at 32;
 // FP64 ChebAv 2% at 4, 7% at 8, 11% at 16 and 32; the FP32 residual step
 // 7-8% at 2, 4, 16 and 32.  The FP32 KPM and FP64 residual rows (neither is
-// on a solver's hot path) keep the layouts of an earlier V-only sweep.
+// on a solver's hot path) keep the layouts of an earlier V-only sweep.  The
+// FP64 KPM row was swept for its two dots a step in both kernels that share
+// it (100^3, row-mask / CSR kernel, us): 2 columns V2R1 13.0 / 23.4 against
+// V1R1 16.9 / 24.3, 4 V2R1 19.2 / 33.1 against V1R2 28.0 / 33.9, 8 V2R2 32.8 /
+// 47.4 against V4R1 37.6 / 54.0.
 //                                    B =  2   4   6   8  16  32
 constexpr int kSpmmLayout[2][3][6] = {{{21, 22, 21, 22, 44, 44},    // FP32 ChebAv
                                        {21, 21, 21, 21, 21, 41},    // FP32 KPM
                                        {12, 14, 21, 22, 44, 44}},   // FP32 residual
                                       {{21, 12, 21, 22, 24, 24},    // FP64 ChebAv
-                                       {11, 12, 21, 41, 41, 41},    // FP64 KPM
+                                       {21, 21, 21, 22, 41, 41},    // FP64 KPM
                                        {21, 11, 21, 22, 21, 22}}};  // FP64 residual
 
 constexpr int spmm_layout(int vsize, int B, int mode) {
@@ -631,6 +635,18 @@ constexpr int spmm_layout(int vsize, int B, int mode) {
 }
 constexpr int spmm_vec(int vsize, int B, int mode) { return spmm_layout(vsize, B, mode) / 10; }
 constexpr int spmm_rows(int vsize, int B, int mode) { return spmm_layout(vsize, B, mode) % 10; }
+
+// Lane layout of the row-mask kernel (spmm_mask.h): 16-byte vectors a lane, one
+// row a lane group.  Swept over V in {1, 2, 4} and R in {1, 2} on the 100^3
+// Laplacian and the 80^3 lattice (us, V1R1 / V2R1 / V4R1 / V4R2): 8 FP32
+// columns 32.6 / 28.4 / 22.7 / 24.3, 16 on the lattice 42.3 / 32.9 / 25.7 /
+// 27.4; 4 FP64 columns 29.0 / 20.4 / - / 23.5 (V2R2 21.7).
+constexpr int mask_layout(int vsize, int B, int mode) {
+  if (mode == kKpm) return spmm_layout(vsize, B, mode);
+  if (B & 1) return 11;
+  if (vsize == 8) return 21;
+  return B % 4 ? 21 : 41;
+}
 
 template <typename VT, int B, int MODE>
 struct SpmmPolicy {

@@ -127,6 +127,13 @@ int spmm_tuner_set(SpmmTuner* t, int B, bool fp32, Mode mode, int layout) {
   return 0;
 }
 
+int spmm_tuner_forced(SpmmTuner* t, int B, bool fp32, Mode mode) {
+  SpmmTuner::Key* k = key_of(t, B, fp32, mode);
+  if (!k) return 0;
+  std::lock_guard<std::mutex> lock(t->mu);
+  return k->policy > 0 ? k->policy : 0;
+}
+
 int spmm_tuner_layout(SpmmTuner* t, int B, bool fp32, Mode mode) {
   const int table = spmm_table_layout(B, fp32, mode);
   SpmmTuner::Key* k = key_of(t, B, fp32, mode);

@@ -51,7 +51,7 @@ EXPORTS = [
     "evsl_amd_server_submit_slice", "evsl_amd_server_submit_dos", "evsl_amd_server_step",
     "evsl_amd_server_status", "evsl_amd_server_slice_result", "evsl_amd_server_dos_result",
     "evsl_amd_server_stats", "evsl_amd_set_mixed_degree_range",
-    "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
+    "evsl_amd_spmm_row_masks", "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
 ]
 
 
@@ -137,6 +137,7 @@ class EVSL:
             "evsl_amd_bench_copy": (I, [C.c_size_t, I, dp]),
             "evsl_amd_bench_dense": (I, [I, I, I, I, I, dp, dp, dp]),
             "evsl_amd_spmm_vec": (I, [I, I, I]),
+            "evsl_amd_spmm_row_masks": (I, [I, I, I]),
             "evsl_amd_spmm_layout": (I, [I, I, I, C.POINTER(I)]),
             "evsl_amd_set_spmm_layout": (I, [I, I, I, I]),
             "evsl_amd_set_spmm_tuning": (I, [I]),
@@ -470,8 +471,13 @@ class EVSL:
         """Template name of the fused filter kernel for (B, prec, mode) on
         the current matrix, as rocprofv3 reports it."""
         vt = "float" if prec == PREC_MIXED and mode != 2 else "double"
+        mask = self.lib.evsl_amd_spmm_row_masks(B, prec, mode)
         ix = self.lib.evsl_amd_spmm_index_mode(B, prec, mode)
         nt = "true" if self.lib.evsl_amd_spmm_streaming(B, prec, mode) else "false"
+        if mask:
+            lay = self.spmm_layout(B, prec, mode)[0]
+            mt = "unsigned char" if mask == 1 else "unsigned short"
+            return f"k_cheb_mask<{vt}, {B}, {lay // 10}, {lay % 10}, {mode}, {mt}, {nt}>"
         return (f"k_cheb_spmm<{vt}, {B}, {self.spmm_vec(B, prec, mode)}, {mode}, true, {ix}, "
                 f"{nt}>")
 

@@ -270,6 +270,16 @@ int evsl_amd_spmm_index_bytes(void);
  * most 8 bytes (one or two FP32 columns, one FP64 column); -1 without a
  * matrix. */
 int evsl_amd_spmm_index_mode(int B, int prec, int mode);
+/* Bytes per row of the row-mask code (no reference counterpart) the launches
+ * for (B, prec, mode) read on the current matrix, 0 when they do not.  A
+ * pattern-coded matrix (below) of at most 16 pairs, whose rows store their
+ * columns in ascending order and all store their diagonal, is also held as
+ * one bit mask per row, and its steps run k_cheb_mask<float|double, B, V, R,
+ * mode, unsigned char|unsigned short, NT> (evsl_amd_spmm_layout gives 10*V +
+ * R) -- the same products in the same order, so the results do not change --
+ * unless evsl_amd_set_spmm_layout forces a lane layout of the CSR kernel.
+ * The index modes and layouts above are the CSR kernel's. */
+int evsl_amd_spmm_row_masks(int B, int prec, int mode);
 /* Pattern codes (no reference counterpart): a matrix whose off-diagonal
  * entries take at most 255 distinct (column offset, value) pairs -- stencil
  * and lattice operators -- is stored for the filter kernels as one byte
