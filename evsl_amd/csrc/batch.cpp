@@ -266,8 +266,10 @@ int filter_columns_phased(int b, const double* const* xin, double* const* yout,
 // differ per column (same cc, dd).  Blocks wider than 8 are padded to 16 or
 // 32 with zero columns whose output goes to a scratch vector.  Nothing here
 // waits for the device.
+// deferred: a series launch's outcome is left to the caller (series_failed at
+// its next synchronisation); otherwise this waits for one.
 int filter_columns(int ncols, const double* const* xin, double* const* yout,
-                   const polparams* const* pols, bool f32, BlockWork& W) {
+                   const polparams* const* pols, bool f32, BlockWork& W, bool deferred = false) {
   Context& c = ctx();
   const int n = c.n;
   if (c.op != 1) {  // user operator: one column at a time through its MVFunc, FP64
@@ -278,6 +280,32 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
   }
   int maxdeg = 0;
   for (int j = 0; j < ncols; ++j) maxdeg = std::max(maxdeg, pols[j]->deg);
+  int mindeg = maxdeg;
+  for (int j = 0; j < ncols; ++j) mindeg = std::min(mindeg, pols[j]->deg);
+  FilterOp sop;
+  if (int e = make_filter_op(pols[0]->cc, pols[0]->dd, f32, &sop)) return e;
+  if (ncols > 0 && series_fits(sop, ncols, mindeg)) {
+    const size_t vs = f32 ? 4 : 8;
+    std::vector<const polparams*> key(pols, pols + ncols);
+    BlockWork::CoefTab* ct = nullptr;
+    // kind -2: the columns' coefficients one after the other
+    if (int e = W.coef_table(key, -2, [&](std::vector<double>& tab, std::vector<size_t>& off) {
+          for (const polparams* p : key) {
+            off.push_back(tab.size());
+            tab.insert(tab.end(), p->mu, p->mu + p->deg + 1);
+          }
+        }, &ct))
+      return e;
+    EVSL_HIP(W.bufs.alloc((size_t)2 * n * vs * ncols));
+    std::vector<SeriesCol> cols;
+    for (int j = 0; j < ncols; ++j)
+      cols.push_back({&sop, xin[j], yout[j], ct->mus.as<double>() + ct->off[j], 1, pols[j]->deg,
+                      W.bufs.as<char>() + (size_t)2 * n * vs * j});
+    if (int e = series_launch(cols)) return e;
+    if (deferred) return 0;
+    EVSL_HIP(hipStreamSynchronize(c.stream));
+    if (!series_failed()) return 0;
+  }
   const int cap = filter_block_cap(c.A.view(), f32, evsl_dev::kCheb);
   for (int j0 = 0; j0 < ncols; j0 += cap) {
     const int b = std::min(cap, ncols - j0);
@@ -842,7 +870,7 @@ struct LanczosGroup::Impl {
         }
       if (ii.empty()) continue;
       if (int e = filter_columns((int)ii.size(), ii.data(), oo.data(), pp.data(), pr == 1,
-                                 pr == 1 ? bw32 : bw64))
+                                 pr == 1 ? bw32 : bw64, true))
         return e;
     }
     return 0;
@@ -1070,20 +1098,24 @@ int LanczosGroup::step() {
   std::vector<FilterCol> cols;
   if (int e = start_cols(cols)) return e;
   if (!cols.empty()) {
-    EVSL_HIP(hipEventRecord(g.ev[0], c.stream));
-    if (int e = g.filter(cols)) return e;
-    EVSL_HIP(hipEventRecord(g.ev[1], c.stream));
-    c.astats.t_filter += elapsed(g.ev[0], g.ev[1]);
+    do {  // once, or again by launches where a series launch has failed
+      EVSL_HIP(hipEventRecord(g.ev[0], c.stream));
+      if (int e = g.filter(cols)) return e;
+      EVSL_HIP(hipEventRecord(g.ev[1], c.stream));
+      c.astats.t_filter += elapsed(g.ev[0], g.ev[1]);
+    } while (series_failed());
     if (int e = start_done()) return e;
   }
   // one blocked filter pass for all active slices
   cols.clear();
   if (int e = step_cols(cols)) return e;
   if (cols.empty()) return 0;
-  EVSL_HIP(hipEventRecord(g.ev[0], c.stream));
-  if (int e = g.filter(cols)) return e;
-  EVSL_HIP(hipEventRecord(g.ev[1], c.stream));
-  c.astats.t_filter += elapsed(g.ev[0], g.ev[1]);
+  do {
+    EVSL_HIP(hipEventRecord(g.ev[0], c.stream));
+    if (int e = g.filter(cols)) return e;
+    EVSL_HIP(hipEventRecord(g.ev[1], c.stream));
+    c.astats.t_filter += elapsed(g.ev[0], g.ev[1]);
+  } while (series_failed());
   return step_done();
 }
 

@@ -31,6 +31,14 @@ struct SpmmTuner;
 constexpr int kPatCodes = 255;
 constexpr unsigned char kPatDiag = 255;
 
+// the pairs of a row-mask code in device memory (series.hip)
+struct SeriesPairs {
+  int np, nneg;
+  int off[16];
+  double val64[16];
+  float val32[16];
+};
+
 // pairs a row-mask code holds (spmm_mask.h)
 constexpr int kMaskPairs = 18;  // 16 in use; the kernel reads whole groups of 6
 
@@ -69,6 +77,7 @@ struct Csr {
   int moff[kMaskPairs] = {};
   double mval64[kMaskPairs] = {};
   float mval32[kMaskPairs] = {};
+  const SeriesPairs* pairs = nullptr;  // the same in device memory, per precision
   // per block width: nblk+1 pairs (first row of the block, its row pointer)
   const int* rb[kNumWidths] = {};
   int nblk[kNumWidths] = {};
@@ -103,6 +112,35 @@ hipError_t cheb_spmm_mask_f32(const Csr& A, int B, Mode mode, const void* xk, co
                               void* xkp1, void* y, const void* v0, const double* s,
                               const double* mu0, double t, double cc, bool first, int yflush,
                               double* part, hipStream_t st);
+// Whole Chebyshev series in one launch (series.hip), one column a job:
+// out = sum_k mu[k * mu_step] T_k(A~) in (k = 0..deg, mu[0] for k = 0), with
+// ring holding 2 n values of the launch's type.  Needs a row-mask matrix.
+constexpr int kSeriesXcds = 8, kSeriesParts = 32, kSeriesStride = 64, kSeriesMaxJobs = 16;
+constexpr int kSeriesMaxHalf = 6, kSeriesMaxRows = 4;  // instances: pairs a side, rows a lane
+struct SeriesJob {
+  const double* in;
+  double* out;
+  const double* mu;
+  const void* rmask;
+  const void* dg;
+  void* ring;
+  const SeriesPairs* pairs;
+  double t1, t2, cc;
+  int n, deg, mu_step, mbytes;
+};
+struct SeriesArgs {
+  SeriesJob job[kSeriesMaxJobs];
+  int njobs, parts;
+  unsigned limit, id;
+  unsigned* words;   // kSeriesXcds x kSeriesStride zeros: arrivals, meetings
+  unsigned* status;  // host memory: [0] = id on failure, [1 + j] = id once job j runs
+};
+// rows per lane a matrix of n rows takes
+int series_rows_per_lane(int n);
+// half: the larger number of pairs on one side of the diagonal, over the jobs
+hipError_t cheb_series(bool fp32, const SeriesArgs& a, int half, int rows_per_lane,
+                       hipStream_t st);
+
 hipError_t cheb_spmm_mask_f64(const Csr& A, int B, Mode mode, const void* xk, const void* xkm1,
                               void* xkp1, void* y, const void* v0, const double* s,
                               const double* mu0, double t, double cc, bool first, int yflush,

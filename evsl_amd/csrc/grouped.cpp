@@ -39,9 +39,51 @@ int class_key(bool f32, int B, bool i16) { return (f32 ? 1000 : 0) + (i16 ? 100 
 
 int grouped_filter(const std::vector<GroupedCols>& parts, GroupedWork& W) {
   Context& c = ctx();
+  // ---- parts that run as series launches, every column a job ---------------
+  // (a column's coefficients stay on the device while its filter comes back)
+  // A launch runs one column an XCD, so eight columns a precision; more of them
+  // would take turns and the grouped launches below cover any number.
+  std::vector<const GroupedCols*> rest;
+  std::vector<SeriesCol> jobs[2];
+  size_t sbuf = 0, njobs[2] = {0, 0};
+  auto fits = [](const GroupedCols& p) {
+    int mindeg = p.cols[0].pol->deg;
+    for (const auto& col : p.cols) mindeg = std::min(mindeg, col.pol->deg);
+    return series_fits(p.op, (int)p.cols.size(), mindeg);
+  };
+  for (const GroupedCols& p : parts)
+    if (fits(p)) njobs[p.op.f32] += p.cols.size();
+  for (const GroupedCols& p : parts) {
+    if (njobs[p.op.f32] > evsl_dev::kSeriesXcds || !fits(p)) {
+      rest.push_back(&p);
+      continue;
+    }
+    for (const auto& col : p.cols) {
+      if (W.series.size() == sbuf) W.series.push_back(std::make_unique<GroupedWork::Bufs>());
+      GroupedWork::Bufs& bw = *W.series[sbuf++];
+      EVSL_HIP(bw.ring.alloc((size_t)2 * p.op.A.n * (p.op.f32 ? 4 : 8)));
+      const std::vector<GroupedWork::PolKey> key{{col.pol, col.pol->mu, col.pol->deg}};
+      if (key != bw.mus_key) {
+        const size_t bytes = (size_t)(col.pol->deg + 1) * sizeof(double);
+        EVSL_HIP(bw.mus.alloc(bytes));
+        EVSL_HIP(hipMemcpy(bw.mus.p, col.pol->mu, bytes, hipMemcpyHostToDevice));
+        bw.mus_key = key;
+      }
+      jobs[p.op.f32].push_back(
+          {&p.op, col.in, col.out, bw.mus.as<double>(), 1, col.pol->deg, bw.ring.p});
+    }
+  }
+  for (auto& js : jobs) {
+    if (js.empty()) continue;
+    // the longest series first: an XCD takes every eighth job
+    std::stable_sort(js.begin(), js.end(),
+                     [](const SeriesCol& x, const SeriesCol& y) { return x.deg > y.deg; });
+    if (int e = series_launch(js)) return e;
+  }
   // ---- blocks of at most 8 columns; degree-0 filters directly -------------
   std::vector<Block> blocks;
-  for (const GroupedCols& p : parts) {
+  for (const GroupedCols* pp : rest) {
+    const GroupedCols& p = *pp;
     const int nc = (int)p.cols.size();
     for (int c0 = 0; c0 < nc; c0 += kGroupMaxWidth) {
       Block b;

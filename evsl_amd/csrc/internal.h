@@ -79,6 +79,8 @@ struct DevMatrix {
   float* dg32s = nullptr;
   // row masks (evsl_dev::Csr::rmask): pair p is table entry mcode[p]
   void* rmask = nullptr;
+  evsl_dev::SeriesPairs* pairs64 = nullptr;
+  evsl_dev::SeriesPairs* pairs32s = nullptr;  // of the shifted FP32 copy
   int mbytes = 0, nneg = 0;
   std::vector<int> mcode, moff;
   // bytes per nonzero of the column index the filter kernels read
@@ -115,6 +117,24 @@ int ensure_red_part(size_t need);
 // matrix lacks stored diagonal entries
 int ensure_a32_shifted(double cc, double scale, bool* ok);
 
+// Series launches (series.cpp): the meetings' device counters, the launches whose
+// outcome has not been read yet, and where they report it
+struct SeriesState {
+  static constexpr int kSlots = 64;     // launches between two checks
+  static constexpr int kSets = 256;     // counter sets (launches between clearings)
+  DevBuf words;
+  unsigned* status = nullptr;           // pinned, kSlots x (1 + kSeriesMaxJobs)
+  unsigned* status_d = nullptr;
+  unsigned id = 0;
+  int limit = 200000;                   // polls of one wait; 0: no series launches
+  bool off = false;                     // a launch has failed
+  struct Pending {
+    unsigned id;
+    int njobs;
+  };
+  std::vector<Pending> pending;         // slot = position
+};
+
 struct Context {
   bool started = false;
   int n = 0;
@@ -145,6 +165,7 @@ struct Context {
   DevBuf red_part, red_scalars;
   // pinned host scalars for device->host reads
   double* pinned = nullptr;
+  SeriesState series;
   evslAmdStats astats;
 };
 
@@ -212,6 +233,25 @@ int make_filter_op(double cc, double dd, bool f32, FilterOp* op);
 // exists (a shifted copy is recomputed in place for another cc, dd)
 bool filter_op_ready(bool f32);
 
+// ---- whole series in one launch (series.cpp) ---------------------------------
+// Whether ncols columns of op's matrix run as a series launch of this degree.
+bool series_fits(const FilterOp& op, int ncols, int deg);
+// One column: out = sum_k mu[k * mu_step] T_k(A~) in, mu on the device, ring of
+// 2 n values of op's vector type.
+struct SeriesCol {
+  const FilterOp* op;
+  const double* in;
+  double* out;
+  const double* mu;
+  int mu_step, deg;
+  void* ring;
+};
+// Launches the columns (every op of one precision).  Nothing waits: after the
+// next synchronisation the caller asks series_failed, and where that is true
+// filters the same columns again, by launches (series launches are off then).
+int series_launch(const std::vector<SeriesCol>& cols);
+bool series_failed();
+
 // ---- filter application (lanczos.cpp) -----------------------------------
 struct ChebWork {
   DevBuf bufs;  // 3 n-vectors
@@ -221,8 +261,10 @@ struct ChebWork {
   int deg_loaded = -1;
   const double* mu_src = nullptr;
 };
-// y = p(A) v (device vectors) with pol; FP64 or FP32 per ctx().filter_prec
-int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int prec);
+// y = p(A) v (device vectors) with pol; FP64 or FP32 per ctx().filter_prec.
+// deferred: the caller asks series_failed at its next synchronisation
+int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int prec,
+            bool deferred = false);
 
 // ---- Lanczos building blocks (lanczos.cpp) ----------------------------------
 // check_intv of INC/internal_header.h:194-217: -1 empty interval, -2 outside
@@ -313,7 +355,7 @@ struct GroupedWork {
     std::vector<PolKey> mus_key;
     int mus_deg = -1;
   };
-  std::vector<std::unique_ptr<Bufs>> bufs;
+  std::vector<std::unique_ptr<Bufs>> bufs, series;
   DevBuf d_tab, d_owner;
   std::vector<int> owner_h;
 };

@@ -87,7 +87,8 @@ double filter_step_bytes(const Context& c, int B, int sa, double vec_bytes) {
 // ---------------------------------------------------------------------
 // y = p((A - cc)/dd) v  -- one fused SpMM launch per degree
 // ---------------------------------------------------------------------
-int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int prec) {
+int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int prec,
+            bool deferred) {
   Context& c = ctx();
   const int n = c.n, m = pol->deg;
   const double cc = pol->cc, t1 = 1.0 / pol->dd, t2 = 2.0 / pol->dd;
@@ -111,6 +112,13 @@ int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int p
     const size_t vs = f32 ? sizeof(float) : sizeof(double);
     FilterOp op;
     if (int e = make_filter_op(cc, pol->dd, f32, &op)) return e;
+    if (series_fits(op, 1, m)) {
+      EVSL_HIP(w.bufs.alloc((size_t)2 * n * vs));
+      if (int e = series_launch({{&op, v, y, mu_d, 1, m, w.bufs.p}})) return e;
+      if (deferred) return 0;
+      EVSL_HIP(hipStreamSynchronize(c.stream));
+      if (!series_failed()) return 0;
+    }
     // the kernel accumulates y in FP64 in both precisions, straight into
     // the caller's vector
     DevBuf& store = f32 ? w.b32 : w.bufs;
@@ -341,19 +349,21 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
     double* v = V + (size_t)k * nl;
     double* vnew = v + nl;
     const double* zold = k > 0 ? v - nl : nullptr;
-    clk.mark(0);
-    if (int e = cheb_av(pol, v, vnew, L.cw, prec)) return e;
-    clk.mark(1);
-    // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; ||vnew||^2
-    if (zold)
-      EVSL_HIP(evsl_dev::axpy_dot(n, -beta, zold, vnew, v, red_part(), c.stream));
-    else
-      EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, red_part(), c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-    EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, red_scalar(0), v, vnew, red_part(), c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(1), c.stream));
     double sc[2];
-    if (int e = read_scalars(red_scalar(0), 2, sc)) return e;
+    do {  // once, or again by launches where a series launch has failed
+      clk.mark(0);
+      if (int e = cheb_av(pol, v, vnew, L.cw, prec, true)) return e;
+      clk.mark(1);
+      // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; ||vnew||^2
+      if (zold)
+        EVSL_HIP(evsl_dev::axpy_dot(n, -beta, zold, vnew, v, red_part(), c.stream));
+      else
+        EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, red_part(), c.stream));
+      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(0), c.stream));
+      EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, red_scalar(0), v, vnew, red_part(), c.stream));
+      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(1), c.stream));
+      if (int e = read_scalars(red_scalar(0), 2, sc)) return e;
+    } while (series_failed());
     const double alpha = sc[0];
     dT[k] = alpha;
     wn += std::fabs(alpha);

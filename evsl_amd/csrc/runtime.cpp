@@ -71,6 +71,7 @@ evsl_dev::Csr DevMatrix::view() const {
     c.mbytes = mbytes;
     c.npair = (int)mcode.size();
     c.nneg = nneg;
+    c.pairs = pairs64;
     for (int p = 0; p < c.npair; ++p) {
       c.moff[p] = moff[p];
       c.mval64[p] = pval_h[mcode[p]];
@@ -97,7 +98,8 @@ void DevMatrix::release() {
   if (a32) (void)hipFree(a32);
   if (a32s) (void)hipFree(a32s);
   for (void* p : {(void*)pc, (void*)pdpos, (void*)poff, (void*)pval64, (void*)dg64, (void*)pval32,
-                  (void*)dg32, (void*)pval32s, (void*)dg32s, rmask})
+                  (void*)dg32, (void*)pval32s, (void*)dg32s, rmask, (void*)pairs64,
+                  (void*)pairs32s})
     if (p) (void)hipFree(p);
   evsl_dev::spmm_tuner_destroy(tune);
   *this = DevMatrix();
@@ -286,6 +288,22 @@ bool encode_masks(int n, const int* ia, const int* ja, const std::vector<unsigne
   return true;
 }
 
+// the row-mask pairs with values times scale (FP32: rounded after it, as
+// shift_scale_f32 does)
+int upload_pairs(const DevMatrix& M, double scale, evsl_dev::SeriesPairs** d) {
+  evsl_dev::SeriesPairs h{};
+  h.np = (int)M.mcode.size();
+  h.nneg = M.nneg;
+  for (int p = 0; p < h.np; ++p) {
+    h.off[p] = M.moff[p];
+    h.val64[p] = M.pval_h[M.mcode[p]];
+    h.val32[p] = (float)(h.val64[p] * scale);
+  }
+  if (!*d) EVSL_HIP(hipMalloc((void**)d, sizeof(h)));
+  EVSL_HIP(hipMemcpy(*d, &h, sizeof(h), hipMemcpyHostToDevice));
+  return 0;
+}
+
 }  // namespace
 
 int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const int* ia_h,
@@ -363,6 +381,7 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
         EVSL_HIP(hipMalloc(&M.rmask, (size_t)n * M.mbytes));
         std::vector<unsigned char> m8;
         if (M.mbytes == 1) m8.assign(mask.begin(), mask.end());
+        if (int e = upload_pairs(M, 1.0, &M.pairs64)) return e;
         EVSL_HIP(hipMemcpy(M.rmask, M.mbytes == 1 ? (const void*)m8.data() : mask.data(),
                            (size_t)n * M.mbytes, hipMemcpyHostToDevice));
       }
@@ -447,6 +466,8 @@ int ensure_a32_shifted(double cc, double scale, bool* ok) {
     EVSL_HIP(hipMemcpy(c.A.pval32s, pv.data(), pv.size() * sizeof(float), hipMemcpyHostToDevice));
     if (!c.A.dg32s) EVSL_HIP(hipMalloc((void**)&c.A.dg32s, (size_t)std::max(c.A.n, 1) * sizeof(float)));
     EVSL_HIP(evsl_dev::shift_diag_f32(c.A.n, c.A.dg64, cc, scale, c.A.dg32s, c.stream));
+    if (c.A.rmask)
+      if (int e = upload_pairs(c.A, scale, &c.A.pairs32s)) return e;
   }
   c.A.shift_cc = cc;
   c.A.shift_scale = scale;
@@ -476,6 +497,7 @@ int make_filter_op(double cc, double dd, bool f32, FilterOp* op) {
     op->A.a32 = c.A.a32s;
     op->A.pval32 = c.A.pval32s;
     op->A.dg32 = c.A.dg32s;
+    op->A.pairs = c.A.pairs32s;
     for (int p = 0; p < op->A.npair; ++p) op->A.mval32[p] = (float)(op->A.mval64[p] * scale);
     op->t1 /= scale;
     op->t2 /= scale;
@@ -582,6 +604,10 @@ int EVSLFinish(void) {
   c.red_scalars.release();
   if (c.pinned) (void)hipHostFree(c.pinned);
   c.pinned = nullptr;
+  if (c.series.status) (void)hipHostFree(c.series.status);
+  c.series.status = nullptr;
+  c.series.words.release();
+  c.series.pending.clear();
   c.op = 0;
   c.n = 0;
   c.func = nullptr;
@@ -745,6 +771,12 @@ int evsl_amd_set_refine_guard(double guard) {
 }
 int evsl_amd_set_grouped_filter(int on) {
   ctx().grouped_filter = on != 0;
+  return 0;
+}
+int evsl_amd_set_series_polls(int polls) {
+  if (polls < 0) return EVSL_ERR_ARG;
+  ctx().series.limit = polls;
+  ctx().series.off = false;
   return 0;
 }
 int evsl_amd_set_refine_widen(double widen) {

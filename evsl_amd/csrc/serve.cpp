@@ -263,6 +263,8 @@ int grouped_pass(evslAmdServer* s, const std::vector<int>& live, bool start) {
     EVSL_HIP(hipEventSynchronize(s->ev[1]));
     EVSL_HIP(hipEventElapsedTime(&ms, s->ev[0], s->ev[1]));
     c.astats.t_filter += ms * 1e-3;
+    // a failed series launch: the same columns once more, by launches
+    if (series_failed()) return grouped_pass(s, live, start);
   }
   if (start)
     for (int mi : live) {

@@ -51,7 +51,7 @@ EXPORTS = [
     "evsl_amd_server_submit_slice", "evsl_amd_server_submit_dos", "evsl_amd_server_step",
     "evsl_amd_server_status", "evsl_amd_server_slice_result", "evsl_amd_server_dos_result",
     "evsl_amd_server_stats", "evsl_amd_set_mixed_degree_range",
-    "evsl_amd_spmm_row_masks", "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
+    "evsl_amd_set_series_polls", "evsl_amd_spmm_row_masks", "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
 ]
 
 
@@ -138,6 +138,7 @@ class EVSL:
             "evsl_amd_bench_dense": (I, [I, I, I, I, I, dp, dp, dp]),
             "evsl_amd_spmm_vec": (I, [I, I, I]),
             "evsl_amd_spmm_row_masks": (I, [I, I, I]),
+            "evsl_amd_set_series_polls": (I, [I]),
             "evsl_amd_spmm_layout": (I, [I, I, I, C.POINTER(I)]),
             "evsl_amd_set_spmm_layout": (I, [I, I, I, I]),
             "evsl_amd_set_spmm_tuning": (I, [I]),
@@ -480,6 +481,10 @@ class EVSL:
             return f"k_cheb_mask<{vt}, {B}, {lay // 10}, {lay % 10}, {mode}, {mt}, {nt}>"
         return (f"k_cheb_spmm<{vt}, {B}, {self.spmm_vec(B, prec, mode)}, {mode}, true, {ix}, "
                 f"{nt}>")
+
+    def set_series_polls(self, polls):
+        """Bound of a series launch's waits; 0 filters one launch a degree."""
+        return self.lib.evsl_amd_set_series_polls(polls)
 
     def set_pattern_codes(self, on):
         return self.lib.evsl_amd_set_pattern_codes(1 if on else 0)

@@ -198,6 +198,14 @@ int evsl_amd_server_stats(evslAmdServer *s, int *queued, int *running, size_t *m
  * the default) or one matrix at a time (0); results are the same bits */
 int evsl_amd_set_grouped_filter(int on);
 
+/* Filters of small row-mask matrices (evsl_amd_spmm_row_masks) run all their
+ * degrees in one launch, whose workgroups wait for each other at every degree.
+ * A wait ends after `polls` looks at the others (default 200000, tens of
+ * milliseconds); the filter is then run again, one launch a degree, as all
+ * later ones are until the next call of this function.  0 runs every filter
+ * one launch a degree.  Results are the same bits either way. */
+int evsl_amd_set_series_polls(int polls);
+
 /* Matrix Market coordinate reader of the reference drivers
  * (TESTS/COMMON/io.c:115-217, read_coo_MM): real/integer, general/symmetric
  * (the stored triangle, then its mirrored off-diagonal entries); indices
