@@ -429,8 +429,6 @@ hipError_t shift_scale_f32(const Csr& A, double cc, double scale, float* out, hi
 // copy, with shift_scale_f32's arithmetic
 hipError_t shift_diag_f32(int n, const double* d, double cc, double scale, float* out,
                           hipStream_t st);
-// Z (k x k, column-major) = identity
-hipError_t set_identity(int k, double* Z, hipStream_t st);
 // precision conversions
 hipError_t f64_to_f32(size_t n, const double* x, float* y, hipStream_t st);
 hipError_t f32_to_f64(size_t n, const float* x, double* y, hipStream_t st);
@@ -482,12 +480,16 @@ hipError_t col_resid(size_t n, int m, const double* W, size_t ldw, const double*
 hipError_t gather_cols(size_t nrow, int m, const double* src, size_t lds, const int* idx,
                        double* dst, size_t ldd, hipStream_t st);
 
-// Apply the plane rotations recorded by the implicit-QL tridiagonal solver to
-// the k x k column-major matrix Z (thread per row).  Sweep s covers rotation
-// indices i = top[s], top[s]-1, ..., top[s]-cnt[s]+1 with cosines/sines
-// cs[2*(off[s]+j)], cs[2*(off[s]+j)+1].
-hipError_t apply_rotations(int k, double* Z, int nsweep, const int* top, const int* cnt,
-                           const long long* off, const double* cs, hipStream_t st);
+// Replay the plane rotations recorded by the implicit-QL tridiagonal solver:
+// Zsel (k x m, column-major) = the columns cols[0..m) of Z = I * rotations.
+// Sweep s covers rotation indices i = top[s], top[s]-1, ..., top[s]-cnt[s]+1;
+// cs holds the nrot (cosine, sine) pairs of all sweeps one after the other.
+// rotations_rows: rows of Z a block holds in LDS, 0 where one does not fit
+// (k > 6144; the caller then replays on the host).
+int rotations_rows(int k);
+hipError_t replay_rotations(int k, int nsweep, const int* top, const int* cnt, int nrot,
+                            const double* cs, int m, const int* cols, double* Zsel,
+                            hipStream_t st);
 
 // block (row-major, B columns) helpers
 // out[c] = ||X(:,c)||^2 partials -> finalised into out (B values)

@@ -86,6 +86,22 @@ int tridiag_ql(int n, double* d, double* e, RotationLog* rec) {
   return 0;
 }
 
+// the recorded rotations on one row of Z
+static void replay_row(const RotationLog& rec, double* z) {
+  for (size_t sw = 0; sw < rec.top.size(); ++sw) {
+    const int ihi = rec.top[sw], cnt = rec.cnt[sw];
+    const double* rot = rec.cs.data() + 2 * rec.off[sw];
+    double carry = z[ihi + 1];
+    for (int j = 0; j < cnt; ++j) {
+      const int i = ihi - j;
+      const double zi = z[i];
+      z[i + 1] = rot[2 * j + 1] * zi + rot[2 * j] * carry;
+      carry = rot[2 * j] * zi - rot[2 * j + 1] * carry;
+    }
+    z[ihi - cnt + 1] = carry;
+  }
+}
+
 int tridiag_eig_host(int n, const double* diag, const double* sdiag, double* eval, double* Z) {
   std::vector<double> e(n + 1, 0.0);
   std::memcpy(eval, diag, n * sizeof(double));
@@ -186,23 +202,8 @@ int sym_eig_host(int n, const double* A, int lda, double* Q, int ldq, double* la
   for (int r = 0; r < n; ++r)
     for (int c = 0; c < n; ++c) R[(size_t)r * n + c] = Z[r + (size_t)c * n];
   // rows are independent: each applies every sweep in order
-  const size_t nsw = rec.top.size();
 #pragma omp parallel for schedule(static) if (n > 128)
-  for (int r = 0; r < n; ++r) {
-    double* z = R.data() + (size_t)r * n;
-    for (size_t sw = 0; sw < nsw; ++sw) {
-      const int ihi = rec.top[sw], cnt = rec.cnt[sw];
-      const double* rot = rec.cs.data() + 2 * rec.off[sw];
-      double carry = z[ihi + 1];
-      for (int j = 0; j < cnt; ++j) {
-        const int i = ihi - j;
-        const double zi = z[i];
-        z[i + 1] = rot[2 * j + 1] * zi + rot[2 * j] * carry;
-        carry = rot[2 * j] * zi - rot[2 * j + 1] * carry;
-      }
-      z[ihi - cnt + 1] = carry;
-    }
-  }
+  for (int r = 0; r < n; ++r) replay_row(rec, R.data() + (size_t)r * n);
   for (int j = 0; j < n; ++j)
     for (int r = 0; r < n; ++r) Q[r + (size_t)j * ldq] = R[(size_t)r * n + rec.perm[j]];
   return 0;
@@ -211,33 +212,41 @@ int sym_eig_host(int n, const double* A, int lda, double* Q, int ldq, double* la
 int tridiag_rotations_to_device(int kdim, const RotationLog& rec, const std::vector<int>& sel,
                                 double* Zsel_d) {
   Context& c = ctx();
-  const int nsw = (int)rec.top.size();
-  const size_t kk = (size_t)kdim * kdim;
-  DevBuf Z, top, cnt, off, cs, idx;
-  EVSL_HIP(Z.alloc(kk * sizeof(double)));
-  EVSL_HIP(evsl_dev::set_identity(kdim, Z.as<double>(), c.stream));
-  if (nsw > 0) {
-    EVSL_HIP(top.alloc(nsw * sizeof(int)));
-    EVSL_HIP(cnt.alloc(nsw * sizeof(int)));
-    EVSL_HIP(off.alloc(nsw * sizeof(long long)));
-    EVSL_HIP(cs.alloc(std::max<size_t>(rec.cs.size(), 2) * sizeof(double)));
-    EVSL_HIP(hipMemcpy(top.p, rec.top.data(), nsw * sizeof(int), hipMemcpyHostToDevice));
-    EVSL_HIP(hipMemcpy(cnt.p, rec.cnt.data(), nsw * sizeof(int), hipMemcpyHostToDevice));
-    EVSL_HIP(hipMemcpy(off.p, rec.off.data(), nsw * sizeof(long long), hipMemcpyHostToDevice));
+  const int nsw = (int)rec.top.size(), m = (int)sel.size();
+  if (m == 0) return 0;
+  std::vector<int> cols(m);
+  for (int j = 0; j < m; ++j) cols[j] = rec.perm[sel[j]];
+  if (evsl_dev::rotations_rows(kdim) == 0) {  // a row of Z outgrows a block's LDS
+    std::vector<double> Z((size_t)kdim * m);
+#pragma omp parallel
+    {
+      std::vector<double> z(kdim);
+#pragma omp for schedule(static)
+      for (int r = 0; r < kdim; ++r) {
+        std::fill(z.begin(), z.end(), 0.0);
+        z[r] = 1.0;
+        replay_row(rec, z.data());
+        for (int j = 0; j < m; ++j) Z[(size_t)j * kdim + r] = z[cols[j]];
+      }
+    }
+    EVSL_HIP(hipMemcpy(Zsel_d, Z.data(), Z.size() * sizeof(double), hipMemcpyHostToDevice));
+    return 0;
+  }
+  DevBuf sweeps, cs;
+  const int nrot = (int)(rec.cs.size() / 2);
+  std::vector<int> h;  // tops, counts, columns
+  h.insert(h.end(), rec.top.begin(), rec.top.end());
+  h.insert(h.end(), rec.cnt.begin(), rec.cnt.end());
+  h.insert(h.end(), cols.begin(), cols.end());
+  EVSL_HIP(sweeps.alloc(h.size() * sizeof(int)));
+  EVSL_HIP(cs.alloc(std::max<size_t>(rec.cs.size(), 2) * sizeof(double)));
+  EVSL_HIP(hipMemcpy(sweeps.p, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (nrot > 0)
     EVSL_HIP(hipMemcpy(cs.p, rec.cs.data(), rec.cs.size() * sizeof(double),
                        hipMemcpyHostToDevice));
-    EVSL_HIP(evsl_dev::apply_rotations(kdim, Z.as<double>(), nsw, top.as<int>(), cnt.as<int>(),
-                                       off.as<long long>(), cs.as<double>(), c.stream));
-  }
-  const int m = (int)sel.size();
-  if (m > 0) {
-    std::vector<int> cols(m);
-    for (int j = 0; j < m; ++j) cols[j] = rec.perm[sel[j]];
-    EVSL_HIP(idx.alloc(m * sizeof(int)));
-    EVSL_HIP(hipMemcpy(idx.p, cols.data(), m * sizeof(int), hipMemcpyHostToDevice));
-    EVSL_HIP(evsl_dev::gather_cols(kdim, m, Z.as<double>(), kdim, idx.as<int>(), Zsel_d, kdim,
-                                   c.stream));
-  }
+  const int* d = sweeps.as<int>();
+  EVSL_HIP(evsl_dev::replay_rotations(kdim, nsw, d, d + nsw, nrot, cs.as<double>(), m, d + 2 * nsw,
+                                      Zsel_d, c.stream));
   EVSL_HIP(hipStreamSynchronize(c.stream));
   return 0;
 }
