@@ -853,6 +853,7 @@ struct LanczosGroup::Impl {
   std::vector<std::unique_ptr<Slot>> slots;
   DevBuf gt_part, hbuf, scal_d, vrand, parts;
   int kcap = 0, scap = 0;
+  size_t gt_stride = 0;
   BlockWork bw32, bw64;  // the FP32 and the FP64 blocked filter passes
   std::vector<int> st_cur, act_cur;  // slots of the phase in progress
   // filters the columns in -> out of this group's matrix, one pass per
@@ -933,21 +934,77 @@ struct LanczosGroup::Impl {
     }
     return 0;
   }
-  hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
-  size_t part_stride() const {
-    const int n = ctx().n;
-    return std::max((size_t)evsl_dev::kRedBlocks, (size_t)(n + evsl_dev::kWG - 1) / evsl_dev::kWG);
+  // the column of slot s at its step k: vnew against the first k + 1 basis vectors
+  evsl_dev::LanCol lan_col(int s) {
+    Slot& sl = *slots[s];
+    Slice& L = sl.L;
+    const int n = ctx().n, k = sl.k;
+    evsl_dev::LanCol q{};
+    q.zold = k > 0 ? L.vcol(k - 1, n) : nullptr;
+    q.v = L.vcol(k, n);
+    q.vnew = L.vcol(k + 1, n);
+    q.V = L.V.as<double>();
+    q.V32 = L.V32.as<float>();
+    q.ld32 = L.ld32;
+    q.beta = L.beta;
+    q.part = part_of(s);
+    q.out = scal_d.as<double>() + 4 * s;
+    q.k = k + 1;
+    return q;
   }
+  // runs `go(columns, count)` over the slots, at most kLanCols at a time
+  template <typename Go>
+  int by_cols(const std::vector<int>& ids, Go go) {
+    for (size_t i0 = 0; i0 < ids.size(); i0 += evsl_dev::kLanCols) {
+      evsl_dev::LanCols cols{};
+      const int nc = (int)std::min((size_t)evsl_dev::kLanCols, ids.size() - i0);
+      for (int j = 0; j < nc; ++j) {
+        cols.c[j] = lan_col(ids[i0 + j]);
+        cols.c[j].gt = gt_part.as<double>() + gt_stride * j;
+      }
+      if (int e = go(cols, nc, &ids[i0])) return e;
+    }
+    return 0;
+  }
+  // A Gram-Schmidt pass of the slots' new vectors and the sums of their norms
+  // (second: of a further pass).  Small matrices: the slots of one basis
+  // precision together; the others one after the other.
+  int cgs_all(const std::vector<int>& ids, bool second) {
+    Context& c = ctx();
+    const int n = c.n;
+    const bool small = evsl_dev::lan_small(n);
+    for (int f32 = 0; f32 < 2; ++f32) {
+      std::vector<int> sub;
+      for (int s : ids)
+        if (slots[s]->L.has32() == (f32 == 1)) sub.push_back(s);
+      if (int e = by_cols(sub, [&](evsl_dev::LanCols& cols, int nc, const int* id) -> int {
+            if (small) {
+              EVSL_HIP(evsl_dev::lan_gram_schmidt(n, cols, nc, f32 == 1, c.stream));
+            } else {
+              for (int j = 0; j < nc; ++j)
+                if (int e2 = cgs_pass(slots[id[j]]->L, slots[id[j]]->k, cols.c[j].vnew,
+                                      cols.c[j].part + 2 * evsl_dev::kRedBlocks, &cols.c[j].np))
+                  return e2;
+            }
+            EVSL_HIP(evsl_dev::lan_sums(n, cols, nc, second, c.stream));
+            return 0;
+          }))
+        return e;
+    }
+    return 0;
+  }
+  hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+  size_t part_stride() const { return evsl_dev::lan_part_elems(ctx().n); }
   double* part_of(int s) { return parts.as<double>() + (size_t)s * part_stride(); }
   int ensure(int maxit) {
     const int n = ctx().n;
     const int ns = (int)slots.size();
-    if (maxit > kcap) {
-      const int nch = evsl_dev::gemv_t_chunks(n);
-      EVSL_HIP(gt_part.alloc((size_t)nch * (maxit + 1) * sizeof(double)));
-      EVSL_HIP(hbuf.alloc((size_t)(maxit + 1) * sizeof(double)));
-      kcap = maxit;
-    }
+    // V^T w partials of kLanCols columns side by side where they run together
+    kcap = std::max(kcap, maxit);
+    gt_stride = (size_t)evsl_dev::gemv_t_chunks(n) * (kcap + 1);
+    EVSL_HIP(gt_part.alloc(gt_stride * (evsl_dev::lan_small(n) ? evsl_dev::kLanCols : 1) *
+                           sizeof(double)));
+    EVSL_HIP(hbuf.alloc((size_t)(kcap + 1) * sizeof(double)));
     if (ns > scap) {
       EVSL_HIP(scal_d.alloc((size_t)4 * ns * sizeof(double)));
       EVSL_HIP(parts.alloc(part_stride() * ns * sizeof(double)));
@@ -1141,25 +1198,14 @@ int LanczosGroup::step_done() {
   const int b = (int)act.size();
   EVSL_HIP(hipEventRecord(g.ev[1], c.stream));
 
-  // ---- recurrence: vnew -= beta vold; alpha; vnew -= alpha v; ||vnew||^2 -----
-  for (int s : act) {
-    Impl::Slot& sl = *g.slots[s];
-    Slice& L = sl.L;
-    const int k = sl.k;
-    double* v = L.vcol(k, n);
-    double* vnew = L.vcol(k + 1, n);
-    if (k > 0)
-      EVSL_HIP(evsl_dev::axpy_dot(n, -L.beta, L.vcol(k - 1, n), vnew, v, g.part_of(s), c.stream));
-    else
-      EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, g.part_of(s), c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(g.part_of(s), evsl_dev::kRedBlocks, sc_d + 4 * s, c.stream));
-    EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, sc_d + 4 * s, v, vnew, g.part_of(s), c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(g.part_of(s), evsl_dev::kRedBlocks, sc_d + 4 * s + 1, c.stream));
-    // first Gram-Schmidt pass
-    int np = 0;
-    if (int e = g.cgs_pass(L, k, vnew, g.part_of(s), &np)) return e;
-    EVSL_HIP(evsl_dev::sum_scalar(g.part_of(s), np, sc_d + 4 * s + 2, c.stream));
-  }
+  // ---- recurrence: vnew -= beta vold; alpha; vnew -= alpha v; ||vnew||^2;
+  // first Gram-Schmidt pass -----
+  if (int e = g.by_cols(act, [&](evsl_dev::LanCols& cols, int nc, const int*) -> int {
+        EVSL_HIP(evsl_dev::lan_recurrence(n, cols, nc, c.stream));
+        return 0;
+      }))
+    return e;
+  if (int e = g.cgs_all(act, false)) return e;
   std::vector<double> hs(4 * g.slots.size());
   EVSL_HIP(hipMemcpy(hs.data(), sc_d, hs.size() * sizeof(double), hipMemcpyDeviceToHost));
   std::vector<int> second;
@@ -1175,21 +1221,16 @@ int LanczosGroup::step_done() {
     c.astats.reorth_bytes += Impl::cgs_bytes(L, n, k);
     if (!(L.nrm > eta * old_nrm)) second.push_back(s);
   }
+  if (int e = g.cgs_all(second, true)) return e;
   for (int s : second) {
-    Impl::Slot& sl = *g.slots[s];
-    Slice& L = sl.L;
-    const int k = sl.k;
-    double* vnew = L.vcol(k + 1, n);
-    int np = 0;
-    if (int e = g.cgs_pass(L, k, vnew, g.part_of(s), &np)) return e;
-    EVSL_HIP(evsl_dev::sum_scalar(g.part_of(s), np, sc_d + 4 * s + 3, c.stream));
     c.astats.n_reorth_pass++;
-    c.astats.reorth_bytes += Impl::cgs_bytes(L, n, k);
+    c.astats.reorth_bytes += Impl::cgs_bytes(g.slots[s]->L, n, g.slots[s]->k);
   }
   if (!second.empty()) {
     EVSL_HIP(hipMemcpy(hs.data(), sc_d, hs.size() * sizeof(double), hipMemcpyDeviceToHost));
     for (int s : second) g.slots[s]->L.nrm = std::sqrt(hs[4 * s + 3]);
   }
+  std::vector<int> scaled;
   for (int s : act) {
     Impl::Slot& sl = *g.slots[s];
     Slice& L = sl.L;
@@ -1220,10 +1261,20 @@ int LanczosGroup::step_done() {
       if (int e = g.scal_col(L, k + 1, 1.0 / nn)) return e;
       L.beta = 0.0;
     } else {
-      if (int e = g.scal_col(L, k + 1, 1.0 / L.beta)) return e;
+      scaled.push_back(s);
     }
     L.eT[k] = L.beta;
   }
+  if (int e = g.by_cols(scaled, [&](evsl_dev::LanCols& cols, int nc, const int* id) -> int {
+        for (int j = 0; j < nc; ++j) {
+          Slice& L = g.slots[id[j]]->L;
+          cols.c[j].beta = 1.0 / L.beta;
+          cols.c[j].x32 = L.has32() ? L.v32col(g.slots[id[j]]->k + 1) : nullptr;
+        }
+        EVSL_HIP(evsl_dev::lan_scale(n, cols, nc, c.stream));
+        return 0;
+      }))
+    return e;
   EVSL_HIP(hipEventRecord(g.ev[2], c.stream));
   c.astats.t_reorth += elapsed(g.ev[1], g.ev[2]);
   c.astats.n_lanczos += b;

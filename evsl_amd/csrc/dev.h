@@ -409,12 +409,6 @@ hipError_t sum_scalar(const double* part, int cnt, double* out, hipStream_t st);
 // y += a*x (a on host); part = partial of y.z   (z may be null: no dot)
 hipError_t axpy_dot(size_t n, double a, const double* x, double* y, const double* z,
                     double* part, hipStream_t st);
-// y += sign * (*a_d) * x; part = partial of y.y
-hipError_t axpy_dev_nrm(size_t n, double sign, const double* a_d, const double* x,
-                        double* y, double* part, hipStream_t st);
-// y += sign * (*a_d) * x; part = partial of y.z
-hipError_t axpy_dev_dot(size_t n, double sign, const double* a_d, const double* x,
-                        double* y, const double* z, double* part, hipStream_t st);
 // x *= a
 hipError_t scal(size_t n, double a, double* x, hipStream_t st);
 // y = a * x
@@ -441,9 +435,6 @@ hipError_t gemv_t(size_t n, int k, const double* V, size_t ld, const double* w,
                   double* part, double* h, hipStream_t st);
 hipError_t gemv_n_sub_nrm(size_t n, int k, const double* V, size_t ld, const double* h,
                           double* w, double* part, hipStream_t st);
-// y = V h (no subtraction)
-hipError_t gemv_n(size_t n, int k, const double* V, size_t ld, const double* h, double* y,
-                  hipStream_t st);
 // The same pass against an FP32 copy of the basis (ld even, columns 8-byte
 // aligned), FP64 products and sums; gemv_n_sub_nrm_f32 leaves
 // gemv_n_sub_f32_blocks(n) partials of ||w||^2 (one per 512 rows).
@@ -454,6 +445,52 @@ hipError_t gemv_n_sub_nrm_f32(size_t n, int k, const float* V, size_t ld, const 
                               double* w, double* part, hipStream_t st);
 // x *= a, x32 = (float)x
 hipError_t scal_f32copy(size_t n, double a, double* x, float* x32, hipStream_t st);
+
+// The vector work of a Lanczos step for up to kLanCols columns at once
+// (lanstep.hip).  A column's basis is V (column-major, ld n) or its FP32 copy V32
+// (ld32 even), k of its columns in use; part holds lan_part_elems(n) doubles, gt
+// and gt2 gemv_t_chunks(n) * k each.
+constexpr int kLanCols = 8;
+struct LanCol {
+  const double* zold;    // previous basis vector, null: none
+  const double* v;       // current one
+  double* vnew;
+  const double* V;
+  const float* V32;
+  size_t ld32;
+  double beta;           // or *beta_d
+  const double* beta_d;
+  const double* hvec;    // projections in memory (lan_mgs)
+  float* x32;            // FP32 copy lan_scale writes, may be null
+  double* part;
+  double* gt;
+  double* gt2;
+  double* out;
+  int k, np;             // np: partials of ||vnew||^2, set by lan_gram_schmidt
+};
+struct LanCols {
+  LanCol c[kLanCols];
+};
+// whether lan_gram_schmidt takes this many rows (at most 16 chunks: larger
+// bases are bandwidth-bound and run gemv_t / gemv_n_sub_nrm, whose partials go
+// to part + 2 * kRedBlocks)
+bool lan_small(size_t n);
+size_t lan_part_elems(size_t n);
+// vnew -= beta zold; out[0] = alpha = vnew.v; vnew -= alpha v
+hipError_t lan_recurrence(size_t n, const LanCols& cols, int ncol, hipStream_t st);
+// vnew -= V V^T vnew against the FP64 bases or (f32) their FP32 copies
+hipError_t lan_gram_schmidt(size_t n, LanCols& cols, int ncol, bool f32, hipStream_t st);
+// out[1] = ||vnew||^2 before the Gram-Schmidt pass, out[2] after it; second:
+// out[3] after another one
+hipError_t lan_sums(size_t n, const LanCols& cols, int ncol, bool second, hipStream_t st);
+// vnew *= beta (or 1 / *beta_d), and its FP32 copy
+hipError_t lan_scale(size_t n, const LanCols& cols, int ncol, hipStream_t st);
+// vnew of the one column minus its projections by a modified Gram-Schmidt sweep
+// over the k basis vectors (the last of them v), through the products
+// V^T [vnew, v] and a small triangular system; G (ld ldg) keeps the products of
+// the basis vectors, hvec takes k doubles; *b2 = ||vnew||^2, *b its root
+hipError_t lan_mgs(size_t n, LanCols& col, double* G, int ldg, double* b2, double* b,
+                   hipStream_t st);
 
 // C(n x m) = A(n x k) * B(k x m), all column-major, FP64
 hipError_t gemm_nn(size_t n, int m, int k, const double* A, size_t lda, const double* B,

@@ -201,25 +201,6 @@ __global__ __launch_bounds__(kWG) void k_axpy_dot(size_t n, double a,
   }
 }
 
-template <bool SELF>
-__global__ __launch_bounds__(kWG) void k_axpy_dev(size_t n, double sign,
-                                                  const double* __restrict__ a_d,
-                                                  const double* __restrict__ x,
-                                                  double* __restrict__ y,
-                                                  const double* __restrict__ z,
-                                                  double* __restrict__ part) {
-  __shared__ double sh[4];
-  const double a = sign * (*a_d);
-  double d = 0.0;
-  for (size_t i = (size_t)blockIdx.x * kWG + threadIdx.x; i < n; i += (size_t)gridDim.x * kWG) {
-    const double v = y[i] + a * x[i];
-    y[i] = v;
-    d += v * (SELF ? v : z[i]);
-  }
-  d = block_sum(d, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = d;
-}
-
 __global__ void k_scal(size_t n, double a, double* __restrict__ x) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
@@ -334,8 +315,7 @@ __global__ __launch_bounds__(64) void k_gemv_t_reduce(const double* __restrict__
 
 constexpr int kHTile = 2048;  // h entries staged in LDS per pass
 
-// w -= V h; part[blk] = partial ||w||^2   (SUB) or y = V h (!SUB)
-template <bool SUB>
+// w -= V h; part[blk] = partial ||w||^2
 __global__ __launch_bounds__(kWG) void k_gemv_n(size_t n, int k, const double* __restrict__ V,
                                                 size_t ld, const double* __restrict__ h,
                                                 double* __restrict__ w,
@@ -367,18 +347,12 @@ __global__ __launch_bounds__(kWG) void k_gemv_n(size_t n, int k, const double* _
   const double acc = (a0 + a1) + (a2 + a3);
   double d = 0.0;
   if (r < n) {
-    if (SUB) {
-      const double v = w[r] - acc;
-      w[r] = v;
-      d = v * v;
-    } else {
-      w[r] = acc;
-    }
+    const double v = w[r] - acc;
+    w[r] = v;
+    d = v * v;
   }
-  if (SUB) {
-    d = block_sum(d, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = d;
-  }
+  d = block_sum(d, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = d;
 }
 
 // The same two passes against an FP32 copy of the basis (V32, ld32 even,
@@ -1274,20 +1248,6 @@ hipError_t axpy_dot(size_t n, double a, const double* x, double* y, const double
   return hipGetLastError();
 }
 
-hipError_t axpy_dev_nrm(size_t n, double sign, const double* a_d, const double* x,
-                        double* y, double* part, hipStream_t st) {
-  hipLaunchKernelGGL(k_axpy_dev<true>, dim3(kRedBlocks), dim3(kWG), 0, st, n, sign, a_d, x,
-                     y, (const double*)nullptr, part);
-  return hipGetLastError();
-}
-
-hipError_t axpy_dev_dot(size_t n, double sign, const double* a_d, const double* x,
-                        double* y, const double* z, double* part, hipStream_t st) {
-  hipLaunchKernelGGL(k_axpy_dev<false>, dim3(kRedBlocks), dim3(kWG), 0, st, n, sign, a_d, x,
-                     y, z, part);
-  return hipGetLastError();
-}
-
 hipError_t scal(size_t n, double a, double* x, hipStream_t st) {
   hipLaunchKernelGGL(k_scal, dim3(grid_for(n, kWG, 4096)), dim3(kWG), 0, st, n, a, x);
   return hipGetLastError();
@@ -1348,7 +1308,7 @@ hipError_t gemv_t(size_t n, int k, const double* V, size_t ld, const double* w,
 hipError_t gemv_n_sub_nrm(size_t n, int k, const double* V, size_t ld, const double* h,
                           double* w, double* part, hipStream_t st) {
   const unsigned g = (unsigned)((n + kWG - 1) / kWG);
-  hipLaunchKernelGGL(k_gemv_n<true>, dim3(g), dim3(kWG), 0, st, n, k, V, ld, h, w, part);
+  hipLaunchKernelGGL(k_gemv_n, dim3(g), dim3(kWG), 0, st, n, k, V, ld, h, w, part);
   return hipGetLastError();
 }
 
@@ -1375,14 +1335,6 @@ hipError_t gemv_n_sub_nrm_f32(size_t n, int k, const float* V, size_t ld, const 
 hipError_t scal_f32copy(size_t n, double a, double* x, float* x32, hipStream_t st) {
   hipLaunchKernelGGL(k_scal_f32copy, dim3(grid_for(n, kWG, 4096)), dim3(kWG), 0, st, n, a, x,
                      x32);
-  return hipGetLastError();
-}
-
-hipError_t gemv_n(size_t n, int k, const double* V, size_t ld, const double* h, double* y,
-                  hipStream_t st) {
-  const unsigned g = (unsigned)((n + kWG - 1) / kWG);
-  hipLaunchKernelGGL(k_gemv_n<false>, dim3(g), dim3(kWG), 0, st, n, k, V, ld, h, y,
-                     (double*)nullptr);
   return hipGetLastError();
 }
 

@@ -23,7 +23,6 @@ namespace evsl {
 namespace {
 
 constexpr double kOrthTol = 1e-14;  // INC/internal_header.h:21
-constexpr int kNgsMax = 2;          // INC/internal_header.h:24
 const double kEpsM = EVSL_DBL_EPS_MULT * DBL_EPSILON;
 
 
@@ -171,27 +170,85 @@ int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int p
   return 0;
 }
 
-// CGS with the DGKS test, two GEMV passes at most (SRC/misc_la.c:221-261).
-// On entry *old2 = ||v||^2 (already known); returns ||v|| in *nrm.
-int cgs_dgks(int n, int k, const double* Q, double* v, double old2, double* nrm, LanWork& L) {
+namespace {
+
+// one Gram-Schmidt pass of q.vnew against the q.k columns of q.V
+int cgs_pass(int n, evsl_dev::LanCols& cols) {
   Context& c = ctx();
-  const double eta = 1.0 / std::sqrt(2.0);
-  double old_nrm = std::sqrt(old2), new_nrm = 0.0;
-  const int nb = (n + evsl_dev::kWG - 1) / evsl_dev::kWG;
-  for (int it = 0; it < kNgsMax; ++it) {
-    EVSL_HIP(evsl_dev::gemv_t(n, k, Q, n, v, L.gt_part.as<double>(), L.h.as<double>(), c.stream));
-    EVSL_HIP(evsl_dev::gemv_n_sub_nrm(n, k, Q, n, L.h.as<double>(), v, red_part(), c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(red_part(), nb, red_scalar(2), c.stream));
-    double s2;
-    if (int e = read_scalars(red_scalar(2), 1, &s2)) return e;
-    new_nrm = std::sqrt(s2);
-    c.astats.n_reorth_pass++;
-    c.astats.reorth_bytes += 16.0 * n * k + 24.0 * n;
-    if (new_nrm > eta * old_nrm) break;
-    old_nrm = new_nrm;
+  evsl_dev::LanCol& q = cols.c[0];
+  c.astats.n_reorth_pass++;
+  c.astats.reorth_bytes += 16.0 * n * q.k + 24.0 * n;
+  if (evsl_dev::lan_small(n)) {
+    EVSL_HIP(evsl_dev::lan_gram_schmidt(n, cols, 1, false, c.stream));
+    return 0;
   }
-  *nrm = new_nrm;
+  double* h = const_cast<double*>(q.hvec);
+  EVSL_HIP(evsl_dev::gemv_t(n, q.k, q.V, n, q.vnew, q.gt, h, c.stream));
+  EVSL_HIP(evsl_dev::gemv_n_sub_nrm(n, q.k, q.V, n, h, q.vnew,
+                                    q.part + 2 * evsl_dev::kRedBlocks, c.stream));
+  q.np = (n + evsl_dev::kWG - 1) / evsl_dev::kWG;
   return 0;
+}
+
+evsl_dev::LanCols lan_col(int k, const double* V, double* vnew, LanWork& L) {
+  evsl_dev::LanCols cols{};
+  evsl_dev::LanCol& q = cols.c[0];
+  q.V = V;
+  q.k = k;
+  q.vnew = vnew;
+  q.hvec = L.h.as<double>();
+  q.part = red_part();
+  q.gt = L.gt_part.as<double>();
+  q.out = red_scalar(0);
+  return cols;
+}
+
+const double kDgksEta = 1.0 / std::sqrt(2.0);
+
+// the second pass of the DGKS test where the first one, from norm old to *nrm,
+// asks for it
+int cgs_second(int n, evsl_dev::LanCols& cols, double old, double* nrm) {
+  if (*nrm > kDgksEta * old) return 0;
+  if (int e = cgs_pass(n, cols)) return e;
+  EVSL_HIP(evsl_dev::lan_sums(n, cols, 1, true, ctx().stream));
+  double s2;
+  if (int e = read_scalars(red_scalar(3), 1, &s2)) return e;
+  *nrm = std::sqrt(s2);
+  return 0;
+}
+
+// vnew -= beta zold, alpha = vnew.v, vnew -= alpha v, then the first
+// Gram-Schmidt pass against the k columns of V (SRC/misc_la.c:221-261): *alpha
+// and the norms before and after the pass come back in one read
+int lan_step(int n, int k, const double* V, double beta, const double* zold, const double* v,
+             double* vnew, LanWork& L, double* alpha, double* old, double* nrm) {
+  evsl_dev::LanCols cols = lan_col(k, V, vnew, L);
+  cols.c[0].zold = zold;
+  cols.c[0].v = v;
+  cols.c[0].beta = beta;
+  EVSL_HIP(evsl_dev::lan_recurrence(n, cols, 1, ctx().stream));
+  if (int e = cgs_pass(n, cols)) return e;
+  EVSL_HIP(evsl_dev::lan_sums(n, cols, 1, false, ctx().stream));
+  double sc[3];
+  if (int e = read_scalars(red_scalar(0), 3, sc)) return e;
+  *alpha = sc[0];
+  *old = std::sqrt(sc[1]);
+  *nrm = std::sqrt(sc[2]);
+  return 0;
+}
+
+}  // namespace
+
+// CGS with the DGKS test, two GEMV passes at most (SRC/misc_la.c:221-261).
+// On entry old2 = ||v||^2 (already known); returns ||v|| in *nrm.
+int cgs_dgks(int n, int k, const double* Q, double* v, double old2, double* nrm, LanWork& L) {
+  evsl_dev::LanCols cols = lan_col(k, Q, v, L);
+  if (int e = cgs_pass(n, cols)) return e;
+  EVSL_HIP(evsl_dev::lan_sums(n, cols, 1, true, ctx().stream));
+  double s2;
+  if (int e = read_scalars(red_scalar(3), 1, &s2)) return e;
+  *nrm = std::sqrt(s2);
+  return cgs_second(n, cols, std::sqrt(old2), nrm);
 }
 
 int nrm2_dev(int n, const double* x, double* out) {
@@ -204,6 +261,75 @@ int nrm2_dev(int n, const double* x, double* out) {
   return 0;
 }
 
+
+namespace {
+
+// Lanczos with full modified Gram-Schmidt re-orthogonalisation (LanBounds,
+// LanDos), enqueued without waiting: step j forms V(:, j+1) from V(:, 0..j) and
+// leaves alpha_j, ||w||^2 and ||w|| in device arrays.  The host looks at them
+// after the steps it asked for; a step past one where the recurrence ended has
+// computed nothing that is used.
+struct MgsChain {
+  int n = 0, msteps = 0;
+  DevBuf V, scal, G, h, gt, part;
+  double* col(int j) const { return V.as<double>() + (size_t)j * n; }
+  double* alp(int j) const { return scal.as<double>() + j; }
+  double* b2(int j) const { return scal.as<double>() + msteps + j; }
+  double* b(int j) const { return scal.as<double>() + 2 * (size_t)msteps + j; }
+  int init(int n_, int msteps_) {
+    n = n_;
+    msteps = msteps_;
+    const size_t nch = evsl_dev::gemv_t_chunks(n);
+    EVSL_HIP(V.alloc((size_t)(msteps + 1) * n * sizeof(double)));
+    EVSL_HIP(scal.alloc((size_t)3 * msteps * sizeof(double)));
+    EVSL_HIP(G.alloc((size_t)msteps * msteps * sizeof(double)));
+    EVSL_HIP(h.alloc((size_t)msteps * sizeof(double)));
+    EVSL_HIP(gt.alloc(2 * nch * msteps * sizeof(double)));
+    EVSL_HIP(part.alloc(evsl_dev::lan_part_elems(n) * sizeof(double)));
+    return 0;
+  }
+  evsl_dev::LanCols cols(int j) const {
+    evsl_dev::LanCols c{};
+    evsl_dev::LanCol& q = c.c[0];
+    q.zold = j ? col(j - 1) : nullptr;
+    q.beta_d = j ? b(j - 1) : nullptr;
+    q.v = col(j);
+    q.vnew = col(j + 1);
+    q.V = V.as<double>();
+    q.hvec = h.as<double>();
+    q.part = part.as<double>();
+    q.gt = gt.as<double>();
+    q.gt2 = gt.as<double>() + (size_t)evsl_dev::gemv_t_chunks(n) * msteps;
+    q.out = alp(j);
+    q.k = j + 1;
+    return c;
+  }
+  // V(:, j+1) minus its projections by a modified Gram-Schmidt sweep, normalised
+  int sweep(int j) {
+    evsl_dev::LanCols c = cols(j);
+    EVSL_HIP(evsl_dev::lan_mgs(n, c, G.as<double>(), msteps, b2(j), b(j), ctx().stream));
+    c.c[0].beta_d = b(j);
+    EVSL_HIP(evsl_dev::lan_scale(n, c, 1, ctx().stream));
+    return 0;
+  }
+  // steps j0 .. j1 - 1
+  int run(int j0, int j1) {
+    for (int j = j0; j < j1; ++j) {
+      if (int e = apply_A(col(j), col(j + 1))) return e;
+      EVSL_HIP(evsl_dev::lan_recurrence(n, cols(j), 1, ctx().stream));
+      if (int e = sweep(j)) return e;
+    }
+    return 0;
+  }
+  // alpha, ||w||^2 and ||w|| of every step (waits)
+  int read(std::vector<double>& out) {
+    out.resize((size_t)3 * msteps);
+    EVSL_HIP(hipMemcpy(out.data(), scal.p, out.size() * sizeof(double), hipMemcpyDeviceToHost));
+    return 0;
+  }
+};
+
+}  // namespace
 
 // Ritz extraction shared by the filtered Lanczos solvers: given the
 // tridiagonal T_kdim (dT, eT) and the basis V, compute Ritz pairs of A for
@@ -349,25 +475,23 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
     double* v = V + (size_t)k * nl;
     double* vnew = v + nl;
     const double* zold = k > 0 ? v - nl : nullptr;
-    double sc[2];
+    const double beta_prev = beta;
+    double alpha, old;
     do {  // once, or again by launches where a series launch has failed
       clk.mark(0);
       if (int e = cheb_av(pol, v, vnew, L.cw, prec, true)) return e;
       clk.mark(1);
-      // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; ||vnew||^2
-      if (zold)
-        EVSL_HIP(evsl_dev::axpy_dot(n, -beta, zold, vnew, v, red_part(), c.stream));
-      else
-        EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-      EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, red_scalar(0), v, vnew, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-      if (int e = read_scalars(red_scalar(0), 2, sc)) return e;
+      // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; re-orthogonalise
+      if (int e = lan_step(n, k + 1, V, beta_prev, zold, v, vnew, L, &alpha, &old,
+                           &beta))
+        return e;
     } while (series_failed());
-    const double alpha = sc[0];
     dT[k] = alpha;
     wn += std::fabs(alpha);
-    if (int e = cgs_dgks(n, k + 1, V, vnew, sc[1], &beta, L)) return e;
+    {
+      evsl_dev::LanCols cols = lan_col(k + 1, V, vnew, L);
+      if (int e = cgs_second(n, cols, old, &beta)) return e;
+    }
     clk.mark(2);
     wn += 2.0 * beta;
     nwn += 3;
@@ -427,42 +551,23 @@ int LanBounds(int msteps, double* vin, double* lmin, double* lmax) {
   Context& c = ctx();
   if (c.op == 0) return EVSL_ERR_NOMAT;
   const int n = c.n;
-  const size_t nl = n;
   msteps = std::min(n, msteps);
-  std::vector<double> alp(msteps), bet(msteps);
-  DevBuf Vb, vtmp;
-  EVSL_HIP(Vb.alloc((msteps + 1) * nl * sizeof(double)));
-  double* V = Vb.as<double>();
+  std::vector<double> alp(msteps), bet(msteps), sc;
+  DevBuf vtmp;
+  MgsChain ch;
+  if (int e = ch.init(n, msteps)) return e;
   const double* v;
   if (int e = as_device_vector(vin, n, vtmp, &v)) return e;
   double nv;
   if (int e = nrm2_dev(n, v, &nv)) return e;
-  EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, v, V, c.stream));
+  EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, v, ch.col(0), c.stream));
+  if (int e = ch.run(0, msteps)) return e;
+  if (int e = ch.read(sc)) return e;
+  const int m0 = msteps;
   double wn = 0.0;
-  double* part = red_part();
   for (int j = 0; j < msteps; ++j) {
-    double* vj = V + j * nl;
-    double* vn = vj + nl;
-    if (int e = apply_A(vj, vn)) return e;
-    if (j)
-      EVSL_HIP(evsl_dev::axpy_dot(n, -bet[j - 1], vj - nl, vn, vj, part, c.stream));
-    else
-      EVSL_HIP(evsl_dev::dot_partial(n, vn, vj, part, c.stream));
-    EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-    // vn -= alp vj, then modified Gram-Schmidt against V(:,0..j): each step
-    // subtracts the projection computed by the previous launch
-    EVSL_HIP(evsl_dev::axpy_dev_dot(n, -1.0, red_scalar(0), vj, vn, V, part, c.stream));
-    for (int i = 0; i <= j; ++i) {
-      EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-      const double* next = (i < j) ? V + (i + 1) * nl : vn;
-      EVSL_HIP(evsl_dev::axpy_dev_dot(n, -1.0, red_scalar(1), V + i * nl, vn, next, part,
-                                      c.stream));
-    }
-    EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(2), c.stream));
-    double a_b[3];
-    if (int e = read_scalars(red_scalar(0), 3, a_b)) return e;
-    alp[j] = a_b[0];
-    bet[j] = a_b[2];
+    alp[j] = sc[j];
+    bet[j] = sc[m0 + j];
     wn += alp[j] * alp[j];
     if (bet[j] * (j + 1) < kOrthTol * wn) {
       std::fprintf(stdout, "lanbounds: lucky break, j=%d, beta=%e, break\n", j, bet[j]);
@@ -471,7 +576,6 @@ int LanBounds(int msteps, double* vin, double* lmin, double* lmax) {
     }
     wn += 2.0 * bet[j];
     bet[j] = std::sqrt(bet[j]);
-    EVSL_HIP(evsl_dev::scal(n, 1.0 / bet[j], vn, c.stream));
   }
   const double bottomBeta = bet[msteps - 1];
   std::vector<double> S((size_t)msteps * msteps), ritz(msteps);
@@ -492,7 +596,6 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
   Context& c = ctx();
   if (c.op == 0) return EVSL_ERR_NOMAT;
   const int n = c.n;
-  const size_t nl = n;
   const size_t ml0 = msteps;
   std::vector<double> y(npts, 0.0), S(ml0 * ml0), gamma2(msteps), ritz(msteps);
   std::vector<int> ind(npts);
@@ -506,40 +609,30 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
   const double sigma2 = 2 * sigma * sigma;
   const double width = sigma * std::sqrt(-2.0 * std::log(1e-08));
   linspace(aa, bb, npts, xdos);
-  std::vector<double> alp(msteps), bet(msteps), hv(nl);
-  DevBuf Vb, vb;
-  EVSL_HIP(Vb.alloc((msteps + 1) * nl * sizeof(double)));
-  EVSL_HIP(vb.alloc(nl * sizeof(double)));
-  double* V = Vb.as<double>();
-  double* part = red_part();
+  std::vector<double> alp(msteps), bet(msteps), hv(n), sc;
+  DevBuf vb;
+  EVSL_HIP(vb.alloc(n * sizeof(double)));
+  MgsChain ch;
+  if (int e = ch.init(n, msteps)) return e;
+  const int m0 = msteps;
+  bool drawn = false;  // hv holds draws not used yet
   for (int m = 0; m < nvec; ++m) {
-    randn_double(n, hv.data());
-    EVSL_HIP(hipMemcpy(vb.p, hv.data(), nl * sizeof(double), hipMemcpyHostToDevice));
+    if (!drawn) randn_double(n, hv.data());
+    drawn = false;
+    EVSL_HIP(hipMemcpy(vb.p, hv.data(), n * sizeof(double), hipMemcpyHostToDevice));
     double nv;
     if (int e = nrm2_dev(n, vb.as<double>(), &nv)) return e;
-    EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, vb.as<double>(), V, c.stream));
+    EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, vb.as<double>(), ch.col(0), c.stream));
+    if (int e = ch.run(0, msteps)) return e;
+    if (m + 1 < nvec) {  // the next vector's draws while the device runs this one
+      randn_double(n, hv.data());
+      drawn = true;
+    }
+    if (int e = ch.read(sc)) return e;
     double wn = 0.0;
     for (int j = 0; j < msteps; ++j) {
-      double* vj = V + j * nl;
-      double* vn = vj + nl;
-      if (int e = apply_A(vj, vn)) return e;
-      if (j)
-        EVSL_HIP(evsl_dev::axpy_dot(n, -bet[j - 1], vj - nl, vn, vj, part, c.stream));
-      else
-        EVSL_HIP(evsl_dev::dot_partial(n, vn, vj, part, c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-      EVSL_HIP(evsl_dev::axpy_dev_dot(n, -1.0, red_scalar(0), vj, vn, V, part, c.stream));
-      for (int i = 0; i <= j; ++i) {
-        EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-        const double* next = (i < j) ? V + (i + 1) * nl : vn;
-        EVSL_HIP(evsl_dev::axpy_dev_dot(n, -1.0, red_scalar(1), V + i * nl, vn, next, part,
-                                        c.stream));
-      }
-      EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(2), c.stream));
-      double a_b[3];
-      if (int e = read_scalars(red_scalar(0), 3, a_b)) return e;
-      alp[j] = a_b[0];
-      bet[j] = a_b[2];
+      alp[j] = sc[j];
+      bet[j] = sc[m0 + j];
       wn += alp[j] * alp[j];
       if (bet[j] * (j + 1) < kOrthTol * wn) {
         std::fprintf(stdout, "lanbounds: lucky break, j=%d, beta=%e, break\n", j, bet[j]);
@@ -549,25 +642,24 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
       if (bet[j] > tolBdwn) {
         wn += 2.0 * bet[j];
         bet[j] = std::sqrt(bet[j]);
-        EVSL_HIP(evsl_dev::scal(n, 1.0 / bet[j], vn, c.stream));
       } else {
         // the reference draws the replacement into v, which is then unused
         // (SRC/landos.c:130-144); the stream of rand() calls is kept the same
-        randn_double(n, hv.data());
-        EVSL_HIP(evsl_dev::dot_partial(n, vn, V, part, c.stream));
-        for (int i = 0; i <= j; ++i) {
-          EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-          const double* next = (i < j) ? V + (i + 1) * nl : vn;
-          EVSL_HIP(evsl_dev::axpy_dev_dot(n, -1.0, red_scalar(1), V + i * nl, vn, next, part,
-                                          c.stream));
-        }
-        EVSL_HIP(evsl_dev::sum_scalar(part, evsl_dev::kRedBlocks, red_scalar(2), c.stream));
-        double b2;
-        if (int e = read_scalars(red_scalar(2), 1, &b2)) return e;
-        wn += 2.0 * b2;
-        const double bj = std::sqrt(b2);
-        EVSL_HIP(evsl_dev::scal(n, 1.0 / bj, vn, c.stream));
+        // (draws made ahead for the next vector are the ones it would take)
+        if (!drawn) randn_double(n, hv.data());
+        drawn = false;
+        // another sweep of V(:, j+1), which stands normalised: its norm is
+        // taken back into the squared norm of what it was
+        if (int e = ch.sweep(j)) return e;
+        const double was = bet[j];
+        double again;
+        if (int e = read_scalars(ch.b2(j), 1, &again)) return e;
+        wn += 2.0 * was * again;
         bet[j] = 0;
+        const double zero = 0.0;
+        EVSL_HIP(hipMemcpy(ch.b(j), &zero, sizeof(double), hipMemcpyHostToDevice));
+        if (int e = ch.run(j + 1, msteps)) return e;
+        if (int e = ch.read(sc)) return e;
       }
     }
     if (tridiag_eig_host(msteps, alp.data(), bet.data(), ritz.data(), S.data()))
@@ -765,20 +857,15 @@ int ChebLanTr(int lanm, int nev, double* intv, int maxit, double tol, double* vi
       clk.mark(1);
       ++it;
       if (int e = deflate(vnew)) return e;
-      // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; ||vnew||^2
-      if (zold)
-        EVSL_HIP(evsl_dev::axpy_dot(n, -beta, zold, vnew, v, red_part(), c.stream));
-      else
-        EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-      EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, red_scalar(0), v, vnew, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-      double sc[2];
-      if (int e = read_scalars(red_scalar(0), 2, sc)) return e;
-      const double alpha = sc[0];
+      // vnew -= beta*zold; alpha = v.vnew; vnew -= alpha*v; re-orthogonalise
+      double alpha, old;
+      if (int e = lan_step(n, k, V, beta, zold, v, vnew, L, &alpha, &old, &beta)) return e;
       T[(k - 1) * L1 + (k - 1)] = alpha;
       wn += std::fabs(alpha);
-      if (int e = cgs_dgks(n, k, V, vnew, sc[1], &beta, L)) return e;
+      {
+        evsl_dev::LanCols cols = lan_col(k, V, vnew, L);
+        if (int e = cgs_second(n, cols, old, &beta)) return e;
+      }
       clk.mark(2);
       wn += 2.0 * beta;
       nwn += 3;
@@ -1050,18 +1137,14 @@ int LanTrbounds(int lanm, int maxit, double tol, double* vinit, int bndtype, dou
       double* vnew = v + nl;
       if (int e = apply_A(v, vnew)) return e;
       ++it;
-      if (zold)
-        EVSL_HIP(evsl_dev::axpy_dot(n, -beta, zold, vnew, v, red_part(), c.stream));
-      else
-        EVSL_HIP(evsl_dev::dot_partial(n, vnew, v, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(0), c.stream));
-      EVSL_HIP(evsl_dev::axpy_dev_nrm(n, -1.0, red_scalar(0), v, vnew, red_part(), c.stream));
-      EVSL_HIP(evsl_dev::sum_scalar(red_part(), evsl_dev::kRedBlocks, red_scalar(1), c.stream));
-      double sc[2];
-      if (int e = read_scalars(red_scalar(0), 2, sc)) return e;
-      T[(k - 1) * L1 + (k - 1)] = sc[0];
-      wn += std::fabs(sc[0]);
-      if (int e = cgs_dgks(n, k, V, vnew, sc[1], &beta, L)) return e;
+      double alpha, old;
+      if (int e = lan_step(n, k, V, beta, zold, v, vnew, L, &alpha, &old, &beta)) return e;
+      T[(k - 1) * L1 + (k - 1)] = alpha;
+      wn += std::fabs(alpha);
+      {
+        evsl_dev::LanCols cols = lan_col(k, V, vnew, L);
+        if (int e = cgs_second(n, cols, old, &beta)) return e;
+      }
       wn += 2.0 * beta;
       nwn += 3;
       zold = v;

@@ -414,9 +414,9 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
     EVSL_HIP(hipMemcpy(M.rb[w], rbp.data(), rbp.size() * sizeof(int), hipMemcpyHostToDevice));
     need = std::max(need, (size_t)(M.nblk[w] + 1) * 2 * B);  // kpm_dots in FP64
   }
-  // reduction scratch: the largest per-row-block partial buffer and one
-  // partial per 256 rows
-  *red_need = std::max(need, (size_t)n / evsl_dev::kWG + 1);
+  // reduction scratch: the largest per-row-block partial buffer and a Lanczos
+  // step's partials
+  *red_need = std::max(need, evsl_dev::lan_part_elems(n));
   return 0;
 }
 
