@@ -17,6 +17,7 @@
 //    partials; V h with h staged in LDS.  Both stream V once (HBM-bound).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dev.h"
@@ -838,18 +839,28 @@ __global__ void k_rm_cm(size_t n, int B, const double* __restrict__ src,
 }
 
 // Gram panel: part[s][j][i] = sum over rows of chunk s of A(r,i) * B(r,j)
-constexpr int kGnRows = 8192;  // rows per split
+// Rows per split: 8192, or fewer (from 256) where that leaves less than 1024
+// workgroups -- 32,640 rows of 40 columns were four workgroups of 512 row
+// steps, 1395 us; now 48 us (and 33 us
+// for the sum over the splits).
+static size_t gn_rows(size_t n, int m, int p) {
+  const size_t tiles = (size_t)((m + kTM - 1) / kTM) * ((p + kTN - 1) / kTN);
+  const size_t want = (1024 + tiles - 1) / tiles;
+  const size_t rows = ((n + want - 1) / want + 255) / 256 * 256;
+  return rows < 256 ? 256 : rows > 8192 ? 8192 : rows;
+}
 __global__ __launch_bounds__(kWG) void k_gemm_tn_partial(size_t n, int m, int p,
                                                          const double* __restrict__ A,
                                                          size_t lda,
                                                          const double* __restrict__ Bm,
                                                          size_t ldb,
-                                                         double* __restrict__ part) {
+                                                         double* __restrict__ part,
+                                                         size_t rows) {
   __shared__ double As[kTK][kTM + 1];
   __shared__ double Bs[kTK][kTN + 1];
   const int i0 = blockIdx.x * kTM, j0 = blockIdx.y * kTN;
-  const size_t rbeg = (size_t)blockIdx.z * kGnRows;
-  const size_t rend = min(n, rbeg + kGnRows);
+  const size_t rbeg = (size_t)blockIdx.z * rows;
+  const size_t rend = min(n, rbeg + rows);
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
   double c[4][4];
 #pragma unroll
@@ -1517,16 +1528,23 @@ hipError_t cm_to_rm(size_t n, int B, const double* P, size_t ld, double* X, hipS
 }
 
 size_t gemm_tn_part_elems(size_t n, int m, int p) {
-  const size_t nsplit = (n + kGnRows - 1) / kGnRows;
-  return nsplit * (size_t)m * p;
+  // over all smaller m, p: at most 1024 / tiles + 1 splits of 64 x 64 tiles where
+  // the rows per split are lowered, else one split per 8192 rows
+  const size_t mp = (size_t)m * p;
+  const size_t tiles = (size_t)((m + kTM - 1) / kTM) * ((p + kTN - 1) / kTN);
+  const size_t full = (n + 8191) / 8192 * mp;
+  const size_t fine = std::min((n + 255) / 256 * mp, (1024 + tiles) * (size_t)(kTM * kTN));
+  return std::max(full, fine);
 }
 
 hipError_t gemm_tn(size_t n, int m, int p, const double* A, size_t lda, const double* B,
                    size_t ldb, double* C, size_t ldc, double* part, hipStream_t st) {
   if (m <= 0 || p <= 0) return hipSuccess;
-  const int nsplit = (int)((n + kGnRows - 1) / kGnRows);
+  const size_t rows = gn_rows(n, m, p);
+  const int nsplit = (int)((n + rows - 1) / rows);
   dim3 grid((m + kTM - 1) / kTM, (p + kTN - 1) / kTN, nsplit);
-  hipLaunchKernelGGL(k_gemm_tn_partial, grid, dim3(kWG), 0, st, n, m, p, A, lda, B, ldb, part);
+  hipLaunchKernelGGL(k_gemm_tn_partial, grid, dim3(kWG), 0, st, n, m, p, A, lda, B, ldb, part,
+                     rows);
   const size_t cnt = (size_t)m * p;
   hipLaunchKernelGGL(k_sum_splits, dim3(grid_for(cnt, kWG, 4096)), dim3(kWG), 0, st, nsplit, cnt,
                      part, m, C, ldc);
