@@ -285,7 +285,6 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
   FilterOp sop;
   if (int e = make_filter_op(pols[0]->cc, pols[0]->dd, f32, &sop)) return e;
   if (ncols > 0 && series_fits(sop, ncols, mindeg)) {
-    const size_t vs = f32 ? 4 : 8;
     std::vector<const polparams*> key(pols, pols + ncols);
     BlockWork::CoefTab* ct = nullptr;
     // kind -2: the columns' coefficients one after the other
@@ -296,11 +295,10 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
           }
         }, &ct))
       return e;
-    EVSL_HIP(W.bufs.alloc((size_t)2 * n * vs * ncols));
     std::vector<SeriesCol> cols;
     for (int j = 0; j < ncols; ++j)
-      cols.push_back({&sop, xin[j], yout[j], ct->mus.as<double>() + ct->off[j], 1, pols[j]->deg,
-                      W.bufs.as<char>() + (size_t)2 * n * vs * j});
+      cols.push_back({&sop, xin[j], yout[j], ct->mus.as<double>() + ct->off[j], 1,
+                      pols[j]->deg});
     if (int e = series_launch(cols)) return e;
     if (deferred) return 0;
     EVSL_HIP(hipStreamSynchronize(c.stream));

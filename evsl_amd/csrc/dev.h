@@ -74,6 +74,7 @@ struct Csr {
   // whose value is dg64 / dg32.
   const void* rmask = nullptr;
   int mbytes = 0, npair = 0, nneg = 0;
+  int mrow = 0;  // most pairs in a row
   int moff[kMaskPairs] = {};
   double mval64[kMaskPairs] = {};
   float mval32[kMaskPairs] = {};
@@ -114,9 +115,11 @@ hipError_t cheb_spmm_mask_f32(const Csr& A, int B, Mode mode, const void* xk, co
                               double* part, hipStream_t st);
 // Whole Chebyshev series in one launch (series.hip), one column a job:
 // out = sum_k mu[k * mu_step] T_k(A~) in (k = 0..deg, mu[0] for k = 0), with
-// ring holding 2 n values of the launch's type.  Needs a row-mask matrix.
-constexpr int kSeriesXcds = 8, kSeriesParts = 32, kSeriesStride = 64, kSeriesMaxJobs = 16;
-constexpr int kSeriesMaxHalf = 6, kSeriesMaxRows = 4;  // instances: pairs a side, rows a lane
+// ring holding 2 n cells (series_cell) that carry no tag of tag .. tag + deg yet.
+// Needs a row-mask matrix whose rows reach each other in pairs (r has r + o's
+// column exactly if r + o has r's).
+constexpr int kSeriesXcds = 8, kSeriesParts = 64, kSeriesStride = 64, kSeriesMaxJobs = 16;
+constexpr int kSeriesMaxHalf = 6, kSeriesMaxRows = 2;  // instances: pairs a side, rows a lane
 struct SeriesJob {
   const double* in;
   double* out;
@@ -131,14 +134,16 @@ struct SeriesJob {
 struct SeriesArgs {
   SeriesJob job[kSeriesMaxJobs];
   int njobs, parts;
-  unsigned limit, id;
-  unsigned* words;   // kSeriesXcds x kSeriesStride zeros: arrivals, meetings
+  unsigned limit, id, tag;
+  unsigned* words;   // kSeriesXcds x kSeriesStride zeros: arrivals
   unsigned* status;  // host memory: [0] = id on failure, [1 + j] = id once job j runs
 };
+constexpr size_t series_cell(bool fp32) { return fp32 ? 8 : 16; }
 // rows per lane a matrix of n rows takes
 int series_rows_per_lane(int n);
-// half: the larger number of pairs on one side of the diagonal, over the jobs
-hipError_t cheb_series(bool fp32, const SeriesArgs& a, int half, int rows_per_lane,
+// half: the larger number of pairs on one side of the diagonal, row: the most
+// entries of a row off the diagonal, both over the jobs
+hipError_t cheb_series(bool fp32, const SeriesArgs& a, int half, int row, int rows_per_lane,
                        hipStream_t st);
 
 hipError_t cheb_spmm_mask_f64(const Csr& A, int B, Mode mode, const void* xk, const void* xkm1,

@@ -41,27 +41,32 @@ int grouped_filter(const std::vector<GroupedCols>& parts, GroupedWork& W) {
   Context& c = ctx();
   // ---- parts that run as series launches, every column a job ---------------
   // (a column's coefficients stay on the device while its filter comes back)
-  // A launch runs one column an XCD, so eight columns a precision; more of them
-  // would take turns and the grouped launches below cover any number.
+  // Eight columns run side by side and more take turns, 0.8 to 1.4 us a step and
+  // turn where a lane has one row and up to 2.4 where it has two; the grouped
+  // launches below cover any number of matrices and columns in about 4.4 us.  So
+  // three turns or one.
   std::vector<const GroupedCols*> rest;
   std::vector<SeriesCol> jobs[2];
-  size_t sbuf = 0, njobs[2] = {0, 0};
+  size_t sbuf = 0, njobs[2] = {0, 0}, most[2] = {~(size_t)0, ~(size_t)0};
   auto fits = [](const GroupedCols& p) {
     int mindeg = p.cols[0].pol->deg;
     for (const auto& col : p.cols) mindeg = std::min(mindeg, col.pol->deg);
     return series_fits(p.op, (int)p.cols.size(), mindeg);
   };
   for (const GroupedCols& p : parts)
-    if (fits(p)) njobs[p.op.f32] += p.cols.size();
+    if (fits(p)) {
+      njobs[p.op.f32] += p.cols.size();
+      const size_t turns = evsl_dev::series_rows_per_lane(p.op.A.n) == 1 ? 3 : 1;
+      most[p.op.f32] = std::min(most[p.op.f32], turns * evsl_dev::kSeriesXcds);
+    }
   for (const GroupedCols& p : parts) {
-    if (njobs[p.op.f32] > evsl_dev::kSeriesXcds || !fits(p)) {
+    if (njobs[p.op.f32] > most[p.op.f32] || !fits(p)) {
       rest.push_back(&p);
       continue;
     }
     for (const auto& col : p.cols) {
       if (W.series.size() == sbuf) W.series.push_back(std::make_unique<GroupedWork::Bufs>());
       GroupedWork::Bufs& bw = *W.series[sbuf++];
-      EVSL_HIP(bw.ring.alloc((size_t)2 * p.op.A.n * (p.op.f32 ? 4 : 8)));
       const std::vector<GroupedWork::PolKey> key{{col.pol, col.pol->mu, col.pol->deg}};
       if (key != bw.mus_key) {
         const size_t bytes = (size_t)(col.pol->deg + 1) * sizeof(double);
@@ -70,7 +75,7 @@ int grouped_filter(const std::vector<GroupedCols>& parts, GroupedWork& W) {
         bw.mus_key = key;
       }
       jobs[p.op.f32].push_back(
-          {&p.op, col.in, col.out, bw.mus.as<double>(), 1, col.pol->deg, bw.ring.p});
+          {&p.op, col.in, col.out, bw.mus.as<double>(), 1, col.pol->deg});
     }
   }
   for (auto& js : jobs) {

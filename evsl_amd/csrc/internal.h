@@ -82,6 +82,7 @@ struct DevMatrix {
   evsl_dev::SeriesPairs* pairs64 = nullptr;
   evsl_dev::SeriesPairs* pairs32s = nullptr;  // of the shifted FP32 copy
   int mbytes = 0, nneg = 0;
+  int mrow = 0;
   std::vector<int> mcode, moff;
   // bytes per nonzero of the column index the filter kernels read
   int idx_bytes() const { return pc ? 1 : (jd ? 2 : 4); }
@@ -117,12 +118,15 @@ int ensure_red_part(size_t need);
 // matrix lacks stored diagonal entries
 int ensure_a32_shifted(double cc, double scale, bool* ok);
 
-// Series launches (series.cpp): the meetings' device counters, the launches whose
-// outcome has not been read yet, and where they report it
+// Series launches (series.cpp): arrival counters, the rings with the tag their
+// cells carry next, the launches whose outcome has not been read yet, and where
+// they report it
 struct SeriesState {
   static constexpr int kSlots = 64;     // launches between two checks
   static constexpr int kSets = 256;     // counter sets (launches between clearings)
   DevBuf words;
+  DevBuf ring;
+  unsigned tag = 0;
   unsigned* status = nullptr;           // pinned, kSlots x (1 + kSeriesMaxJobs)
   unsigned* status_d = nullptr;
   unsigned id = 0;
@@ -236,15 +240,13 @@ bool filter_op_ready(bool f32);
 // ---- whole series in one launch (series.cpp) ---------------------------------
 // Whether ncols columns of op's matrix run as a series launch of this degree.
 bool series_fits(const FilterOp& op, int ncols, int deg);
-// One column: out = sum_k mu[k * mu_step] T_k(A~) in, mu on the device, ring of
-// 2 n values of op's vector type.
+// One column: out = sum_k mu[k * mu_step] T_k(A~) in, mu on the device.
 struct SeriesCol {
   const FilterOp* op;
   const double* in;
   double* out;
   const double* mu;
   int mu_step, deg;
-  void* ring;
 };
 // Launches the columns (every op of one precision).  Nothing waits: after the
 // next synchronisation the caller asks series_failed, and where that is true

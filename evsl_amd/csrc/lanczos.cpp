@@ -112,8 +112,7 @@ int cheb_av(const polparams* pol, const double* v, double* y, ChebWork& w, int p
     FilterOp op;
     if (int e = make_filter_op(cc, pol->dd, f32, &op)) return e;
     if (series_fits(op, 1, m)) {
-      EVSL_HIP(w.bufs.alloc((size_t)2 * n * vs));
-      if (int e = series_launch({{&op, v, y, mu_d, 1, m, w.bufs.p}})) return e;
+      if (int e = series_launch({{&op, v, y, mu_d, 1, m}})) return e;
       if (deferred) return 0;
       EVSL_HIP(hipStreamSynchronize(c.stream));
       if (!series_failed()) return 0;

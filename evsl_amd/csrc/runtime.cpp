@@ -71,6 +71,7 @@ evsl_dev::Csr DevMatrix::view() const {
     c.mbytes = mbytes;
     c.npair = (int)mcode.size();
     c.nneg = nneg;
+    c.mrow = mrow;
     c.pairs = pairs64;
     for (int p = 0; p < c.npair; ++p) {
       c.moff[p] = moff[p];
@@ -288,6 +289,20 @@ bool encode_masks(int n, const int* ia, const int* ja, const std::vector<unsigne
   return true;
 }
 
+// Whether the rows of a mask matrix reach each other in pairs: row r stores an
+// entry at r + o exactly if row r + o stores one at r.
+bool paired_rows(int n, const std::vector<int>& off, const std::vector<unsigned short>& mask) {
+  const int np = (int)off.size();
+  std::vector<unsigned short> back(np, 0);  // the pairs of the opposite offset
+  for (int p = 0; p < np; ++p)
+    for (int q = 0; q < np; ++q)
+      if (off[q] == -off[p]) back[p] |= (unsigned short)(1u << q);
+  for (int r = 0; r < n; ++r)
+    for (int p = 0; p < np; ++p)
+      if (((mask[r] >> p) & 1) && !(mask[r + off[p]] & back[p])) return false;
+  return true;
+}
+
 // the row-mask pairs with values times scale (FP32: rounded after it, as
 // shift_scale_f32 does)
 int upload_pairs(const DevMatrix& M, double scale, evsl_dev::SeriesPairs** d) {
@@ -374,6 +389,7 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
       if (encode_masks(n, ia_h, ja_h, code, off, val, M.mcode, mask)) {
         M.mbytes = M.npat <= 8 ? 1 : 2;
         M.nneg = 0;
+        for (unsigned short m : mask) M.mrow = std::max(M.mrow, __builtin_popcount(m));
         for (int c : M.mcode) {
           M.moff.push_back(off[c]);
           M.nneg += off[c] < 0;
@@ -381,7 +397,10 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
         EVSL_HIP(hipMalloc(&M.rmask, (size_t)n * M.mbytes));
         std::vector<unsigned char> m8;
         if (M.mbytes == 1) m8.assign(mask.begin(), mask.end());
-        if (int e = upload_pairs(M, 1.0, &M.pairs64)) return e;
+        // the series kernel's, which needs rows paired up
+        if (evsl_dev::series_rows_per_lane(n) <= evsl_dev::kSeriesMaxRows &&
+            paired_rows(n, M.moff, mask))
+          if (int e = upload_pairs(M, 1.0, &M.pairs64)) return e;
         EVSL_HIP(hipMemcpy(M.rmask, M.mbytes == 1 ? (const void*)m8.data() : mask.data(),
                            (size_t)n * M.mbytes, hipMemcpyHostToDevice));
       }
@@ -466,7 +485,7 @@ int ensure_a32_shifted(double cc, double scale, bool* ok) {
     EVSL_HIP(hipMemcpy(c.A.pval32s, pv.data(), pv.size() * sizeof(float), hipMemcpyHostToDevice));
     if (!c.A.dg32s) EVSL_HIP(hipMalloc((void**)&c.A.dg32s, (size_t)std::max(c.A.n, 1) * sizeof(float)));
     EVSL_HIP(evsl_dev::shift_diag_f32(c.A.n, c.A.dg64, cc, scale, c.A.dg32s, c.stream));
-    if (c.A.rmask)
+    if (c.A.pairs64)
       if (int e = upload_pairs(c.A, scale, &c.A.pairs32s)) return e;
   }
   c.A.shift_cc = cc;
@@ -607,6 +626,7 @@ int EVSLFinish(void) {
   if (c.series.status) (void)hipHostFree(c.series.status);
   c.series.status = nullptr;
   c.series.words.release();
+  c.series.ring.release();
   c.series.pending.clear();
   c.op = 0;
   c.n = 0;

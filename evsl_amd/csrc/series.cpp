@@ -1,5 +1,5 @@
 // series.cpp -- host side of the series launches (series.hip): when a filter
-// runs as one, the meeting's memory, and how a failed launch is noticed.
+// runs as one, the launches' memory, and how a failed one is noticed.
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -9,17 +9,19 @@
 
 namespace evsl {
 
-// Up to eight columns (an XCD each) of a row-mask matrix of at most 65,536 rows
-// (four a lane): there a step takes 1.7 to 3.8 us against 3.3 to 5.6 by
-// launches (series.hip), less than the launches' own 3.5 us wherever the rows
-// are few, and at least as fast at the upper end in both precisions.  Larger
-// matrices are left to the launches, which use all XCDs for one column; more
-// columns would take turns on the XCDs.  Eight degrees pay for the launch and
-// its meetings' first trip.
+// Row-mask matrices of at most 65,536 rows (two a lane) whose rows are paired.
+// Eight columns run side by side, an XCD each, and further ones take turns; by
+// launches a step takes (us; 8 / 16 / 24 / 32 columns, FP64) 3.5 / 4.1 / 4.8 /
+// 4.7 on a 100 x 97 grid, 5.2 / 5.8 / 8.1 / 8.1 on 31 x 32 x 33 and 5.6 / 7.9 /
+// 14.2 / 14.4 on 40^3, as series 0.8 / 1.6 / 2.3 / 3.1, 1.4 / 2.5 / 3.7 / 4.9 and
+// 2.3 / 4.5 / 6.7 / 9.0; FP32 likewise (40^3: 4.5 / 6.0 / 8.8 / 8.8 against 2.0 /
+// 3.9 / 5.9 / 7.8).  So any number of columns does.  Larger matrices are left to
+// the launches, which use all XCDs for one column.  Eight degrees pay for the
+// launch.
 bool series_fits(const FilterOp& op, int ncols, int deg) {
   const SeriesState& s = ctx().series;
   if (s.off || s.limit == 0 || !op.A.rmask || !op.A.pairs) return false;
-  if (deg < 8 || ncols > 8) return false;
+  if (deg < 8 || ncols > SeriesState::kSlots / 2 * evsl_dev::kSeriesMaxJobs) return false;
   if (std::max(op.A.nneg, op.A.npair - op.A.nneg) > evsl_dev::kSeriesMaxHalf) return false;
   return evsl_dev::series_rows_per_lane(op.A.n) <= evsl_dev::kSeriesMaxRows;
 }
@@ -65,7 +67,26 @@ int series_launch(const std::vector<SeriesCol>& cols) {
     a.words = s.words.as<unsigned>() + (size_t)(s.id % SeriesState::kSets) * kSetWords;
     a.id = ++s.id;
     a.status = s.status_d + s.pending.size() * (1 + evsl_dev::kSeriesMaxJobs);
-    int half = 0, rpl = 1;
+    // rings and tags: a cell's tag is one that no earlier launch has stored
+    const bool f32 = cols[j0].op->f32;
+    size_t cells = 0;
+    int deg = 0;
+    for (int j = 0; j < a.njobs; ++j) {
+      cells += (size_t)2 * cols[j0 + j].op->A.n;
+      deg = std::max(deg, cols[j0 + j].deg);
+    }
+    const size_t bytes = cells * evsl_dev::series_cell(f32);
+    const bool grow = s.ring.bytes < bytes;
+    if (grow) EVSL_HIP(s.ring.alloc(bytes));
+    if (grow || s.tag > ~0u - (unsigned)deg - 2u) {
+      EVSL_HIP(evsl_dev::fill_u32(s.ring.bytes / sizeof(unsigned), 0u, s.ring.as<unsigned>(),
+                                  c.stream));
+      s.tag = 0;
+    }
+    a.tag = s.tag + 1;
+    s.tag += (unsigned)deg + 1;
+    char* ring = s.ring.as<char>();
+    int half = 0, row = 0, rpl = 1;
     for (int j = 0; j < a.njobs; ++j) {
       const SeriesCol& col = cols[j0 + j];
       const evsl_dev::Csr& A = col.op->A;
@@ -75,7 +96,8 @@ int series_launch(const std::vector<SeriesCol>& cols) {
       q.mu = col.mu;
       q.rmask = A.rmask;
       q.dg = col.op->f32 ? (const void*)A.dg32 : (const void*)A.dg64;
-      q.ring = col.ring;
+      q.ring = ring;
+      ring += (size_t)2 * A.n * evsl_dev::series_cell(f32);
       q.pairs = A.pairs;
       q.t1 = col.op->t1;
       q.t2 = col.op->t2;
@@ -85,12 +107,13 @@ int series_launch(const std::vector<SeriesCol>& cols) {
       q.mu_step = col.mu_step;
       q.mbytes = A.mbytes;
       half = std::max(half, std::max(A.nneg, A.npair - A.nneg));
+      row = std::max(row, A.mrow);
       rpl = std::max(rpl, evsl_dev::series_rows_per_lane(A.n));
       c.astats.filter_bytes += A.n * (A.mbytes + (col.op->f32 ? 4.0 : 8.0)) * col.deg;
       c.astats.n_filter_steps += col.deg;
       c.astats.n_filter_cols += col.deg;
     }
-    EVSL_HIP(evsl_dev::cheb_series(cols[j0].op->f32, a, half, rpl, c.stream));
+    EVSL_HIP(evsl_dev::cheb_series(f32, a, half, row, rpl, c.stream));
     s.pending.push_back({a.id, a.njobs});
   }
   return 0;
