@@ -471,6 +471,9 @@ struct LanCol {
   double* gt;
   double* gt2;
   double* out;
+  double *G, *b2, *b;    // lan_mgs
+  double *xi, *wi;       // this column of an interleaved block, null: none
+  int ldi;               // the block's columns
   int k, np;             // np: partials of ||vnew||^2, set by lan_gram_schmidt
 };
 struct LanCols {
@@ -481,21 +484,24 @@ struct LanCols {
 // to part + 2 * kRedBlocks)
 bool lan_small(size_t n);
 size_t lan_part_elems(size_t n);
-// vnew -= beta zold; out[0] = alpha = vnew.v; vnew -= alpha v
+// vnew -= beta zold; out[0] = alpha = vnew.v; vnew -= alpha v; where there is an
+// interleaved block wi, vnew is taken from it
 hipError_t lan_recurrence(size_t n, const LanCols& cols, int ncol, hipStream_t st);
 // vnew -= V V^T vnew against the FP64 bases or (f32) their FP32 copies
 hipError_t lan_gram_schmidt(size_t n, LanCols& cols, int ncol, bool f32, hipStream_t st);
 // out[1] = ||vnew||^2 before the Gram-Schmidt pass, out[2] after it; second:
 // out[3] after another one
 hipError_t lan_sums(size_t n, const LanCols& cols, int ncol, bool second, hipStream_t st);
-// vnew *= beta (or 1 / *beta_d), and its FP32 copy
+// vnew *= beta (or 1 / *beta_d), and its copies in FP32 and in the block xi
 hipError_t lan_scale(size_t n, const LanCols& cols, int ncol, hipStream_t st);
-// vnew of the one column minus its projections by a modified Gram-Schmidt sweep
-// over the k basis vectors (the last of them v), through the products
+// vnew minus its projections by a modified Gram-Schmidt sweep over the k basis
+// vectors (the last of them v; the same k in every column), through the products
 // V^T [vnew, v] and a small triangular system; G (ld ldg) keeps the products of
 // the basis vectors, hvec takes k doubles; *b2 = ||vnew||^2, *b its root
-hipError_t lan_mgs(size_t n, LanCols& col, double* G, int ldg, double* b2, double* b,
-                   hipStream_t st);
+hipError_t lan_mgs(size_t n, LanCols& cols, int ncol, int ldg, hipStream_t st);
+// vnew normalised: *b2 = ||vnew||^2 from kRedBlocks partials behind P1 and P2 in
+// part, *b its root
+hipError_t lan_normalise(size_t n, LanCols& cols, int ncol, hipStream_t st);
 
 // C(n x m) = A(n x k) * B(k x m), all column-major, FP64
 hipError_t gemm_nn(size_t n, int m, int k, const double* A, size_t lda, const double* B,

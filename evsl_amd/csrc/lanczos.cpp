@@ -267,63 +267,108 @@ namespace {
 // LanDos), enqueued without waiting: step j forms V(:, j+1) from V(:, 0..j) and
 // leaves alpha_j, ||w||^2 and ||w|| in device arrays.  The host looks at them
 // after the steps it asked for; a step past one where the recurrence ended has
-// computed nothing that is used.
+// computed nothing that is used.  Up to `slots` runs from different vectors
+// advance together, a column each of the step's launches, A applied to all of
+// them as one interleaved block; the bits of a run do not depend on the others.
 struct MgsChain {
   int n = 0, msteps = 0;
-  DevBuf V, scal, G, h, gt, part;
-  double* col(int j) const { return V.as<double>() + (size_t)j * n; }
-  double* alp(int j) const { return scal.as<double>() + j; }
-  double* b2(int j) const { return scal.as<double>() + msteps + j; }
-  double* b(int j) const { return scal.as<double>() + 2 * (size_t)msteps + j; }
-  int init(int n_, int msteps_) {
+  size_t nch = 0;
+  DevBuf V, scal, G, h, gt, part, xi, wi;
+  double* col(int j, int s) const {
+    return V.as<double>() + ((size_t)s * (msteps + 1) + j) * n;
+  }
+  size_t nscal() const { return 3 * (size_t)msteps + 2; }
+  double* sc(int s) const { return scal.as<double>() + s * nscal(); }
+  double* b2(int j, int s) const { return sc(s) + msteps + j; }
+  double* b(int j, int s) const { return sc(s) + 2 * (size_t)msteps + j; }
+  size_t npart() const {
+    return std::max(evsl_dev::lan_part_elems(n), (size_t)3 * evsl_dev::kRedBlocks);
+  }
+  int init(int n_, int msteps_, int slots = 1) {
     n = n_;
     msteps = msteps_;
-    const size_t nch = evsl_dev::gemv_t_chunks(n);
-    EVSL_HIP(V.alloc((size_t)(msteps + 1) * n * sizeof(double)));
-    EVSL_HIP(scal.alloc((size_t)3 * msteps * sizeof(double)));
-    EVSL_HIP(G.alloc((size_t)msteps * msteps * sizeof(double)));
-    EVSL_HIP(h.alloc((size_t)msteps * sizeof(double)));
-    EVSL_HIP(gt.alloc(2 * nch * msteps * sizeof(double)));
-    EVSL_HIP(part.alloc(evsl_dev::lan_part_elems(n) * sizeof(double)));
-    return 0;
-  }
-  evsl_dev::LanCols cols(int j) const {
-    evsl_dev::LanCols c{};
-    evsl_dev::LanCol& q = c.c[0];
-    q.zold = j ? col(j - 1) : nullptr;
-    q.beta_d = j ? b(j - 1) : nullptr;
-    q.v = col(j);
-    q.vnew = col(j + 1);
-    q.V = V.as<double>();
-    q.hvec = h.as<double>();
-    q.part = part.as<double>();
-    q.gt = gt.as<double>();
-    q.gt2 = gt.as<double>() + (size_t)evsl_dev::gemv_t_chunks(n) * msteps;
-    q.out = alp(j);
-    q.k = j + 1;
-    return c;
-  }
-  // V(:, j+1) minus its projections by a modified Gram-Schmidt sweep, normalised
-  int sweep(int j) {
-    evsl_dev::LanCols c = cols(j);
-    EVSL_HIP(evsl_dev::lan_mgs(n, c, G.as<double>(), msteps, b2(j), b(j), ctx().stream));
-    c.c[0].beta_d = b(j);
-    EVSL_HIP(evsl_dev::lan_scale(n, c, 1, ctx().stream));
-    return 0;
-  }
-  // steps j0 .. j1 - 1
-  int run(int j0, int j1) {
-    for (int j = j0; j < j1; ++j) {
-      if (int e = apply_A(col(j), col(j + 1))) return e;
-      EVSL_HIP(evsl_dev::lan_recurrence(n, cols(j), 1, ctx().stream));
-      if (int e = sweep(j)) return e;
+    nch = evsl_dev::gemv_t_chunks(n);
+    const size_t S = slots * sizeof(double);
+    EVSL_HIP(V.alloc((size_t)(msteps + 1) * n * S));
+    EVSL_HIP(scal.alloc(nscal() * S));
+    EVSL_HIP(G.alloc((size_t)msteps * msteps * S));
+    EVSL_HIP(h.alloc((size_t)msteps * S));
+    EVSL_HIP(gt.alloc(2 * nch * msteps * S));
+    EVSL_HIP(part.alloc(npart() * S));
+    if (slots > 1) {
+      EVSL_HIP(xi.alloc((size_t)n * S));
+      EVSL_HIP(wi.alloc((size_t)n * S));
     }
     return 0;
   }
-  // alpha, ||w||^2 and ||w|| of every step (waits)
-  int read(std::vector<double>& out) {
-    out.resize((size_t)3 * msteps);
-    EVSL_HIP(hipMemcpy(out.data(), scal.p, out.size() * sizeof(double), hipMemcpyDeviceToHost));
+  // step j of the runs s0 .. s0 + cnt - 1
+  evsl_dev::LanCols cols(int j, int s0, int cnt) const {
+    evsl_dev::LanCols c{};
+    for (int i = 0; i < cnt; ++i) {
+      const int s = s0 + i;
+      evsl_dev::LanCol& q = c.c[i];
+      q.zold = j ? col(j - 1, s) : nullptr;
+      q.beta_d = j ? b(j - 1, s) : nullptr;
+      q.v = col(j, s);
+      q.vnew = col(j + 1, s);
+      q.V = col(0, s);
+      q.hvec = h.as<double>() + (size_t)s * msteps;
+      q.part = part.as<double>() + s * npart();
+      q.gt = gt.as<double>() + (size_t)2 * s * nch * msteps;
+      q.gt2 = q.gt + nch * msteps;
+      q.out = sc(s) + j;
+      q.G = G.as<double>() + (size_t)s * msteps * msteps;
+      q.b2 = b2(j, s);
+      q.b = b(j, s);
+      q.k = j + 1;
+      if (cnt > 1) {
+        q.xi = xi.as<double>() + i;
+        q.wi = wi.as<double>() + i;
+        q.ldi = cnt;
+      }
+    }
+    return c;
+  }
+  // V(:, 0), which holds a start vector, normalised
+  int start(int s0, int cnt) {
+    evsl_dev::LanCols c = cols(0, s0, cnt);
+    for (int i = 0; i < cnt; ++i) {
+      c.c[i].vnew = col(0, s0 + i);
+      c.c[i].b2 = sc(s0 + i) + 3 * (size_t)msteps;
+      c.c[i].b = c.c[i].b2 + 1;
+    }
+    EVSL_HIP(evsl_dev::lan_normalise(n, c, cnt, ctx().stream));
+    return 0;
+  }
+  // V(:, j+1) minus its projections by a modified Gram-Schmidt sweep, normalised
+  int sweep(int j, int s0 = 0, int cnt = 1) {
+    evsl_dev::LanCols c = cols(j, s0, cnt);
+    EVSL_HIP(evsl_dev::lan_mgs(n, c, cnt, msteps, ctx().stream));
+    for (int i = 0; i < cnt; ++i) c.c[i].beta_d = c.c[i].b;
+    EVSL_HIP(evsl_dev::lan_scale(n, c, cnt, ctx().stream));
+    return 0;
+  }
+  // steps j0 .. j1 - 1 (more than one run: from step 0, after start())
+  int run(int j0, int j1, int s0 = 0, int cnt = 1) {
+    Context& c = ctx();
+    for (int j = j0; j < j1; ++j) {
+      if (cnt > 1) {
+        EVSL_HIP(evsl_dev::cheb_spmm(c.A.view(), cnt, false, evsl_dev::kPlain, xi.p, nullptr, wi.p,
+                                     nullptr, nullptr, nullptr, nullptr, 1.0, 0.0, false, 0,
+                                     nullptr, c.stream));
+      } else if (int e = apply_A(col(j, s0), col(j + 1, s0))) {
+        return e;
+      }
+      EVSL_HIP(evsl_dev::lan_recurrence(n, cols(j, s0, cnt), cnt, c.stream));
+      if (int e = sweep(j, s0, cnt)) return e;
+    }
+    return 0;
+  }
+  // alpha, ||w||^2 and ||w|| of every step of run s, nscal() apart (waits)
+  int read(std::vector<double>& out, int s, int cnt = 1) {
+    out.resize(std::max(out.size(), (s + cnt) * nscal()));
+    EVSL_HIP(hipMemcpy(out.data() + s * nscal(), sc(s), cnt * nscal() * sizeof(double),
+                       hipMemcpyDeviceToHost));
     return 0;
   }
 };
@@ -559,9 +604,9 @@ int LanBounds(int msteps, double* vin, double* lmin, double* lmax) {
   if (int e = as_device_vector(vin, n, vtmp, &v)) return e;
   double nv;
   if (int e = nrm2_dev(n, v, &nv)) return e;
-  EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, v, ch.col(0), c.stream));
+  EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, v, ch.col(0, 0), c.stream));
   if (int e = ch.run(0, msteps)) return e;
-  if (int e = ch.read(sc)) return e;
+  if (int e = ch.read(sc, 0)) return e;
   const int m0 = msteps;
   double wn = 0.0;
   for (int j = 0; j < msteps; ++j) {
@@ -608,30 +653,53 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
   const double sigma2 = 2 * sigma * sigma;
   const double width = sigma * std::sqrt(-2.0 * std::log(1e-08));
   linspace(aa, bb, npts, xdos);
-  std::vector<double> alp(msteps), bet(msteps), hv(n), sc;
-  DevBuf vb;
-  EVSL_HIP(vb.alloc(n * sizeof(double)));
-  MgsChain ch;
-  if (int e = ch.init(n, msteps)) return e;
-  const int m0 = msteps;
-  bool drawn = false;  // hv holds draws not used yet
-  for (int m = 0; m < nvec; ++m) {
-    if (!drawn) randn_double(n, hv.data());
-    drawn = false;
-    EVSL_HIP(hipMemcpy(vb.p, hv.data(), n * sizeof(double), hipMemcpyHostToDevice));
-    double nv;
-    if (int e = nrm2_dev(n, vb.as<double>(), &nv)) return e;
-    EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, vb.as<double>(), ch.col(0), c.stream));
-    if (int e = ch.run(0, msteps)) return e;
-    if (m + 1 < nvec) {  // the next vector's draws while the device runs this one
-      randn_double(n, hv.data());
-      drawn = true;
+  // Runs from several vectors advance together on matrices whose step is launches
+  // rather than bandwidth, in groups of 2, 4 and then 8: the first of them soon has
+  // the device busy while the host draws the next group's vectors.
+  int slots = 1;
+  if (c.op == 1 && evsl_dev::lan_small(n))
+    while (slots < evsl_dev::kLanCols && 2 * slots <= nvec) slots *= 2;
+  std::vector<double> alp(msteps), bet(msteps), sc;
+  // vectors drawn ahead of their use, in the order of the draws
+  std::vector<std::vector<double>> drawn;
+  auto draw = [&](size_t count) {
+    while (drawn.size() < count) {
+      drawn.emplace_back(n);
+      randn_double(n, drawn.back().data());
     }
-    if (int e = ch.read(sc)) return e;
+  };
+  MgsChain ch;
+  if (int e = ch.init(n, msteps, slots)) return e;
+  const int m0 = msteps;
+  int have = 0, next = 0, group = 1;  // runs of the current group, the next one to look at
+  for (int m = 0; m < nvec; ++m) {
+    if (next == have) {
+      auto size_of = [&](int left) {
+        int g = std::min(slots, 2 * group);
+        while (g > left) g /= 2;
+        return g;
+      };
+      have = size_of(nvec - m);
+      group = have;
+      next = 0;
+      draw(have);
+      for (int s = 0; s < have; ++s)
+        EVSL_HIP(hipMemcpy(ch.col(0, s), drawn[s].data(), n * sizeof(double),
+                           hipMemcpyHostToDevice));
+      drawn.erase(drawn.begin(), drawn.begin() + have);
+      if (int e = ch.start(0, have)) return e;
+      if (int e = ch.run(0, msteps, 0, have)) return e;
+      // the next group's draws while the device runs this one
+      const int left = nvec - m - have;
+      if (left > 0) draw(size_of(left));
+      if (int e = ch.read(sc, 0, have)) return e;
+    }
+    const int s = next++;
+    const double* scs = sc.data() + s * ch.nscal();
     double wn = 0.0;
     for (int j = 0; j < msteps; ++j) {
-      alp[j] = sc[j];
-      bet[j] = sc[m0 + j];
+      alp[j] = scs[j];
+      bet[j] = scs[m0 + j];
       wn += alp[j] * alp[j];
       if (bet[j] * (j + 1) < kOrthTol * wn) {
         std::fprintf(stdout, "lanbounds: lucky break, j=%d, beta=%e, break\n", j, bet[j]);
@@ -643,22 +711,27 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
         bet[j] = std::sqrt(bet[j]);
       } else {
         // the reference draws the replacement into v, which is then unused
-        // (SRC/landos.c:130-144); the stream of rand() calls is kept the same
-        // (draws made ahead for the next vector are the ones it would take)
-        if (!drawn) randn_double(n, hv.data());
-        drawn = false;
+        // (SRC/landos.c:130-144); the stream of rand() calls is kept the same:
+        // the replacement is the next draw, whose run is left out where there
+        // is one already
+        if (next < have) {
+          ++next;
+        } else {
+          draw(1);
+          drawn.erase(drawn.begin());
+        }
         // another sweep of V(:, j+1), which stands normalised: its norm is
         // taken back into the squared norm of what it was
-        if (int e = ch.sweep(j)) return e;
+        if (int e = ch.sweep(j, s)) return e;
         const double was = bet[j];
         double again;
-        if (int e = read_scalars(ch.b2(j), 1, &again)) return e;
+        if (int e = read_scalars(ch.b2(j, s), 1, &again)) return e;
         wn += 2.0 * was * again;
         bet[j] = 0;
         const double zero = 0.0;
-        EVSL_HIP(hipMemcpy(ch.b(j), &zero, sizeof(double), hipMemcpyHostToDevice));
-        if (int e = ch.run(j + 1, msteps)) return e;
-        if (int e = ch.read(sc)) return e;
+        EVSL_HIP(hipMemcpy(ch.b(j, s), &zero, sizeof(double), hipMemcpyHostToDevice));
+        if (int e = ch.run(j + 1, msteps, s)) return e;
+        if (int e = ch.read(sc, s)) return e;
       }
     }
     if (tridiag_eig_host(msteps, alp.data(), bet.data(), ritz.data(), S.data()))

@@ -12,7 +12,10 @@
 // Gram-Schmidt pass, so the bits are the same.  Measured on 9,700 rows and 165
 // basis vectors: V^T w 17.0 -> 5.2 us (16 rows a thread went one after the
 // other; now two columns a workgroup and four rows in flight), w - V h 10.5 ->
-// 9.3 us (four threads a row, one for each of its four sums).
+// 9.3 us (four threads a row, one for each of its four sums).  The runs of an
+// LanDos call go through the step's nine launches eight at a time: 20 runs of 40
+// steps on a 20^3 grid with the bounds before them 44.0 -> 23.7 ms, the rest of
+// it the host's draws of the vectors and the bounds' steps.
 #include <hip/hip_runtime.h>
 
 #include "dev.h"
@@ -45,21 +48,22 @@ __device__ __forceinline__ double sum_all(const double* __restrict__ part, int c
   return sum256(a, sh);
 }
 
-// vnew -= beta zold; P1 = partials of vnew.v
+// vnew -= beta zold (vnew from the block wi where there is one); P1 = partials
+// of vnew.v
 __global__ __launch_bounds__(256) void k_lan_axpy(size_t n, const LanCols cols) {
   __shared__ double sh[4];
   const LanCol& q = cols.c[blockIdx.y];
   const double* __restrict__ zold = q.zold;
   const double* __restrict__ v = q.v;
   double* __restrict__ w = q.vnew;
+  const double* __restrict__ wi = q.wi;
+  const size_t ldi = q.ldi;
   const double a = zold ? -(q.beta_d ? *q.beta_d : q.beta) : 0.0;
   double d = 0.0;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    double x = w[i];
-    if (zold) {
-      x = __builtin_fma(a, zold[i], x);
-      w[i] = x;
-    }
+    double x = wi ? wi[i * ldi] : w[i];
+    if (zold) x = __builtin_fma(a, zold[i], x);
+    if (zold || wi) w[i] = x;
     d = __builtin_fma(x, v[i], d);
   }
   d = sum256(d, sh);
@@ -265,16 +269,19 @@ __global__ __launch_bounds__(256) void k_lan_sums(const LanCols cols, int rb, in
   if (threadIdx.x == 0) q.out[p3 ? slot : 1] = s;
 }
 
-// vnew *= a and its FP32 copy; a = beta, or 1 / *beta_d
+// vnew *= a and its copies in FP32 and in the block xi; a = beta, or 1 / *beta_d
 __global__ __launch_bounds__(256) void k_lan_scal(size_t n, const LanCols cols) {
   const LanCol& q = cols.c[blockIdx.y];
   const double a = q.beta_d ? 1.0 / *q.beta_d : q.beta;
   double* __restrict__ x = q.vnew;
   float* __restrict__ x32 = q.x32;
+  double* __restrict__ xi = q.xi;
+  const size_t ldi = q.ldi;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
     const double y = x[i] * a;
     x[i] = y;
     if (x32) x32[i] = (float)y;
+    if (xi) xi[i * ldi] = y;
   }
 }
 
@@ -282,11 +289,12 @@ __global__ __launch_bounds__(256) void k_lan_scal(size_t n, const LanCols cols) 
 // a_i = v_i.w and G(i, l) = v_i.v_l (l < i), the sweep's
 // h_i = v_i.(w - sum_{l < i} h_l v_l) are the solution of (I + G) h = a.  Sums
 // the partials of a (gt) and of the newest basis vector's row of G (gt2, kept
-// in G), then solves in panels of 64 rows.  One workgroup.
-__global__ __launch_bounds__(256) void k_mgs_solve(const LanCols cols, int nch, double* G, int ldg) {
+// in G), then solves in panels of 64 rows.  One workgroup a column.
+__global__ __launch_bounds__(256) void k_mgs_solve(const LanCols cols, int nch, int ldg) {
   __shared__ double s_g[64][65];
   __shared__ double s_p[64];
-  const LanCol& q = cols.c[0];
+  const LanCol& q = cols.c[blockIdx.y];
+  double* G = q.G;
   const int k = q.k, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   double* h = const_cast<double*>(q.hvec);
   for (int c = wid; c < k; c += 4) {
@@ -330,13 +338,13 @@ __global__ __launch_bounds__(256) void k_mgs_solve(const LanCols cols, int nch, 
 }
 
 // *b2 = sum of P3, *b = its root
-__global__ __launch_bounds__(256) void k_lan_norm(const LanCols cols, double* b2, double* b) {
+__global__ __launch_bounds__(256) void k_lan_norm(const LanCols cols) {
   __shared__ double sh[4];
-  const LanCol& q = cols.c[0];
+  const LanCol& q = cols.c[blockIdx.y];
   const double s = sum_all(q.part + 2 * kRedBlocks, q.np, sh);
   if (threadIdx.x == 0) {
-    *b2 = s;
-    *b = sqrt(s);
+    *q.b2 = s;
+    *q.b = sqrt(s);
   }
 }
 
@@ -388,22 +396,31 @@ hipError_t lan_scale(size_t n, const LanCols& cols, int ncol, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t lan_mgs(size_t n, LanCols& col, double* G, int ldg, double* b2, double* b,
-                   hipStream_t st) {
-  LanCol& q = col.c[0];
-  const int nch = gemv_t_chunks(n);
+hipError_t lan_mgs(size_t n, LanCols& cols, int ncol, int ldg, hipStream_t st) {
+  const int nch = gemv_t_chunks(n), k = cols.c[0].k;
   const unsigned gn = (unsigned)((n + 255) / 256);
-  q.np = (int)gn;
+  for (int j = 0; j < ncol; ++j) cols.c[j].np = (int)gn;
   if (lan_small(n))
-    hipLaunchKernelGGL((k_lan_gemv_t<2, false, true>), dim3(nch * ((q.k + 1) / 2)), dim3(256), 0, st,
-                       n, col, nch);
+    hipLaunchKernelGGL((k_lan_gemv_t<2, false, true>), dim3(nch * ((k + 1) / 2), ncol), dim3(256),
+                       0, st, n, cols, nch);
   else
-    hipLaunchKernelGGL((k_lan_gemv_t<8, false, true>), dim3(nch * ((q.k + 7) / 8)), dim3(256), 0, st,
-                       n, col, nch);
-  hipLaunchKernelGGL(k_mgs_solve, dim3(1), dim3(256), 0, st, col, nch, G, ldg);
-  hipLaunchKernelGGL((k_lan_gemv_n<false, false>), dim3(gn), dim3(1024), 0, st, n, col, nch);
-  hipLaunchKernelGGL(k_lan_norm, dim3(1), dim3(256), 0, st, col, b2, b);
+    hipLaunchKernelGGL((k_lan_gemv_t<8, false, true>), dim3(nch * ((k + 7) / 8), ncol), dim3(256),
+                       0, st, n, cols, nch);
+  hipLaunchKernelGGL(k_mgs_solve, dim3(1, ncol), dim3(256), 0, st, cols, nch, ldg);
+  hipLaunchKernelGGL((k_lan_gemv_n<false, false>), dim3(gn, ncol), dim3(1024), 0, st, n, cols, nch);
+  hipLaunchKernelGGL(k_lan_norm, dim3(1, ncol), dim3(256), 0, st, cols);
   return hipGetLastError();
+}
+
+hipError_t lan_normalise(size_t n, LanCols& cols, int ncol, hipStream_t st) {
+  for (int j = 0; j < ncol; ++j) {
+    LanCol& q = cols.c[j];
+    if (hipError_t e = dot_partial(n, q.vnew, q.vnew, q.part + 2 * kRedBlocks, st)) return e;
+    q.np = kRedBlocks;
+    q.beta_d = q.b;
+  }
+  hipLaunchKernelGGL(k_lan_norm, dim3(1, ncol), dim3(256), 0, st, cols);
+  return lan_scale(n, cols, ncol, st);
 }
 
 }  // namespace evsl_dev
