@@ -369,6 +369,21 @@ struct ChebGroupEntry {
 hipError_t cheb_group_step(bool fp32, int B, bool i16, const ChebGroupEntry* tab,
                            const int* owner, int total, int k, hipStream_t st);
 
+// The start block of a request of a grouped KPM run: n x B unit vectors of `seed`
+// from column col0 on, as rm_random, rm_col_nrm2 and rm_col_scale_rsqrt make them;
+// part holds g = kpm_start_blocks(n, B) times B doubles, nrm2 B.
+struct KpmStartEntry {
+  void* x0;
+  double* part;
+  double* nrm2;
+  unsigned long long seed;
+  int n, g;
+};
+int kpm_start_blocks(size_t n, int B);
+// x0 of nr requests of at most maxn rows (a device table)
+hipError_t kpm_group_start(bool fp32, int B, const KpmStartEntry* tab, int nr, int maxn, int kind,
+                           int col0, hipStream_t st);
+
 // The partial sums of one grouped matrix: nblk block partials (W = kpm_dots
 // per block) of each of nd degrees, summed as sum_block_partials does (G
 // first-level blocks into scratch, then one; or directly when G == 1) into

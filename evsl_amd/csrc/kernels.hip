@@ -752,28 +752,71 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
   return z ^ (z >> 31);
 }
 
+// column `col`'s value in row r: kind 0 Rademacher, 1 Gaussian (Box-Muller on two
+// 53-bit uniforms)
+__device__ __forceinline__ double rm_value(int kind, unsigned long long seed, int col, size_t r) {
+  const unsigned long long key =
+      mix64(seed + 0x9e3779b97f4a7c15ULL * (unsigned long long)(col + 1)) ^ (r * 0xd1b54a32d192ed03ULL);
+  const unsigned long long h = mix64(key);
+  if (kind == 0) return (h >> 63) ? 1.0 : -1.0;
+  const unsigned long long h2 = mix64(key ^ 0x632be59bd9b4e019ULL);
+  const double u1 = ((h >> 11) + 1) * (1.0 / 9007199254740993.0);
+  const double u2 = (h2 >> 11) * (1.0 / 9007199254740992.0);
+  return sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
+}
+
 __global__ void k_rm_random(size_t n, int B, int kind, unsigned long long seed, int col0,
                             int ncols, double* __restrict__ X) {
   const size_t tot = n * (size_t)B;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
        i += (size_t)gridDim.x * blockDim.x) {
     const int c = (int)(i % B);
-    const size_t r = i / B;
-    double v = 0.0;
-    if (c < ncols) {
-      const unsigned long long key =
-          mix64(seed + 0x9e3779b97f4a7c15ULL * (unsigned long long)(col0 + c + 1)) ^ (r * 0xd1b54a32d192ed03ULL);
-      const unsigned long long h = mix64(key);
-      if (kind == 0) {  // Rademacher
-        v = (h >> 63) ? 1.0 : -1.0;
-      } else {          // Gaussian, Box-Muller on two 53-bit uniforms
-        const unsigned long long h2 = mix64(key ^ 0x632be59bd9b4e019ULL);
-        const double u1 = ((h >> 11) + 1) * (1.0 / 9007199254740993.0);
-        const double u2 = (h2 >> 11) * (1.0 / 9007199254740992.0);
-        v = sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
-      }
-    }
-    X[i] = v;
+    X[i] = c < ncols ? rm_value(kind, seed, col0 + c, i / B) : 0.0;
+  }
+}
+
+// The start blocks of many requests (blockIdx.y): rm_random, rm_col_nrm2 and
+// rm_col_scale_rsqrt of each in three launches for all, the vectors drawn again
+// rather than kept in between.  Six launches a request for a few microseconds of
+// work, and buffers of their own for each, were half of a run over 32 requests of
+// 10^3 - 10^4 rows (12.1 ms).
+__global__ __launch_bounds__(kWG) void k_kpm_start_norm(const KpmStartEntry* __restrict__ tab,
+                                                        int B, int kind, int col0) {
+  __shared__ double s_red[kWG];
+  const KpmStartEntry& e = tab[blockIdx.y];
+  if ((int)blockIdx.x >= e.g) return;
+  const int col = threadIdx.x % B, grp = threadIdx.x / B, NG = kWG / B;
+  double a = 0.0;
+  for (size_t r = (size_t)blockIdx.x * NG + grp; r < (size_t)e.n; r += (size_t)e.g * NG) {
+    const double v = rm_value(kind, e.seed, col0 + col, r);
+    a += v * v;
+  }
+  s_red[threadIdx.x] = a;
+  __syncthreads();
+  for (int st = NG / 2; st > 0; st >>= 1) {
+    if (grp < st) s_red[threadIdx.x] += s_red[threadIdx.x + st * B];
+    __syncthreads();
+  }
+  if (grp == 0) e.part[(size_t)blockIdx.x * B + col] = s_red[col];
+}
+
+__global__ __launch_bounds__(kWG) void k_kpm_start_sum(const KpmStartEntry* __restrict__ tab,
+                                                       int B) {
+  __shared__ double s_red[kWG];
+  const KpmStartEntry& e = tab[blockIdx.y];
+  sum_partials_block(e.part, e.g, B, e.nrm2, 0, 1, s_red);
+}
+
+template <typename VT>
+__global__ __launch_bounds__(kWG) void k_kpm_start(const KpmStartEntry* __restrict__ tab, int B,
+                                                   int kind, int col0) {
+  const KpmStartEntry& e = tab[blockIdx.y];
+  VT* x0 = static_cast<VT*>(e.x0);
+  const size_t tot = (size_t)e.n * B;
+  for (size_t i = (size_t)blockIdx.x * kWG + threadIdx.x; i < tot; i += (size_t)gridDim.x * kWG) {
+    const int c = (int)(i % B);
+    const double s = e.nrm2[c];
+    x0[i] = (VT)(s > 0.0 ? rm_value(kind, e.seed, col0 + c, i / B) / sqrt(s) : 0.0);
   }
 }
 
@@ -1463,6 +1506,26 @@ hipError_t rm_random(size_t n, int B, int kind, unsigned long long seed, int col
                      double* X, hipStream_t st) {
   hipLaunchKernelGGL(k_rm_random, dim3(grid_for(n * B, kWG, 8192)), dim3(kWG), 0, st, n, B,
                      kind, seed, col0, ncols, X);
+  return hipGetLastError();
+}
+
+int kpm_start_blocks(size_t n, int B) { return (int)grid_for(n, kWG / B, 1024); }
+
+hipError_t kpm_group_start(bool fp32, int B, const KpmStartEntry* tab, int nr, int maxn, int kind,
+                           int col0, hipStream_t st) {
+  if (B < 1 || B > kWG || (kWG % B) != 0) return hipErrorInvalidValue;
+  const unsigned gn = kpm_start_blocks(maxn, B), gw = grid_for((size_t)maxn * B, 4 * kWG, 1024);
+  constexpr int kMaxY = 32768;
+  for (int r = 0; r < nr; r += kMaxY) {
+    const unsigned y = (unsigned)(nr - r < kMaxY ? nr - r : kMaxY);
+    hipLaunchKernelGGL(k_kpm_start_norm, dim3(gn, y), dim3(kWG), 0, st, tab + r, B, kind, col0);
+    hipLaunchKernelGGL(k_kpm_start_sum, dim3(1, y), dim3(kWG), 0, st, tab + r, B);
+    if (fp32)
+      hipLaunchKernelGGL(k_kpm_start<float>, dim3(gw, y), dim3(kWG), 0, st, tab + r, B, kind, col0);
+    else
+      hipLaunchKernelGGL(k_kpm_start<double>, dim3(gw, y), dim3(kWG), 0, st, tab + r, B, kind,
+                         col0);
+  }
   return hipGetLastError();
 }
 

@@ -27,56 +27,66 @@
 namespace evsl {
 namespace {
 
+// Places in one allocation, 256 bytes apart: a call's buffers are many and small,
+// and an allocation and a free of its own for each cost more than the kernels.
+struct Places {
+  size_t end = 0;
+  size_t take(size_t bytes) {
+    const size_t at = end;
+    end += (bytes + 255) / 256 * 256;
+    return at;
+  }
+};
+
 // one distinct matrix of the batch, resident for the call
 struct BatchMatrix {
   const csrMat* host = nullptr;
   int n = 0, nnz = 0;
   bool full_diag = false;
   bool regular = false;
-  DevBuf ia, ja, a64;
-  std::map<int, DevBuf> table;  // row-block table by lanes per row
-  std::map<int, int> nblk;
+  size_t ia_at = 0, ja_at = 0, a64_at = 0;
+  const int *ia = nullptr, *ja = nullptr;
+  const double* a64 = nullptr;
+  std::map<int, std::vector<int>> table;  // row-block table by lanes per row
   evsl_dev::Csr view() const {
     evsl_dev::Csr v;
     v.n = n;
     v.nnz = nnz;
-    v.ia = ia.as<int>();
-    v.ja = ja.as<int>();
-    v.a64 = a64.as<double>();
+    v.ia = ia;
+    v.ja = ja;
+    v.a64 = a64;
     return v;
   }
-  int ensure_table(int lanes) {
-    if (table.count(lanes)) return 0;
-    std::vector<int> rb = make_row_blocks(host->ia, n, evsl_dev::rows_cap_for(lanes));
-    std::vector<int> rbp(2 * rb.size());
-    for (size_t i = 0; i < rb.size(); ++i) {
-      rbp[2 * i] = rb[i];
-      rbp[2 * i + 1] = host->ia[rb[i]];
+  const std::vector<int>& row_blocks(int lanes) {
+    std::vector<int>& rbp = table[lanes];
+    if (rbp.empty()) {
+      std::vector<int> rb = make_row_blocks(host->ia, n, evsl_dev::rows_cap_for(lanes));
+      rbp.resize(2 * rb.size());
+      for (size_t i = 0; i < rb.size(); ++i) {
+        rbp[2 * i] = rb[i];
+        rbp[2 * i + 1] = host->ia[rb[i]];
+      }
     }
-    DevBuf& d = table[lanes];
-    EVSL_HIP(d.alloc(rbp.size() * sizeof(int)));
-    EVSL_HIP(hipMemcpy(d.p, rbp.data(), rbp.size() * sizeof(int), hipMemcpyHostToDevice));
-    nblk[lanes] = (int)rb.size() - 1;
-    return 0;
+    return rbp;
   }
 };
 
-// one request's device state
+// FP32 values of a matrix, shared by the requests with its centre and scale
+struct BatchValues {
+  BatchMatrix* mat = nullptr;
+  double ctr = 0, scale = 0;  // scale 0: the values as they are
+  size_t at = 0;
+};
+
+// one request
 struct BatchRequest {
   BatchMatrix* mat = nullptr;
   const double* intv = nullptr;
   unsigned long long seed = 0;
   double ctr = 0, wid = 0, t0 = 0, t = 0, cc = 0;
-  DevBuf a32;  // FP32 values (shifted and scaled when the diagonal is stored)
-  DevBuf x0, ring, part, dots, scratch;
+  int a32 = -1;  // its BatchValues
   std::vector<double> raw;
 };
-
-int upload(DevBuf& d, const void* src, size_t bytes) {
-  EVSL_HIP(d.alloc(std::max<size_t>(bytes, 8)));
-  if (bytes) EVSL_HIP(hipMemcpy(d.p, src, bytes, hipMemcpyHostToDevice));
-  return 0;
-}
 
 }  // namespace
 }  // namespace evsl
@@ -113,10 +123,12 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
   }
   const bool f32 = prec == EVSL_PREC_MIXED;
   const size_t vs = f32 ? 4 : 8;
-  // distinct matrices on the device
+  // distinct matrices, and FP32 values, on the device
   std::vector<std::unique_ptr<BatchMatrix>> mat;
   std::map<const csrMat*, BatchMatrix*> by_ptr;
+  std::vector<BatchValues> values;
   std::vector<BatchRequest> req(nreq);
+  Places mp;
   for (int r = 0; r < nreq; ++r) {
     const csrMat* A = mats[r];
     auto it = by_ptr.find(A);
@@ -125,9 +137,9 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       m->host = A;
       m->n = A->nrows;
       m->nnz = A->ia[A->nrows];
-      if (int e = upload(m->ia, A->ia, (size_t)(m->n + 1) * sizeof(int))) return e;
-      if (int e = upload(m->ja, A->ja, (size_t)m->nnz * sizeof(int))) return e;
-      if (int e = upload(m->a64, A->a, (size_t)m->nnz * sizeof(double))) return e;
+      m->ia_at = mp.take((size_t)(m->n + 1) * sizeof(int));
+      m->ja_at = mp.take((size_t)m->nnz * sizeof(int));
+      m->a64_at = mp.take((size_t)m->nnz * sizeof(double));
       bool full = true;
       for (int i = 0; i < m->n && full; ++i) {
         bool has = false;
@@ -154,28 +166,50 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
     q.cc = q.ctr;
     q.raw.assign(Mdeg + 1, 0.0);
     if (f32 && q.mat->nnz > 0) {
-      EVSL_HIP(q.a32.alloc((size_t)q.mat->nnz * sizeof(float)));
+      BatchValues v;
+      v.mat = q.mat;
       if (q.mat->full_diag) {
         // as the mixed filter: round (A - ctr I) * 2^-s, not A, to FP32
-        const double scale = std::ldexp(1.0, -(int)std::lround(std::log2(q.wid)));
-        EVSL_HIP(evsl_dev::shift_scale_f32(q.mat->view(), q.ctr, scale, q.a32.as<float>(),
-                                           c.stream));
-        q.t0 /= scale;
-        q.t /= scale;
+        v.ctr = q.ctr;
+        v.scale = std::ldexp(1.0, -(int)std::lround(std::log2(q.wid)));
+        q.t0 /= v.scale;
+        q.t /= v.scale;
         q.cc = 0.0;
-      } else {
-        EVSL_HIP(evsl_dev::f64_to_f32(q.mat->nnz, q.mat->a64.as<double>(), q.a32.as<float>(),
-                                      c.stream));
+      }
+      for (size_t i = 0; i < values.size() && q.a32 < 0; ++i)
+        if (values[i].mat == v.mat && values[i].ctr == v.ctr && values[i].scale == v.scale)
+          q.a32 = (int)i;
+      if (q.a32 < 0) {
+        v.at = mp.take((size_t)q.mat->nnz * sizeof(float));
+        q.a32 = (int)values.size();
+        values.push_back(v);
       }
     }
   }
-  int maxn = 0;
-  for (auto& m : mat) maxn = std::max(maxn, m->n);
-  DevBuf x64, nrm_part, nrm2;
-  EVSL_HIP(x64.alloc((size_t)maxn * 32 * sizeof(double)));
-  EVSL_HIP(nrm_part.alloc((size_t)1024 * 32 * sizeof(double)));
-  EVSL_HIP(nrm2.alloc(32 * sizeof(double)));
-  DevBuf d_tab, d_owner, d_sums, d_owner1, d_first1, d_owner2;
+  DevBuf md;
+  EVSL_HIP(md.alloc(mp.end));
+  for (auto& m : mat) {
+    char* base = md.as<char>();
+    m->ia = reinterpret_cast<const int*>(base + m->ia_at);
+    m->ja = reinterpret_cast<const int*>(base + m->ja_at);
+    m->a64 = reinterpret_cast<const double*>(base + m->a64_at);
+    EVSL_HIP(hipMemcpy(base + m->ia_at, m->host->ia, (size_t)(m->n + 1) * sizeof(int),
+                       hipMemcpyHostToDevice));
+    if (m->nnz == 0) continue;
+    EVSL_HIP(hipMemcpy(base + m->ja_at, m->host->ja, (size_t)m->nnz * sizeof(int),
+                       hipMemcpyHostToDevice));
+    EVSL_HIP(hipMemcpy(base + m->a64_at, m->host->a, (size_t)m->nnz * sizeof(double),
+                       hipMemcpyHostToDevice));
+  }
+  for (auto& v : values) {
+    float* a32 = reinterpret_cast<float*>(md.as<char>() + v.at);
+    if (v.scale != 0.0)
+      EVSL_HIP(evsl_dev::shift_scale_f32(v.mat->view(), v.ctr, v.scale, a32, c.stream));
+    else
+      EVSL_HIP(evsl_dev::f64_to_f32(v.mat->nnz, v.mat->a64, a32, c.stream));
+  }
+  DevBuf work;
+  std::vector<char> up;
   std::vector<double> hdots;
   // the requests whose column blocks start at one width share their launches
   for (int width : {32, 16, 8}) {
@@ -191,96 +225,131 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
       if (V <= 0 || R <= 0) return EVSL_ERR_ARG;
       const int lanes = B / V / R;
-      std::vector<evsl_dev::KpmGroupEntry> tab(nr);
-      std::vector<evsl_dev::KpmSumEntry> sums(nr);
-      std::vector<int> owner, owner1, first1(nr), owner2;
-      int total = 0;
       // values per block partial, steps, and the degrees summed by one launch
       const int W = evsl_dev::kpm_dots(B, f32), steps = evsl_dev::kpm_steps(Mdeg, f32);
       size_t pv = 0;
+      int maxn = 0, total = 0;
+      std::vector<int> nblk(nr), G(nr), owner, owner1, first1(nr), owner2;
       for (int r = 0; r < nr; ++r) {
-        if (int e = reqs[r]->mat->ensure_table(lanes)) return e;
-        pv = std::max(pv, (size_t)reqs[r]->mat->nblk[lanes] * W);
+        BatchMatrix& m = *reqs[r]->mat;
+        nblk[r] = (int)(m.row_blocks(lanes).size() / 2) - 1;
+        G[r] = evsl_dev::sum_levels_blocks(nblk[r], W);
+        pv = std::max(pv, (size_t)nblk[r] * W);
+        maxn = std::max(maxn, m.n);
+        owner.insert(owner.end(), nblk[r], r);
+        first1[r] = (int)owner1.size();
+        owner1.insert(owner1.end(), G[r], r);
+        if (G[r] > 1) owner2.push_back(r);
       }
       const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
+      // what the host fills in comes first and goes over in one copy
+      Places p;
+      const size_t tab_at = p.take(nr * sizeof(evsl_dev::KpmGroupEntry));
+      const size_t sums_at = p.take(nr * sizeof(evsl_dev::KpmSumEntry));
+      const size_t start_at = p.take(nr * sizeof(evsl_dev::KpmStartEntry));
+      const size_t owner_at = p.take(owner.size() * sizeof(int));
+      const size_t owner1_at = p.take(owner1.size() * sizeof(int));
+      const size_t first1_at = p.take(first1.size() * sizeof(int));
+      const size_t owner2_at = p.take(owner2.size() * sizeof(int));
+      std::map<BatchMatrix*, size_t> rbp_at;
+      for (int r = 0; r < nr; ++r)
+        if (!rbp_at.count(reqs[r]->mat))
+          rbp_at[reqs[r]->mat] = p.take(reqs[r]->mat->row_blocks(lanes).size() * sizeof(int));
+      const size_t up_bytes = p.end, dots1 = (size_t)(steps + 1) * W;
+      const size_t dots_at = p.take(nr * dots1 * sizeof(double));
+      struct At {
+        size_t x0, ring, part, scratch, npart, nrm2;
+      };
+      std::vector<At> at(nr);
+      for (int r = 0; r < nr; ++r) {
+        const size_t n = reqs[r]->mat->n, nb = n * B;
+        at[r].x0 = p.take(nb * vs);
+        at[r].ring = p.take(3 * nb * vs);
+        at[r].part = p.take((size_t)nd * nblk[r] * W * sizeof(double));
+        at[r].scratch = p.take(G[r] > 1 ? (size_t)nd * G[r] * W * sizeof(double) : 0);
+        at[r].npart = p.take((size_t)evsl_dev::kpm_start_blocks(n, B) * B * sizeof(double));
+        at[r].nrm2 = p.take(B * sizeof(double));
+      }
+      EVSL_HIP(work.alloc(p.end));
+      char* d = work.as<char>();
+      up.assign(up_bytes, 0);
+      auto* tab = reinterpret_cast<evsl_dev::KpmGroupEntry*>(up.data() + tab_at);
+      auto* sums = reinterpret_cast<evsl_dev::KpmSumEntry*>(up.data() + sums_at);
+      auto* start = reinterpret_cast<evsl_dev::KpmStartEntry*>(up.data() + start_at);
       for (int r = 0; r < nr; ++r) {
         BatchRequest& q = *reqs[r];
         BatchMatrix& m = *q.mat;
-        const int nblk = m.nblk[lanes];
-        const size_t nb = (size_t)m.n * B;
-        EVSL_HIP(q.x0.alloc(nb * vs));
-        EVSL_HIP(q.ring.alloc(3 * nb * vs));
-        EVSL_HIP(q.part.alloc((size_t)nd * std::max(nblk, 1) * W * sizeof(double)));
-        EVSL_HIP(q.dots.alloc((size_t)(steps + 1) * W * sizeof(double)));
-        const int G = evsl_dev::sum_levels_blocks(nblk, W);
-        if (G > 1) EVSL_HIP(q.scratch.alloc((size_t)nd * G * W * sizeof(double)));
         // start block: the kpmdos_ex vectors of this request's seed, unit columns
-        double* xd = f32 ? x64.as<double>() : q.x0.as<double>();
-        EVSL_HIP(evsl_dev::rm_random(m.n, B, vec_kind == EVSL_VEC_RADEMACHER ? 0 : 1, q.seed, done,
-                                     B, xd, c.stream));
-        EVSL_HIP(evsl_dev::rm_col_nrm2(m.n, B, xd, nrm_part.as<double>(), nrm2.as<double>(),
-                                       c.stream));
-        EVSL_HIP(evsl_dev::rm_col_scale_rsqrt(m.n, B, xd, nrm2.as<double>(), c.stream));
-        if (f32) EVSL_HIP(evsl_dev::f64_to_f32(nb, xd, q.x0.as<float>(), c.stream));
+        evsl_dev::KpmStartEntry& b = start[r];
+        b.x0 = d + at[r].x0;
+        b.part = reinterpret_cast<double*>(d + at[r].npart);
+        b.nrm2 = reinterpret_cast<double*>(d + at[r].nrm2);
+        b.seed = q.seed;
+        b.n = m.n;
+        b.g = evsl_dev::kpm_start_blocks(m.n, B);
         evsl_dev::KpmGroupEntry& e = tab[r];
-        e.ia = m.ia.as<int>();
-        e.ja = m.ja.as<int>();
-        e.a = f32 ? (const void*)q.a32.p : (const void*)m.a64.p;
-        e.rbp = m.table[lanes].as<int>();
-        e.x0 = q.x0.p;
-        e.ring = q.ring.p;
-        e.part = q.part.as<double>();
+        e.ia = m.ia;
+        e.ja = m.ja;
+        e.a = m.a64;
+        if (f32) e.a = q.a32 < 0 ? nullptr : md.as<char>() + values[q.a32].at;
+        e.rbp = reinterpret_cast<const int*>(d + rbp_at[q.mat]);
+        e.x0 = b.x0;
+        e.ring = d + at[r].ring;
+        e.part = reinterpret_cast<double*>(d + at[r].part);
         e.t0 = q.t0;
         e.t = q.t;
         e.cc = q.cc;
         e.n = m.n;
         e.blk0 = total;
         e.k0 = 0;
-        e.part_step = nblk * W;
-        owner.insert(owner.end(), nblk, r);
-        total += nblk;
+        e.part_step = nblk[r] * W;
+        total += nblk[r];
         evsl_dev::KpmSumEntry& s = sums[r];
-        s.part = q.part.as<double>();
-        s.scratch = q.scratch.as<double>();
-        s.dots = q.dots.as<double>();
-        s.nblk = nblk;
-        s.G = G;
+        s.part = e.part;
+        s.scratch = G[r] > 1 ? reinterpret_cast<double*>(d + at[r].scratch) : nullptr;
+        s.dots = reinterpret_cast<double*>(d + dots_at) + r * dots1;
+        s.nblk = nblk[r];
+        s.G = G[r];
         s.k0 = 0;
         s.pad = 0;
-        first1[r] = (int)owner1.size();
-        owner1.insert(owner1.end(), G, r);
-        if (G > 1) owner2.push_back(r);
       }
-      if (int e = upload(d_tab, tab.data(), tab.size() * sizeof(tab[0]))) return e;
-      if (int e = upload(d_owner, owner.data(), owner.size() * sizeof(int))) return e;
-      if (int e = upload(d_sums, sums.data(), sums.size() * sizeof(sums[0]))) return e;
-      if (int e = upload(d_owner1, owner1.data(), owner1.size() * sizeof(int))) return e;
-      if (int e = upload(d_first1, first1.data(), first1.size() * sizeof(int))) return e;
-      if (int e = upload(d_owner2, owner2.data(), owner2.size() * sizeof(int))) return e;
+      auto fill = [&](size_t to, const std::vector<int>& v) {
+        if (!v.empty()) std::memcpy(up.data() + to, v.data(), v.size() * sizeof(int));
+      };
+      fill(owner_at, owner);
+      fill(owner1_at, owner1);
+      fill(first1_at, first1);
+      fill(owner2_at, owner2);
+      for (auto& t : rbp_at) fill(t.second, t.first->row_blocks(lanes));
+      EVSL_HIP(hipMemcpy(d, up.data(), up_bytes, hipMemcpyHostToDevice));
+      EVSL_HIP(evsl_dev::kpm_group_start(
+          f32, B, reinterpret_cast<const evsl_dev::KpmStartEntry*>(d + start_at), nr, maxn,
+          vec_kind == EVSL_VEC_RADEMACHER ? 0 : 1, done, c.stream));
       double step_bytes = 0.0;
       for (int r = 0; r < nr; ++r)
         step_bytes += (double)reqs[r]->mat->nnz * (vs + 4) + 4.0 * (reqs[r]->mat->n + 1) +
                       (f32 ? 4.0 : 3.0) * reqs[r]->mat->n * B * vs;
+      auto ints = [&](size_t from) { return reinterpret_cast<const int*>(d + from); };
       for (int k = 0; k < steps; ++k) {
-        EVSL_HIP(evsl_dev::kpm_group_step(f32, B, d_tab.as<evsl_dev::KpmGroupEntry>(),
-                                          d_owner.as<int>(), total, k, k % nd, c.stream));
+        EVSL_HIP(evsl_dev::kpm_group_step(
+            f32, B, reinterpret_cast<const evsl_dev::KpmGroupEntry*>(d + tab_at), ints(owner_at),
+            total, k, k % nd, c.stream));
         if ((k + 1) % nd == 0 || k + 1 == steps) {
           const int have = k % nd + 1;
-          EVSL_HIP(evsl_dev::kpm_group_sums(f32, B, d_sums.as<evsl_dev::KpmSumEntry>(),
-                                            k + 1 - have, have, d_owner1.as<int>(),
-                                            d_first1.as<int>(), (int)owner1.size(),
-                                            d_owner2.as<int>(), (int)owner2.size(), c.stream));
+          EVSL_HIP(evsl_dev::kpm_group_sums(
+              f32, B, reinterpret_cast<const evsl_dev::KpmSumEntry*>(d + sums_at), k + 1 - have,
+              have, ints(owner1_at), ints(first1_at), (int)owner1.size(), ints(owner2_at),
+              (int)owner2.size(), c.stream));
         }
         c.astats.filter_bytes += step_bytes;
       }
       c.astats.n_filter_steps += steps;
       c.astats.n_filter_cols += (size_t)steps * B * nr;
-      hdots.resize((size_t)(steps + 1) * W);
-      for (int r = 0; r < nr; ++r) {
-        EVSL_HIP(hipMemcpy(hdots.data(), reqs[r]->dots.p, hdots.size() * sizeof(double),
-                           hipMemcpyDeviceToHost));
-        kpm_add_dots(Mdeg, f32, B, hdots.data(), reqs[r]->raw.data());
-      }
+      hdots.resize(nr * dots1);
+      EVSL_HIP(hipMemcpy(hdots.data(), d + dots_at, hdots.size() * sizeof(double),
+                         hipMemcpyDeviceToHost));
+      for (int r = 0; r < nr; ++r)
+        kpm_add_dots(Mdeg, f32, B, hdots.data() + r * dots1, reqs[r]->raw.data());
       done += B;
     }
   }
