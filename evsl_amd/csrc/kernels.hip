@@ -49,10 +49,11 @@ __device__ __forceinline__ double block_sum(double v, double* sh /*>=4*/) {
 // row-block table, its vector blocks and its recurrence factors; step k
 // reads T_k and T_{k-1} from the matrix's ring and writes T_{k+1} and the
 // block's moment partials, as the one-matrix kKpm launch does.
-template <typename VT, int B, int V>
+template <typename VT, int B, int V, int R>
 __global__ __launch_bounds__(kWG) void k_kpm_group(const KpmGroupEntry* __restrict__ tab,
                                                    const int* __restrict__ owner, int total,
                                                    int k, int d) {
+  extern __shared__ int s_dyn[];  // the block's row pointers when R > 1
   const int gb = xcd_remap(blockIdx.x, total);
   const KpmGroupEntry& e = tab[owner[gb]];
   k -= e.k0;  // this matrix's own step
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(kWG) void k_kpm_group(const KpmGroupEntry* __restri
   cheb_spmm_block<VT, B, V, kKpm, true, 0, false>(
       gb - e.blk0, e.ia, e.ja, nullptr, static_cast<const VT*>(e.a),
       reinterpret_cast<const int2*>(e.rbp), xk, xkm1, xkp1, nullptr, x0, nullptr, nullptr,
-      k == 0 ? e.t0 : e.t, e.cc, 0, 0, e.part + (size_t)d * e.part_step);
+      k == 0 ? e.t0 : e.t, e.cc, 0, 0, e.part + (size_t)d * e.part_step, R > 1 ? s_dyn : nullptr);
 }
 
 // the y-flush schedule of evsl_dev::y_flush, for the grouped launch (each
@@ -1237,8 +1238,11 @@ hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int*
                           int total, int k, int d, hipStream_t st) {
   if (total <= 0 || d < 0) return hipErrorInvalidValue;
 #define EVSL_KPM_GROUP(VT_, B_)                                                           \
-  hipLaunchKernelGGL((k_kpm_group<VT_, B_, SpmmPolicy<VT_, B_, kKpm>::V>), dim3(total),   \
-                     dim3(kWG), 0, st, tab, owner, total, k, d)
+  hipLaunchKernelGGL(                                                                     \
+      (k_kpm_group<VT_, B_, SpmmPolicy<VT_, B_, kKpm>::V, SpmmPolicy<VT_, B_, kKpm>::R>), \
+      dim3(total), dim3(kWG),                                                             \
+      (SpmmPolicy<VT_, B_, kKpm>::R > 1) ? (kRowsCap + 1) * sizeof(int) : 0, st, tab, owner, \
+      total, k, d)
 #define EVSL_KPM_GROUP_B(VT_)                  \
   switch (B) {                                 \
     case 1: EVSL_KPM_GROUP(VT_, 1); break;     \

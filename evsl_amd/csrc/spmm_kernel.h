@@ -615,15 +615,21 @@ hipError_t launch_variant(const Csr& A, const void* xk, const void* xkm1, void* 
 // widths only admit V = R = 1.  Time saved by the chosen R over the best
 // R = 1 layout: FP32 ChebAv 7% at 4 columns, 9% at 8, 15% at 16, 19% at 32;
 // FP64 ChebAv 2% at 4, 7% at 8, 11% at 16 and 32; the FP32 residual step
-// 7-8% at 2, 4, 16 and 32.  The FP32 KPM and FP64 residual rows (neither is
-// on a solver's hot path) keep the layouts of an earlier V-only sweep.  The
-// FP64 KPM row was swept for its two dots a step in both kernels that share
+// 7-8% at 2, 4, 16 and 32.  The FP64 residual row (not on a solver's hot path)
+// keeps the layouts of an earlier V-only sweep.  The FP32 KPM row, which the
+// batched densities of the mixed form run, was swept over six matrices of 2^15 -
+// 2^18 rows (grids and random ones), where more rows a block share their x rows in
+// the L1, and over 32 requests of 10^3 - 10^4 rows, where the layouts differ by
+// little (us a degree of all requests, R = 1 layout -> the one taken, large /
+// small): 4 columns V2R1 46 -> V2R2 35 / 9.2 -> 9.4, 8 V2R1 60 -> V4R2 42 / 10.2
+// -> 10.5, 16 V2R1 87 -> V4R4 57 / 15.0 -> 15.5, 32 V4R1 154 -> V4R8 98 / 24.4 ->
+// 24.2.  The FP64 KPM row was swept for its two dots a step in both kernels that share
 // it (100^3, row-mask / CSR kernel, us): 2 columns V2R1 13.0 / 23.4 against
 // V1R1 16.9 / 24.3, 4 V2R1 19.2 / 33.1 against V1R2 28.0 / 33.9, 8 V2R2 32.8 /
 // 47.4 against V4R1 37.6 / 54.0.
 //                                    B =  2   4   6   8  16  32
 constexpr int kSpmmLayout[2][3][6] = {{{21, 22, 21, 22, 44, 44},    // FP32 ChebAv
-                                       {21, 21, 21, 21, 21, 41},    // FP32 KPM
+                                       {21, 22, 21, 42, 44, 48},    // FP32 KPM
                                        {12, 14, 21, 22, 44, 44}},   // FP32 residual
                                       {{21, 12, 21, 22, 24, 24},    // FP64 ChebAv
                                        {21, 21, 21, 22, 41, 41},    // FP64 KPM
