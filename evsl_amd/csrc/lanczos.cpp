@@ -14,6 +14,8 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <future>
+#include <system_error>
 #include <vector>
 
 #include "internal.h"
@@ -375,6 +377,39 @@ struct MgsChain {
 
 }  // namespace
 
+namespace {
+
+// The restricted-trace test of ChebLanNr: the eigenvalues of T_kdim, found by a
+// thread of their own while the device goes on with the next steps
+struct TraceTest {
+  int kdim = 0;  // 0: none under way
+  int due = 0;   // the step at whose end its answer is looked at
+  std::vector<double> eval, e;
+  std::future<int> info;
+  void set(int k, const std::vector<double>& dT, const std::vector<double>& eT) {
+    kdim = k;
+    eval.assign(dT.begin(), dT.begin() + k);
+    e.assign(k + 1, 0.0);
+    std::copy(eT.begin(), eT.begin() + (k - 1), e.begin());
+  }
+  int solve() { return tridiag_ql(kdim, eval.data(), e.data(), nullptr); }
+};
+
+// Steps that a test of kdim may lag.  The QL iteration takes about 0.022 kdim^2 us
+// of one core (2.4 ms at 331); a step on a matrix of at most 65,536 rows takes
+// about 80 us and 1 us for each degree of its filter.  Steps past the test that
+// ends the run are lost, so a test lags no longer than it takes, and not at all
+// where that is less than a step, on larger matrices or with a user's operator.
+// A count, not a look at the clock: the steps of a run do not depend on timing.
+int trace_test_lag(int kdim, int deg, int cycle) {
+  Context& c = ctx();
+  if (c.op != 1 || !evsl_dev::lan_small(c.n)) return 0;
+  const double steps = 0.022 * kdim * kdim / (80.0 + deg);
+  return std::min((int)steps, cycle - 1);
+}
+
+}  // namespace
+
 // Ritz extraction shared by the filtered Lanczos solvers: given the
 // tridiagonal T_kdim (dT, eT) and the basis V, compute Ritz pairs of A for
 // the eigenvalues of T at or above bar, keep those in [a, b] with residual
@@ -499,7 +534,7 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
   EVSL_HIP(L.h.alloc((size_t)(maxit + 1) * sizeof(double)));
   EVSL_HIP(L.vrand.alloc(nl * sizeof(double)));
   double* V = L.V.as<double>();
-  std::vector<double> dT(maxit), eT(maxit), EvalT(maxit);
+  std::vector<double> dT(maxit), eT(maxit);
   DevBuf vtmp;
   const double* v0;
   if (int e = as_device_vector(vinit, n, vtmp, &v0)) return e;
@@ -515,6 +550,27 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
   double wn = 0.0, beta = 0.0, tr0 = 0.0;
   int nwn = 0, kdim = 0, k;
   const int Ntest = 30, cycle = 20;
+  TraceTest test;
+  // the answer of the test under way; 1: converged (SRC/cheblanNr.c:269-309)
+  auto judge = [&](int info) -> int {
+    kdim = test.kdim;
+    test.kdim = 0;
+    if (info) return EVSL_ERR_EIG;
+    double tr1 = 0.0;
+    int nconv = 0;
+    for (double x : test.eval)
+      if (x + kEpsM >= bar) {
+        tr1 += x;
+        ++nconv;
+      }
+    if (fstats)
+      std::fprintf(fstats, "k %4d: nconv %4d  tr1 %21.15e\n", kdim - 1, nconv, tr1);
+    const bool done = std::fabs(tr1 - tr0) < 2e-12 || std::fabs(tr1) + std::fabs(tr0) < 1e-10;
+    tr0 = tr1;
+    return done ? 1 : 0;
+  };
+  auto collect = [&]() -> int { return test.kdim ? judge(test.info.get()) : 0; };
+  int done = 0;
   for (k = 0; k < maxit; ++k) {
     double* v = V + (size_t)k * nl;
     double* vnew = v + nl;
@@ -540,6 +596,7 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
     wn += 2.0 * beta;
     nwn += 3;
     if (beta * nwn < kOrthTol * wn) {  // lucky breakdown (SRC/cheblanNr.c:225-256)
+      if ((done = collect())) break;  // ends before this step: no draw
       if (fstats) std::fprintf(fstats, "it %4d: Lucky breakdown, beta = %.15e\n", k, beta);
       rand_double_device(n, L.vrand.as<double>());
       if (int e = cheb_av(pol, L.vrand.as<double>(), vnew, L.cw, prec)) return e;
@@ -555,26 +612,27 @@ int ChebLanNr(double* intv, int maxit, double tol, double* vinit, polparams* pol
     c.astats.t_filter += clk.secs(0, 1);
     c.astats.t_reorth += clk.secs(1, 2);
     c.astats.n_lanczos++;
+    if (test.kdim && k >= test.due && (done = collect())) break;
     if ((k < Ntest || (k - Ntest) % cycle != 0) && k != maxit - 1) continue;
-    // restricted-trace convergence test (SRC/cheblanNr.c:269-309)
-    kdim = k + 1;
+    // restricted-trace convergence test
+    if ((done = collect())) break;
     const double te = evsl_timer();
-    std::vector<double> e(kdim + 1, 0.0);
-    std::memcpy(EvalT.data(), dT.data(), kdim * sizeof(double));
-    std::memcpy(e.data(), eT.data(), (kdim - 1) * sizeof(double));
-    if (tridiag_ql(kdim, EvalT.data(), e.data(), nullptr)) return EVSL_ERR_EIG;
-    c.astats.t_eig += evsl_timer() - te;
-    double tr1 = 0.0;
-    int nconv = 0;
-    for (int i = 0; i < kdim; ++i)
-      if (EvalT[i] + kEpsM >= bar) {
-        tr1 += EvalT[i];
-        ++nconv;
+    test.set(k + 1, dT, eT);
+    const int lag = k == maxit - 1 ? 0 : trace_test_lag(test.kdim, pol->deg, cycle);
+    bool started = false;
+    if (lag > 0) {
+      test.due = k + lag;
+      try {
+        test.info = std::async(std::launch::async, [&test] { return test.solve(); });
+        started = true;
+      } catch (const std::system_error&) {  // no thread to be had
       }
-    if (fstats) std::fprintf(fstats, "k %4d: nconv %4d  tr1 %21.15e\n", k, nconv, tr1);
-    if (std::fabs(tr1 - tr0) < 2e-12 || std::fabs(tr1) + std::fabs(tr0) < 1e-10) break;
-    tr0 = tr1;
+    }
+    if (!started) done = judge(test.solve());
+    c.astats.t_eig += evsl_timer() - te;
+    if (done) break;
   }
+  if (done < 0) return done;
   if (k >= maxit && fstats)
     std::fprintf(fstats, "The max number of iterations [%d] has been reached. The eigenvalues "
                          "computed may not have converged\n", maxit);
