@@ -589,7 +589,7 @@ hipError_t cm_to_rm(size_t n, int B, const double* P, size_t ld, double* X, hipS
 
 // C(m x p) = A(n x m)^T * B(n x p), all column-major FP64; tall-skinny
 // (split over rows, partials summed by a second launch).  part must hold
-// gemm_tn_part_elems(n, m, p) doubles, which also do for any smaller m and p.
+// gemm_tn_part_elems(n, m, p) doubles.
 size_t gemm_tn_part_elems(size_t n, int m, int p);
 hipError_t gemm_tn(size_t n, int m, int p, const double* A, size_t lda, const double* B,
                    size_t ldb, double* C, size_t ldc, double* part, hipStream_t st);

@@ -883,28 +883,18 @@ __global__ void k_rm_cm(size_t n, int B, const double* __restrict__ src,
 }
 
 // Gram panel: part[s][j][i] = sum over rows of chunk s of A(r,i) * B(r,j)
-// Rows per split: 8192, or fewer (from 256) where that leaves less than 1024
-// workgroups -- 32,640 rows of 40 columns were four workgroups of 512 row
-// steps, 1395 us; now 48 us (and 33 us
-// for the sum over the splits).
-static size_t gn_rows(size_t n, int m, int p) {
-  const size_t tiles = (size_t)((m + kTM - 1) / kTM) * ((p + kTN - 1) / kTN);
-  const size_t want = (1024 + tiles - 1) / tiles;
-  const size_t rows = ((n + want - 1) / want + 255) / 256 * 256;
-  return rows < 256 ? 256 : rows > 8192 ? 8192 : rows;
-}
+constexpr int kGnRows = 8192;  // rows per split
 __global__ __launch_bounds__(kWG) void k_gemm_tn_partial(size_t n, int m, int p,
                                                          const double* __restrict__ A,
                                                          size_t lda,
                                                          const double* __restrict__ Bm,
                                                          size_t ldb,
-                                                         double* __restrict__ part,
-                                                         size_t rows) {
+                                                         double* __restrict__ part) {
   __shared__ double As[kTK][kTM + 1];
   __shared__ double Bs[kTK][kTN + 1];
   const int i0 = blockIdx.x * kTM, j0 = blockIdx.y * kTN;
-  const size_t rbeg = (size_t)blockIdx.z * rows;
-  const size_t rend = min(n, rbeg + rows);
+  const size_t rbeg = (size_t)blockIdx.z * kGnRows;
+  const size_t rend = min(n, rbeg + kGnRows);
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
   double c[4][4];
 #pragma unroll
@@ -947,6 +937,48 @@ __global__ __launch_bounds__(kWG) void k_gemm_tn_partial(size_t n, int m, int p,
       if (gi < m) out[(size_t)gj * m + gi] = c[i][j];
     }
   }
+}
+
+// The same panel where 64 x 64 tiles leave most of the chip idle: a wave an 8 x 8
+// tile, an output a lane, the next rows' operands on their way in registers.
+// Every output adds its rows one after the other as above, and so has the same
+// bits: the eigenvectors of the small matrices that these products make are open
+// to a sign, which their last bits would decide anew.  Bound: the chain of 8192
+// additions and the LDS reads that feed it.
+constexpr int kGsTile = 8, kGsRows = 64;
+__global__ __launch_bounds__(64) void k_gemm_tn_small(size_t n, int m, int p,
+                                                      const double* __restrict__ A, size_t lda,
+                                                      const double* __restrict__ Bm, size_t ldb,
+                                                      double* __restrict__ part) {
+  __shared__ double As[kGsTile][kGsRows + 2], Bs[kGsTile][kGsRows + 2];
+  const int i0 = blockIdx.x * kGsTile, j0 = blockIdx.y * kGsTile;
+  const size_t rbeg = (size_t)blockIdx.z * kGnRows, rend = min(n, rbeg + kGnRows);
+  const int lane = threadIdx.x, ti = lane % kGsTile, tj = lane / kGsTile;
+  double a[kGsTile], b[kGsTile];
+  auto load = [&](size_t r0) {
+    const size_t r = r0 + lane;
+#pragma unroll
+    for (int c = 0; c < kGsTile; ++c) {
+      a[c] = r < rend && i0 + c < m ? A[(size_t)(i0 + c) * lda + r] : 0.0;
+      b[c] = r < rend && j0 + c < p ? Bm[(size_t)(j0 + c) * ldb + r] : 0.0;
+    }
+  };
+  load(rbeg);
+  double s = 0.0;
+  for (size_t r0 = rbeg; r0 < rend; r0 += kGsRows) {
+#pragma unroll
+    for (int c = 0; c < kGsTile; ++c) {
+      As[c][lane] = a[c];
+      Bs[c][lane] = b[c];
+    }
+    __syncthreads();
+    load(r0 + kGsRows);  // zeros past the end
+#pragma unroll
+    for (int k = 0; k < kGsRows; ++k) s = __builtin_fma(As[ti][k], Bs[tj][k], s);
+    __syncthreads();
+  }
+  if (i0 + ti < m && j0 + tj < p)
+    part[(size_t)blockIdx.z * m * p + (size_t)(j0 + tj) * m + i0 + ti] = s;
 }
 
 __global__ void k_sum_splits(int nsplit, size_t cnt, const double* __restrict__ part,
@@ -1595,23 +1627,22 @@ hipError_t cm_to_rm(size_t n, int B, const double* P, size_t ld, double* X, hipS
 }
 
 size_t gemm_tn_part_elems(size_t n, int m, int p) {
-  // over all smaller m, p: at most 1024 / tiles + 1 splits of 64 x 64 tiles where
-  // the rows per split are lowered, else one split per 8192 rows
-  const size_t mp = (size_t)m * p;
-  const size_t tiles = (size_t)((m + kTM - 1) / kTM) * ((p + kTN - 1) / kTN);
-  const size_t full = (n + 8191) / 8192 * mp;
-  const size_t fine = std::min((n + 255) / 256 * mp, (1024 + tiles) * (size_t)(kTM * kTN));
-  return std::max(full, fine);
+  const size_t nsplit = (n + kGnRows - 1) / kGnRows;
+  return nsplit * (size_t)m * p;
 }
 
 hipError_t gemm_tn(size_t n, int m, int p, const double* A, size_t lda, const double* B,
                    size_t ldb, double* C, size_t ldc, double* part, hipStream_t st) {
   if (m <= 0 || p <= 0) return hipSuccess;
-  const size_t rows = gn_rows(n, m, p);
-  const int nsplit = (int)((n + rows - 1) / rows);
-  dim3 grid((m + kTM - 1) / kTM, (p + kTN - 1) / kTN, nsplit);
-  hipLaunchKernelGGL(k_gemm_tn_partial, grid, dim3(kWG), 0, st, n, m, p, A, lda, B, ldb, part,
-                     rows);
+  const int nsplit = (int)((n + kGnRows - 1) / kGnRows);
+  const dim3 grid((m + kTM - 1) / kTM, (p + kTN - 1) / kTN, nsplit);
+  // fewer than 256 workgroups of 64 x 64 tiles: 8 x 8 ones
+  if ((size_t)grid.x * grid.y * nsplit < 256)
+    hipLaunchKernelGGL(k_gemm_tn_small,
+                       dim3((m + kGsTile - 1) / kGsTile, (p + kGsTile - 1) / kGsTile, nsplit),
+                       dim3(64), 0, st, n, m, p, A, lda, B, ldb, part);
+  else
+    hipLaunchKernelGGL(k_gemm_tn_partial, grid, dim3(kWG), 0, st, n, m, p, A, lda, B, ldb, part);
   const size_t cnt = (size_t)m * p;
   hipLaunchKernelGGL(k_sum_splits, dim3(grid_for(cnt, kWG, 4096)), dim3(kWG), 0, st, nsplit, cnt,
                      part, m, C, ldc);

@@ -1,7 +1,6 @@
-"""GPU: the split of the Gram product U^T U over rows, at row counts and block
-sizes around its edges (256-row splits, splits between 256 and 8192 rows,
-8192-row splits), through the mixed batched solver and ChebSI, whose
-Rayleigh-Ritz steps it carries.
+"""GPU: the Gram product U^T U in small tiles, at row counts around its 64-row
+stages and 8192-row splits and at block sizes that are no multiple of a tile,
+through the mixed batched solver and ChebSI, whose Rayleigh-Ritz steps it carries.
 
 Bar: eigenpairs of the closed-form spectrum within 1e-10, residuals below tol."""
 import numpy as np
@@ -14,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("size", [(15, 17, 1), (16, 16, 1), (64, 67, 1), (200, 203, 1)])
-def test_gram_splits_in_the_solvers(ev, size):
+def test_gram_in_the_solvers(ev, size):
     nx, ny, nz = size
     A = M.perturb_diag(M.laplacian(nx, ny, nz), 1e-3, seed=2)
     n = A.n
