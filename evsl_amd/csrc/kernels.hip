@@ -674,6 +674,9 @@ __global__ __launch_bounds__(64) void k_replay_rotations(
       }
       const double2* r = &s_cs[(g / kRotChunk) & 1][gi];
       const int todo = min(c - j, kRotChunk - gi);
+      // which product of a pair is rounded is spelled out: left to the compiler it
+      // changes with the loop around it, and with it the signs of the mixed form's
+      // eigenvectors, which hang on the last bits
       // groups of kRotUnroll, whose operands are loaded together (loading a
       // group while the one before it runs was slower, 4.0 ms)
       int u = 0;
@@ -690,8 +693,8 @@ __global__ __launch_bounds__(64) void k_replay_rotations(
         load(u, zc, rc);
 #pragma unroll
         for (int q = 0; q < kRotUnroll; ++q) {
-          const double o = rc[q].y * zc[q] + rc[q].x * carry;
-          carry = rc[q].x * zc[q] - rc[q].y * carry;
+          const double o = __builtin_fma(rc[q].x, carry, rc[q].y * zc[q]);
+          carry = __builtin_fma(rc[q].x, zc[q], -(rc[q].y * carry));
           z[-(u + q) * RW] = o;
         }
         u += kRotUnroll;
@@ -700,8 +703,8 @@ __global__ __launch_bounds__(64) void k_replay_rotations(
       for (; u < todo; ++u) {
         const double zi = z[-RW];
         const double2 ru = r[u];
-        z[0] = ru.y * zi + ru.x * carry;
-        carry = ru.x * zi - ru.y * carry;
+        z[0] = __builtin_fma(ru.x, carry, ru.y * zi);
+        carry = __builtin_fma(ru.x, zi, -(ru.y * carry));
         z -= RW;
       }
       j += todo;
