@@ -608,6 +608,8 @@ int EVSLStart(void) {
   // this fails, and reports the error there)
   void* scratch = nullptr;
   if (hipError_t e = evsl_dev::noalloc_scratch(&scratch); e != hipSuccess) (void)hipGetLastError();
+  c.series.off = false;
+  c.series.launched = c.series.failures = 0;
   c.started = true;
   StatsReset();
   std::memset(&c.astats, 0, sizeof(c.astats));
@@ -797,6 +799,13 @@ int evsl_amd_set_series_polls(int polls) {
   if (polls < 0) return EVSL_ERR_ARG;
   ctx().series.limit = polls;
   ctx().series.off = false;
+  return 0;
+}
+int evsl_amd_series_counts(long long* launched, long long* failed, int* off) {
+  const SeriesState& s = ctx().series;
+  if (launched) *launched = s.launched;
+  if (failed) *failed = s.failures;
+  if (off) *off = s.off;
   return 0;
 }
 int evsl_amd_set_refine_widen(double widen) {

@@ -115,6 +115,7 @@ int series_launch(const std::vector<SeriesCol>& cols) {
     }
     EVSL_HIP(evsl_dev::cheb_series(f32, a, half, row, rpl, c.stream));
     s.pending.push_back({a.id, a.njobs});
+    ++s.launched;
   }
   return 0;
 }
@@ -124,8 +125,10 @@ bool series_failed() {
   bool bad = false;
   for (size_t i = 0; i < s.pending.size(); ++i) {
     const volatile unsigned* st = s.status + i * (1 + evsl_dev::kSeriesMaxJobs);
-    bad = bad || st[0] == s.pending[i].id;
-    for (int j = 0; j < s.pending[i].njobs; ++j) bad = bad || st[1 + j] != s.pending[i].id;
+    bool one = st[0] == s.pending[i].id;
+    for (int j = 0; j < s.pending[i].njobs; ++j) one = one || st[1 + j] != s.pending[i].id;
+    s.failures += one;
+    bad = bad || one;
   }
   s.pending.clear();
   s.off = s.off || bad;

@@ -200,11 +200,15 @@ int evsl_amd_set_grouped_filter(int on);
 
 /* Filters of small row-mask matrices (evsl_amd_spmm_row_masks) run all their
  * degrees in one launch, whose workgroups wait for each other at every degree.
- * A wait ends after `polls` looks at the others (default 200000, tens of
+ * A wait ends after `polls` looks at the others (default 200000, 60 - 100
  * milliseconds); the filter is then run again, one launch a degree, as all
- * later ones are until the next call of this function.  0 runs every filter
- * one launch a degree.  Results are the same bits either way. */
+ * later ones are until the next call of this function or EVSLStart.  0 runs
+ * every filter one launch a degree.  Results are the same bits either way. */
 int evsl_amd_set_series_polls(int polls);
+/* Since EVSLStart: such launches, and those of them whose filters were run
+ * again; *off is 1 while filters run one launch a degree because of that.
+ * Any of the pointers may be null. */
+int evsl_amd_series_counts(long long *launched, long long *failed, int *off);
 
 /* Matrix Market coordinate reader of the reference drivers
  * (TESTS/COMMON/io.c:115-217, read_coo_MM): real/integer, general/symmetric

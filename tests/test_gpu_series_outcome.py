@@ -1,0 +1,85 @@
+"""GPU: what becomes of a series launch (evsl_amd_series_counts): that the filters
+of small row-mask matrices run as one and succeed, and that a failed one is
+noticed and its filter run again.
+
+Bar: the bits of the filter run one launch a degree (0 polls)."""
+import numpy as np
+import pytest
+
+from evsl_amd import matrices as M
+from evsl_amd.evsl import PREC_FP64, PREC_MIXED
+from test_gpu_series_tags import POLLS, sym_band
+
+pytestmark = pytest.mark.gpu
+
+
+def filters(ev, A, ncols, deg=30):
+    lo, hi = M.gershgorin(A)
+    lo, hi = lo - 0.1, hi + 0.1
+    out = []
+    for i in range(ncols):
+        pol = ev.default_pol()
+        pol.deg = deg + i % 3
+        a = lo + (0.2 + 0.02 * i) * (hi - lo)
+        assert ev.find_pol(np.array([a, a + 0.1 * (hi - lo), lo, hi]), pol) == 0
+        out.append(pol)
+    return out
+
+
+def run(ev, pols, X, prec=PREC_FP64, polls=POLLS):
+    """The filtered columns, and the series launches and failures they took."""
+    ev.set_series_polls(polls)
+    n0, f0, _ = ev.series_counts()
+    err, Y = ev.cheb_av_cols(pols, X, prec)
+    assert err == 0, ev.last_error()
+    n1, f1, _ = ev.series_counts()
+    return Y, n1 - n0, f1 - f0
+
+
+@pytest.fixture
+def series(ev):
+    yield ev
+    ev.set_series_polls(POLLS)
+
+
+@pytest.mark.parametrize("n", [1, 63, 2049, 16385, 65536])
+@pytest.mark.parametrize("offsets", [[1], [1, 3, 7], [1, 2, 5, 9, 40, 900]])
+def test_series_run_and_fail(series, n, offsets):
+    ev = series
+    A = sym_band(n, offsets, seed=n)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, 8)
+    X = np.random.default_rng(5).uniform(-1.0, 1.0, (n, 8))
+    for prec in (PREC_FP64, PREC_MIXED):
+        for cols in (1, 3, 8):
+            ref, launched, _ = run(ev, pols[:cols], X[:, :cols], prec, 0)
+            assert launched == 0
+            Y, launched, failed = run(ev, pols[:cols], X[:, :cols], prec)
+            assert (launched, failed) == (1, 0) and np.array_equal(Y, ref)
+            Y, launched, failed = run(ev, pols[:cols], X[:, :cols], prec, 1)
+            assert launched == 1 and np.array_equal(Y, ref)
+            if n > 2000:  # several waves: none of them sees the others at one look
+                assert failed == 1 and ev.series_counts()[2]
+    for p in pols:
+        ev.free_pol(p)
+
+
+def test_a_failure_lasts_until_the_next_start(series):
+    ev = series
+    A = sym_band(5000, [1, 70], seed=1)
+    X = np.random.default_rng(5).uniform(-1.0, 1.0, (A.n, 1))
+    pols = filters(ev, A, 1)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    assert run(ev, pols, X, polls=1)[2] == 1
+    n0 = ev.series_counts()[0]
+    err, ref = ev.cheb_av_cols(pols, X)
+    assert err == 0 and ev.series_counts()[0] == n0 and ev.series_counts()[2]
+    assert ev.finish() == 0 and ev.start() == 0, ev.last_error()
+    assert ev.series_counts() == (0, 0, False)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    ev.set_series_polls(POLLS)
+    err, Y = ev.cheb_av_cols(pols, X)
+    assert err == 0 and np.array_equal(Y, ref)
+    assert ev.series_counts() == (1, 0, False)
+    for p in pols:
+        ev.free_pol(p)
