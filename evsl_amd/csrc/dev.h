@@ -134,9 +134,10 @@ struct SeriesJob {
 struct SeriesArgs {
   SeriesJob job[kSeriesMaxJobs];
   int njobs, parts;
+  int grid;          // workgroups of the launch
   unsigned limit, id, tag;
   unsigned* words;   // kSeriesXcds x kSeriesStride zeros: arrivals
-  unsigned* status;  // host memory: [0] = id on failure, [1 + j] = id once job j runs
+  unsigned* status;  // host memory: [0] = id on failure, [1 + j] = id once all shares of job j run
 };
 constexpr size_t series_cell(bool fp32) { return fp32 ? 8 : 16; }
 // rows per lane a matrix of n rows takes

@@ -131,6 +131,7 @@ struct SeriesState {
   unsigned* status_d = nullptr;
   unsigned id = 0;
   int limit = 200000;                   // polls of one wait; 0: no series launches
+  int workgroups = evsl_dev::kSeriesXcds * evsl_dev::kSeriesParts;  // of a launch
   bool off = false;                     // a launch has failed (until set_series_polls, EVSLStart)
   long long launched = 0, failures = 0; // since EVSLStart
   struct Pending {

@@ -801,6 +801,12 @@ int evsl_amd_set_series_polls(int polls) {
   ctx().series.off = false;
   return 0;
 }
+int evsl_amd_set_series_workgroups(int workgroups) {
+  constexpr int all = evsl_dev::kSeriesXcds * evsl_dev::kSeriesParts;
+  if (workgroups < 1 || workgroups > all) return EVSL_ERR_ARG;
+  ctx().series.workgroups = workgroups;
+  return 0;
+}
 int evsl_amd_series_counts(long long* launched, long long* failed, int* off) {
   const SeriesState& s = ctx().series;
   if (launched) *launched = s.launched;

@@ -63,6 +63,7 @@ int series_launch(const std::vector<SeriesCol>& cols) {
     evsl_dev::SeriesArgs a{};
     a.njobs = (int)std::min((size_t)evsl_dev::kSeriesMaxJobs, cols.size() - j0);
     a.parts = evsl_dev::kSeriesParts;
+    a.grid = s.workgroups;
     a.limit = (unsigned)s.limit;
     a.words = s.words.as<unsigned>() + (size_t)(s.id % SeriesState::kSets) * kSetWords;
     a.id = ++s.id;

@@ -35,8 +35,11 @@
 // Waits are bounded.  A wave that does not see its cells in `limit` looks --
 // the others are not resident because other work holds their CUs -- reports
 // the launch as failed and leaves, as do the others; the host then runs the
-// series by launches.  A job whose XCD got no workgroup never reports its
-// start, which counts as failed as well.
+// series by launches.  Which XCD a workgroup comes to is the hardware's choice:
+// the one that takes an XCD's last share reports the start of its jobs, and a
+// job that is not reported counts as failed as well.  So every share of a job
+// that counts as done had a workgroup, and every wave of those has either ended
+// it or reported that it gave up.
 #include <hip/hip_runtime.h>
 
 #include "dev.h"
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(kSerWG, 4) void k_cheb_series(const SeriesArgs a) {
   if (rank >= a.parts) return;
   for (int j = (int)xcc; j < a.njobs; j += kSeriesXcds) {
     const SeriesJob& q = a.job[j];
-    if (rank == 0 && tid == 0)
+    if (rank == a.parts - 1 && tid == 0)
       __hip_atomic_store(a.status + 1 + j, a.id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const int n = q.n;
     const int chunk = ((n + a.parts - 1) / a.parts + 63) & ~63;
@@ -291,9 +294,10 @@ int series_rows_per_lane(int n) {
 hipError_t cheb_series(bool fp32, const SeriesArgs& a, int half, int row, int rows_per_lane,
                        hipStream_t st) {
   if (a.njobs < 1 || a.njobs > kSeriesMaxJobs || a.parts < 1 || a.parts > 64 ||
+      a.grid < 1 || a.grid > kSeriesXcds * kSeriesParts ||
       half < 0 || half > kSeriesMaxHalf || rows_per_lane < 1 || rows_per_lane > kSeriesMaxRows)
     return hipErrorInvalidValue;
-  const int grid = kSeriesXcds * a.parts;
+  const int grid = a.grid;
   const bool slot = half > 3 && row <= 6;
   if (slot) half = 3;
   return fp32 ? launch_series<float>(half, slot, rows_per_lane, grid, a, st)

@@ -51,7 +51,8 @@ EXPORTS = [
     "evsl_amd_server_submit_slice", "evsl_amd_server_submit_dos", "evsl_amd_server_step",
     "evsl_amd_server_status", "evsl_amd_server_slice_result", "evsl_amd_server_dos_result",
     "evsl_amd_server_stats", "evsl_amd_set_mixed_degree_range",
-    "evsl_amd_set_series_polls", "evsl_amd_series_counts", "evsl_amd_spmm_row_masks", "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
+    "evsl_amd_set_series_polls", "evsl_amd_series_counts",
+    "evsl_amd_set_series_workgroups", "evsl_amd_spmm_row_masks", "evsl_amd_spmm_layout", "evsl_amd_set_spmm_layout", "evsl_amd_set_spmm_tuning",
 ]
 
 
@@ -139,6 +140,7 @@ class EVSL:
             "evsl_amd_spmm_vec": (I, [I, I, I]),
             "evsl_amd_spmm_row_masks": (I, [I, I, I]),
             "evsl_amd_set_series_polls": (I, [I]),
+            "evsl_amd_set_series_workgroups": (I, [I]),
             "evsl_amd_series_counts": (I, [C.POINTER(C.c_longlong), C.POINTER(C.c_longlong),
                                            C.POINTER(I)]),
             "evsl_amd_spmm_layout": (I, [I, I, I, C.POINTER(I)]),
@@ -487,6 +489,10 @@ class EVSL:
     def set_series_polls(self, polls):
         """Bound of a series launch's waits; 0 filters one launch a degree."""
         return self.lib.evsl_amd_set_series_polls(polls)
+
+    def set_series_workgroups(self, workgroups):
+        """Workgroups of a series launch (512 by default)."""
+        return self.lib.evsl_amd_set_series_workgroups(workgroups)
 
     def series_counts(self):
         """(series launches, those that failed, whether they are off) since

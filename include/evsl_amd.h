@@ -205,6 +205,9 @@ int evsl_amd_set_grouped_filter(int on);
  * later ones are until the next call of this function or EVSLStart.  0 runs
  * every filter one launch a degree.  Results are the same bits either way. */
 int evsl_amd_set_series_polls(int polls);
+/* Workgroups of such a launch (1 .. 512, the default).  With fewer, shares of
+ * the rows have none, and the filter is run again as after a wait that ended. */
+int evsl_amd_set_series_workgroups(int workgroups);
 /* Since EVSLStart: such launches, and those of them whose filters were run
  * again; *off is 1 while filters run one launch a degree because of that.
  * Any of the pointers may be null. */

@@ -5,12 +5,16 @@ noticed and its filter run again.
 Bar: the bits of the filter run one launch a degree (0 polls)."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from evsl_amd import matrices as M
 from evsl_amd.evsl import PREC_FP64, PREC_MIXED
+from evsl_amd.types import HostCsr
 from test_gpu_series_tags import POLLS, sym_band
 
 pytestmark = pytest.mark.gpu
+
+ALL = 512  # workgroups of a series launch
 
 
 def filters(ev, A, ncols, deg=30):
@@ -40,6 +44,7 @@ def run(ev, pols, X, prec=PREC_FP64, polls=POLLS):
 def series(ev):
     yield ev
     ev.set_series_polls(POLLS)
+    ev.set_series_workgroups(ALL)
 
 
 @pytest.mark.parametrize("n", [1, 63, 2049, 16385, 65536])
@@ -81,5 +86,30 @@ def test_a_failure_lasts_until_the_next_start(series):
     err, Y = ev.cheb_av_cols(pols, X)
     assert err == 0 and np.array_equal(Y, ref)
     assert ev.series_counts() == (1, 0, False)
+    for p in pols:
+        ev.free_pol(p)
+
+
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("matrix", ["diagonal", "blocks", "chain"])
+def test_missing_workgroups(series, matrix, prec):
+    ev = series
+    n = 65536
+    offsets = [] if matrix == "diagonal" else [1]
+    A = sym_band(n, offsets, seed=2, keep=1.0)
+    if matrix == "blocks":  # no entry across a multiple of 1024 rows, a workgroup's share
+        S = A.to_scipy().tocoo()
+        keep = S.row // 1024 == S.col // 1024
+        S = sp.csr_matrix(sp.coo_matrix((S.data[keep], (S.row[keep], S.col[keep])), shape=(n, n)))
+        S.sort_indices()
+        A = HostCsr.from_scipy(S)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, 9)
+    X = np.random.default_rng(5).uniform(-1.0, 1.0, (n, 9))
+    ref, _, _ = run(ev, pols, X, prec, 0)
+    for groups in (1, ALL // 2, ALL - 8):
+        assert ev.set_series_workgroups(groups) == 0
+        Y, launched, failed = run(ev, pols, X, prec, 2000)
+        assert (launched, failed) == (1, 1) and np.array_equal(Y, ref), groups
     for p in pols:
         ev.free_pol(p)
