@@ -1710,6 +1710,15 @@ int evsl_amd_cheb_av_cols(int ncols, const polparams* pols, const double* X, dou
     EVSL_HIP(yt.alloc(tot * sizeof(double)));
     yd = yt.as<double>();
   }
+  // X and Y may share memory.  A block's columns are packed before any of them is
+  // written, which in place is all it takes; a series launch that fails has
+  // written some outputs before its columns are filtered again, and in a shifted
+  // range an output is a later block's input: X is copied for those.
+  if (yd < xd + tot && xd < yd + tot && (xd != yd || series_size(c.n, ncols))) {
+    EVSL_HIP(xt.alloc(tot * sizeof(double)));
+    EVSL_HIP(hipMemcpyAsync(xt.p, xd, tot * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
+    xd = xt.as<double>();
+  }
   std::vector<const double*> in(ncols);
   std::vector<double*> out(ncols);
   std::vector<const polparams*> pp(ncols);

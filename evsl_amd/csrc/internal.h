@@ -242,6 +242,8 @@ bool filter_op_ready(bool f32);
 // ---- whole series in one launch (series.cpp) ---------------------------------
 // Whether ncols columns of op's matrix run as a series launch of this degree.
 bool series_fits(const FilterOp& op, int ncols, int deg);
+// whether ncols columns of n rows are within what a series launch takes
+bool series_size(int n, int ncols);
 // One column: out = sum_k mu[k * mu_step] T_k(A~) in, mu on the device.
 struct SeriesCol {
   const FilterOp* op;

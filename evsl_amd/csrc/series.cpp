@@ -21,9 +21,13 @@ namespace evsl {
 bool series_fits(const FilterOp& op, int ncols, int deg) {
   const SeriesState& s = ctx().series;
   if (s.off || s.limit == 0 || !op.A.rmask || !op.A.pairs) return false;
-  if (deg < 8 || ncols > SeriesState::kSlots / 2 * evsl_dev::kSeriesMaxJobs) return false;
-  if (std::max(op.A.nneg, op.A.npair - op.A.nneg) > evsl_dev::kSeriesMaxHalf) return false;
-  return evsl_dev::series_rows_per_lane(op.A.n) <= evsl_dev::kSeriesMaxRows;
+  return deg >= 8 && series_size(op.A.n, ncols) &&
+         std::max(op.A.nneg, op.A.npair - op.A.nneg) <= evsl_dev::kSeriesMaxHalf;
+}
+
+bool series_size(int n, int ncols) {
+  return ncols <= SeriesState::kSlots / 2 * evsl_dev::kSeriesMaxJobs &&
+         evsl_dev::series_rows_per_lane(n) <= evsl_dev::kSeriesMaxRows;
 }
 
 namespace {

@@ -137,7 +137,7 @@ int ChebLanNr_batch(int nslices, double *intvs, int maxit, double tol, double *v
  * internal ChebAv, SRC/chebpoly.c:519-598): prec EVSL_PREC_FP64, or
  * EVSL_PREC_MIXED for the FP32 filter on the shifted matrix.  pols[j] (from
  * find_pol) may differ per column but must share cc and dd.  X and Y may be
- * host or device memory. */
+ * host or device memory, and may overlap. */
 int evsl_amd_cheb_av_cols(int ncols, const polparams *pols, const double *X, double *Y,
                           int prec);
 

@@ -3,13 +3,15 @@ of small row-mask matrices run as one and succeed, and that a failed one is
 noticed and its filter run again.
 
 Bar: the bits of the filter run one launch a degree (0 polls)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
 
 from evsl_amd import matrices as M
 from evsl_amd.evsl import PREC_FP64, PREC_MIXED
-from evsl_amd.types import HostCsr
+from evsl_amd.types import HostCsr, PolParams
 from test_gpu_series_tags import POLLS, sym_band
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +115,56 @@ def test_missing_workgroups(series, matrix, prec):
         assert (launched, failed) == (1, 1) and np.array_equal(Y, ref), groups
     for p in pols:
         ev.free_pol(p)
+
+
+def on_device(ev, pols, p_in, p_out, prec):
+    P = (PolParams * len(pols))(*pols)
+    return ev.lib.evsl_amd_cheb_av_cols(len(pols), P, C.cast(p_in, C.POINTER(C.c_double)),
+                                        C.cast(p_out, C.POINTER(C.c_double)), prec)
+
+
+@pytest.mark.parametrize("prec", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("cols", [1, 9])
+@pytest.mark.parametrize("n", [5000, 65536])
+def test_in_place(series, n, cols, prec):
+    ev = series
+    A = sym_band(n, [1], seed=2, keep=1.0)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, cols, deg=9)
+    X = np.asfortranarray(np.random.default_rng(5).uniform(-1.0, 1.0, (n, cols)))
+    ref, _, _ = run(ev, pols, X, prec, 0)
+    # one workgroup of an XCD missing: the rows far from its share are done before
+    # its neighbours' waits end
+    for polls, groups in ((POLLS, ALL), (2000, ALL - 8), (1, ALL)):
+        ev.set_series_workgroups(groups)
+        ev.set_series_polls(polls)
+        p = ev.to_device(X.T)
+        assert on_device(ev, pols, p, p, prec) == 0, ev.last_error()
+        Y = ev.from_device(p, n * cols).reshape(cols, n).T
+        ev.free_device(p)
+        assert np.array_equal(Y, ref), (polls, groups)
+    for q in pols:
+        ev.free_pol(q)
+
+
+@pytest.mark.parametrize("shift", [-3, 1, 5])
+@pytest.mark.parametrize("size,cols", [((64, 60, 1), 9), ((450, 450, 1), 20)])
+def test_ranges_that_overlap(series, size, cols, shift):
+    ev = series
+    A = M.laplacian(*size)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, cols, deg=9)
+    X = np.asfortranarray(np.random.default_rng(5).uniform(-1.0, 1.0, (A.n, cols)))
+    for prec in (PREC_FP64, PREC_MIXED):
+        ref, _, _ = run(ev, pols, X, prec, 0)
+        ev.set_series_polls(POLLS)
+        at = max(0, -shift)
+        whole = np.zeros((cols + abs(shift), A.n))
+        whole[at:at + cols] = X.T
+        p = ev.to_device(whole)
+        assert on_device(ev, pols, p + 8 * A.n * at, p + 8 * A.n * (at + shift), prec) == 0
+        Y = ev.from_device(p, whole.size).reshape(whole.shape)[at + shift:at + shift + cols].T
+        ev.free_device(p)
+        assert np.array_equal(Y, ref), prec
+    for q in pols:
+        ev.free_pol(q)
