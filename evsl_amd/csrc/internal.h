@@ -122,7 +122,7 @@ int ensure_a32_shifted(double cc, double scale, bool* ok);
 // cells carry next, the launches whose outcome has not been read yet, and where
 // they report it
 struct SeriesState {
-  static constexpr int kSlots = 64;     // launches between two checks
+  static constexpr int kSlots = 64;     // launches whose outcome may be open
   static constexpr int kSets = 256;     // counter sets (launches between clearings)
   DevBuf words;
   DevBuf ring;
@@ -132,6 +132,7 @@ struct SeriesState {
   unsigned id = 0;
   int limit = 200000;                   // polls of one wait; 0: no series launches
   int workgroups = evsl_dev::kSeriesXcds * evsl_dev::kSeriesParts;  // of a launch
+  bool failed = false;                  // one did since the last series_failed
   bool off = false;                     // a launch has failed (until set_series_polls, EVSLStart)
   long long launched = 0, failures = 0; // since EVSLStart
   struct Pending {

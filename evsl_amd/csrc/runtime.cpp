@@ -608,7 +608,7 @@ int EVSLStart(void) {
   // this fails, and reports the error there)
   void* scratch = nullptr;
   if (hipError_t e = evsl_dev::noalloc_scratch(&scratch); e != hipSuccess) (void)hipGetLastError();
-  c.series.off = false;
+  c.series.off = c.series.failed = false;
   c.series.launched = c.series.failures = 0;
   c.started = true;
   StatsReset();

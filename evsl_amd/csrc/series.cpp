@@ -49,6 +49,20 @@ int ensure_series() {
   return 0;
 }
 
+// reads the outcome of the pending launches, which have ended
+void collect() {
+  SeriesState& s = ctx().series;
+  for (size_t i = 0; i < s.pending.size(); ++i) {
+    const volatile unsigned* st = s.status + i * (1 + evsl_dev::kSeriesMaxJobs);
+    bool bad = st[0] == s.pending[i].id;
+    for (int j = 0; j < s.pending[i].njobs; ++j) bad = bad || st[1 + j] != s.pending[i].id;
+    s.failures += bad;
+    s.failed = s.failed || bad;
+  }
+  s.pending.clear();
+  s.off = s.off || s.failed;
+}
+
 }  // namespace
 
 int series_launch(const std::vector<SeriesCol>& cols) {
@@ -56,9 +70,9 @@ int series_launch(const std::vector<SeriesCol>& cols) {
   SeriesState& s = c.series;
   if (int e = ensure_series()) return e;
   for (size_t j0 = 0; j0 < cols.size(); j0 += evsl_dev::kSeriesMaxJobs) {
-    if ((int)s.pending.size() == SeriesState::kSlots) {  // none of the callers comes near
-      set_error_msg("series_launch: too many launches before a check");
-      return EVSL_ERR_DEVICE;
+    if ((int)s.pending.size() == SeriesState::kSlots) {  // many matrices, each on its own
+      EVSL_HIP(hipStreamSynchronize(c.stream));
+      collect();
     }
     // each launch has its own counters, cleared kSets launches at a time
     if (s.id % SeriesState::kSets == 0)
@@ -127,16 +141,9 @@ int series_launch(const std::vector<SeriesCol>& cols) {
 
 bool series_failed() {
   SeriesState& s = ctx().series;
-  bool bad = false;
-  for (size_t i = 0; i < s.pending.size(); ++i) {
-    const volatile unsigned* st = s.status + i * (1 + evsl_dev::kSeriesMaxJobs);
-    bool one = st[0] == s.pending[i].id;
-    for (int j = 0; j < s.pending[i].njobs; ++j) one = one || st[1 + j] != s.pending[i].id;
-    s.failures += one;
-    bad = bad || one;
-  }
-  s.pending.clear();
-  s.off = s.off || bad;
+  collect();
+  const bool bad = s.failed;
+  s.failed = false;
   return bad;
 }
 

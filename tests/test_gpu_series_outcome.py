@@ -10,7 +10,7 @@ import pytest
 import scipy.sparse as sp
 
 from evsl_amd import matrices as M
-from evsl_amd.evsl import PREC_FP64, PREC_MIXED
+from evsl_amd.evsl import PREC_FP64, PREC_MIXED, Server
 from evsl_amd.types import HostCsr, PolParams
 from test_gpu_series_tags import POLLS, sym_band
 
@@ -168,3 +168,39 @@ def test_ranges_that_overlap(series, size, cols, shift):
         assert np.array_equal(Y, ref), prec
     for q in pols:
         ev.free_pol(q)
+
+
+@pytest.mark.parametrize("polls", [POLLS, 1])
+def test_many_launches_before_a_check(series, polls):
+    # 33 matrices that are filtered each on its own (more than 32 MB a launch), two
+    # launches of at most 16 columns for each
+    ev = series
+    A = M.laplacian(65536, 1, 1)
+    lo, hi = M.gershgorin(A)
+    pol = ev.default_pol()
+    pol.damping, pol.thresh_int, pol.thresh_ext, pol.max_deg = 2, 0.8, 0.2, 300
+    v = np.random.default_rng(3).uniform(-1.0, 1.0, A.n)
+    got = []
+    for p in (0, polls):
+        ev.set_series_polls(p)
+        n0, f0, _ = ev.series_counts()
+        srv = Server(ev, 1 << 37, PREC_FP64)
+        ids = []
+        for m in range(33):
+            mid = srv.add_matrix(A, lo, hi)
+            for s in range(17):
+                a = lo + 0.4 + 0.1 * s
+                ids.append(srv.submit_slice(mid, a, a + 0.15, 3, 1e-8, v, pol))
+        while (more := srv.step()) > 0:
+            pass
+        assert more == 0, ev.last_error()
+        n1, f1, off = ev.series_counts()
+        if p == POLLS:
+            assert n1 - n0 >= 66 and f1 == f0 and not off
+        elif p == 1:
+            assert n1 - n0 >= 64 and f1 > f0 and off
+        out = [srv.slice_result(i, A.n) for i in ids]
+        got.append(out)
+        srv.close()
+    for a, b in zip(*got):
+        assert a[0] == b[0] == 0 and all(np.array_equal(x, y) for x, y in zip(a[1:], b[1:]))
