@@ -232,6 +232,8 @@ void spmm_tuner_destroy(SpmmTuner* t);
 int spmm_tuner_set(SpmmTuner* t, int B, bool fp32, Mode mode, int layout);
 // the layout a key is forced to, 0 when it is not
 int spmm_tuner_forced(SpmmTuner* t, int B, bool fp32, Mode mode);
+// whether a key of any width is
+bool spmm_tuner_any_forced(SpmmTuner* t, bool fp32, Mode mode);
 // layout the key launches now: the forced or chosen one, or the table's
 // while undecided
 int spmm_tuner_layout(SpmmTuner* t, int B, bool fp32, Mode mode);

@@ -17,10 +17,12 @@ namespace evsl {
 // 2.3 / 4.5 / 6.7 / 9.0; FP32 likewise (40^3: 4.5 / 6.0 / 8.8 / 8.8 against 2.0 /
 // 3.9 / 5.9 / 7.8).  So any number of columns does.  Larger matrices are left to
 // the launches, which use all XCDs for one column.  Eight degrees pay for the
-// launch.
+// launch.  A forced lane layout asks for the CSR kernel, whose launches the blocks
+// of any width then are.
 bool series_fits(const FilterOp& op, int ncols, int deg) {
   const SeriesState& s = ctx().series;
   if (s.off || s.limit == 0 || !op.A.rmask || !op.A.pairs) return false;
+  if (op.A.tune && evsl_dev::spmm_tuner_any_forced(op.A.tune, op.f32, evsl_dev::kCheb)) return false;
   return deg >= 8 && series_size(op.A.n, ncols) &&
          std::max(op.A.nneg, op.A.npair - op.A.nneg) <= evsl_dev::kSeriesMaxHalf;
 }

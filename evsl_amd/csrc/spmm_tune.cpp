@@ -134,6 +134,14 @@ int spmm_tuner_forced(SpmmTuner* t, int B, bool fp32, Mode mode) {
   return k->policy > 0 ? k->policy : 0;
 }
 
+bool spmm_tuner_any_forced(SpmmTuner* t, bool fp32, Mode mode) {
+  if (!t || (mode != kCheb && mode != kRes)) return false;
+  std::lock_guard<std::mutex> lock(t->mu);
+  for (const auto& k : t->key[fp32 ? 1 : 0][mode == kRes ? 1 : 0])
+    if (k.policy > 0) return true;
+  return false;
+}
+
 int spmm_tuner_layout(SpmmTuner* t, int B, bool fp32, Mode mode) {
   const int table = spmm_table_layout(B, fp32, mode);
   SpmmTuner::Key* k = key_of(t, B, fp32, mode);

@@ -292,7 +292,9 @@ int evsl_amd_spmm_index_mode(int B, int prec, int mode);
  * one bit mask per row, and its steps run k_cheb_mask<float|double, B, V, R,
  * mode, unsigned char|unsigned short, NT> (evsl_amd_spmm_layout gives 10*V +
  * R) -- the same products in the same order, so the results do not change --
- * unless evsl_amd_set_spmm_layout forces a lane layout of the CSR kernel.
+ * unless evsl_amd_set_spmm_layout forces a lane layout of the CSR kernel (one
+ * forced ChebAv width also keeps the precision's filters out of series
+ * launches, evsl_amd_set_series_polls).
  * The index modes and layouts above are the CSR kernel's. */
 int evsl_amd_spmm_row_masks(int B, int prec, int mode);
 /* Pattern codes (no reference counterpart): a matrix whose off-diagonal

@@ -204,3 +204,21 @@ def test_many_launches_before_a_check(series, polls):
         srv.close()
     for a, b in zip(*got):
         assert a[0] == b[0] == 0 and all(np.array_equal(x, y) for x, y in zip(a[1:], b[1:]))
+
+
+def test_forced_layout(series):
+    ev = series
+    A = M.laplacian(24, 24, 24)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, 4)
+    X = np.random.default_rng(5).uniform(-1.0, 1.0, (A.n, 4))
+    ref, launched, _ = run(ev, pols, X)
+    assert launched == 1
+    assert ev.set_spmm_layout(4, PREC_FP64, 1, 11) == 0
+    Y, launched, _ = run(ev, pols, X)
+    assert launched == 0 and np.array_equal(Y, ref)
+    assert run(ev, pols, X, PREC_MIXED)[1] == 1  # the mixed form's layouts are its own
+    assert ev.set_spmm_layout(4, PREC_FP64, 1, -1) == 0
+    assert run(ev, pols, X)[1] == 1
+    for p in pols:
+        ev.free_pol(p)
