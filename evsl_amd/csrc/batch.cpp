@@ -283,8 +283,9 @@ int filter_columns(int ncols, const double* const* xin, double* const* yout,
   int mindeg = maxdeg;
   for (int j = 0; j < ncols; ++j) mindeg = std::min(mindeg, pols[j]->deg);
   FilterOp sop;
-  if (int e = make_filter_op(pols[0]->cc, pols[0]->dd, f32, &sop)) return e;
-  if (ncols > 0 && series_fits(sop, ncols, mindeg)) {
+  if (mindeg > 0 && series_size(n, ncols))
+    if (int e = make_filter_op(pols[0]->cc, pols[0]->dd, f32, &sop)) return e;
+  if (series_fits(sop, ncols, mindeg)) {
     std::vector<const polparams*> key(pols, pols + ncols);
     BlockWork::CoefTab* ct = nullptr;
     // kind -2: the columns' coefficients one after the other
