@@ -163,9 +163,7 @@ hipError_t cheb_spmm_mask_f64(const Csr& A, int B, Mode mode, const void* xk, co
 //             yflush 3: y += s[c-2B]*xkm1, then += s[c-B]*xk, then += s[c]*w
 //             yflush 2: y += s[c-B]*xk, then += s[c]*w;  1: y += s[c]*w
 //             yflush 0: y untouched (neither read nor written)
-//   kKpm  : w as kCheb; xkp1 = w; the block's dots of W = kpm_dots values:
-//           FP64 part[blk*W + c] = sum_rows w*w, part[blk*W + B + c] =
-//           sum_rows w*xk (v0 unused); FP32 part[blk*W + c] = sum_rows w*v0
+//   kKpm  : w as kCheb; xkp1 = w; part[blk*B + c] = sum_rows w*v0
 //   kRes  : w = t*(acc - cc*xk) - xkm1 + s[c]*v0 (v0 = residual block R);
 //           xkp1 = w; y as kCheb with coefficients mu0[0] (this degree),
 //           mu0[-2], mu0[-4] (the two before) and mu0[1] for xk when first
@@ -287,36 +285,32 @@ int cheb_spmm_nblk(const Csr& A, int B, bool fp32, Mode mode);
 // instance (k_cheb_spmm<..., NT = true>)
 bool cheb_spmm_streaming(const Csr& A, int B, bool fp32, Mode mode);
 
-// KPM dots.  With T_a(x) T_b(x) = (T_{a+b}(x) + T_{|a-b|}(x)) / 2, the vectors
-// T_j v and T_{j-1} v give two moments at once,
-//   v.T_{2j} v = 2 T_j v.T_j v - v.v,  v.T_{2j-1} v = 2 T_j v.T_{j-1} v - v.T_1 v,
-// so an FP64 series of Mdeg moments runs (Mdeg + 1) / 2 steps, and both
-// factors are in registers where T_j v is formed (v itself is not read).
-// Measured, 300 moments: 40 vectors on the 100^3 Laplacian 104.0 -> 48.3 ms
-// (half the steps, three vector streams instead of four), 60 on a 100^2 grid
-// 12.4 -> 4.2 ms (with the sums of kKpmSumDegrees degrees in one launch).  The FP32
-// recurrence of the mixed form keeps v.T_k v at every step: its moments carry
-// the recurrence's FP32 rounding, which the products would change.
-constexpr int kpm_dots(int B, bool fp32) { return fp32 ? B : 2 * B; }
-// Columns of a KPM block: 32, or fewer where the three FP64 vector blocks of
-// 32 columns outgrow 200 MB (n > 260,000) and the rows are regular (a row has
-// its neighbour's column offsets, so a gather reads contiguous segments and
-// the matrix is a small part of a step): 16 while that keeps them under it,
-// else 8.  The blocks then stay in the 256 MB Infinity Cache from step to
-// step (100^3, us per column and step at 32 / 16 / 8 columns: row-mask kernel
-// 6.5 / 6.5 / 4.1, CSR kernel 7.1 / 7.5 / 5.9); irregular rows pay for their
-// gathers by the segment, so wider is better (300,000 random rows of 3-9: 2.6
-// / 3.0 / 4.6).  One rule for every KPM path: moments depend on the width.
+// A KPM series forms v.T_k v at every step.  T_j v.T_j v and T_j v.T_{j-1} v would
+// give two moments a step (2 T_a T_b = T_{a+b} + T_{|a-b|}) in half the time, but
+// the rounding of T_j v is correlated with T_j v, not with v, and comes in twice:
+// against an 80-bit recurrence, 200 moments of 20 vectors, of their norm 3.8e-15
+// instead of 2.1e-16 on a 64 x 60 grid, 3.8e-16 instead of 1.0e-16 on 5,000 random
+// rows, and with exact dots still more than v.T_k v.
+
+// Columns of a KPM block: 32, or fewer where the four FP64 vector blocks of a step
+// at 32 columns outgrow 256 MB, the Infinity Cache (n > 250,000), and the rows are
+// regular (a row has its neighbour's column offsets, so a gather reads contiguous
+// segments and the matrix is a small part of a step): 16 while that keeps them
+// under it, else 8.  The blocks then stay there from step to step (us per column
+// and step at 32 / 16 / 8 columns, row-mask kernel, CSR kernel: 58^3 1.0 / 1.1 /
+// 1.3, 1.1 / 1.4 / 1.8; 68^3 2.3 / 1.6 / 1.9, 2.5 / 2.0 / 2.5; 90^3 5.5 / 5.6 /
+// 3.5, 5.8 / 6.2 / 4.6; 100^3 7.4 / 7.5 / 5.6, 7.9 / 8.3 / 8.4); irregular rows pay
+// for their gathers by the segment, so wider is better (131,072 random rows of
+// 3-70: 5.4 / 5.1 / 7.1).  One rule for every KPM path: moments depend on the width.
 inline int kpm_max_width(int n, bool regular) {
-  if (!regular || 24.0 * n * 32 <= 200e6) return 32;
-  return 24.0 * n * 16 <= 200e6 ? 16 : 8;
+  if (!regular || 32.0 * n * 32 <= 256e6) return 32;
+  return 32.0 * n * 16 <= 256e6 ? 16 : 8;
 }
-// steps of a series of Mdeg moments
-inline int kpm_steps(int Mdeg, bool fp32) { return fp32 ? Mdeg : (Mdeg + 1) / 2; }
+
 // degrees whose block partials are kept and then summed by one launch: the
 // sums of one degree are a launch or two of 5-7 us beside a step of 5 us at
 // n = 10^4.  At most kKpmSumDegrees, fewer where the partials of one degree
-// (nblk * W values) are large.
+// (nblk * B values) are large.
 constexpr int kKpmSumDegrees = 16;
 inline int kpm_sum_degrees(size_t part_values) {
   const size_t d = ((size_t)4 << 20) / (part_values ? part_values : 1);
@@ -387,10 +381,9 @@ int kpm_start_blocks(size_t n, int B);
 hipError_t kpm_group_start(bool fp32, int B, const KpmStartEntry* tab, int nr, int maxn, int kind,
                            int col0, hipStream_t st);
 
-// The partial sums of one grouped matrix: nblk block partials (W = kpm_dots
-// per block) of each of nd degrees, summed as sum_block_partials does (G
-// first-level blocks into scratch, then one; or directly when G == 1) into
-// dots + (k+1)*W.
+// The partial sums of one grouped matrix: nblk block partials (B per block) of
+// each of nd degrees, summed as sum_block_partials does (G first-level blocks
+// into scratch, then one; or directly when G == 1) into dots + (k+1)*B.
 struct KpmSumEntry {
   const double* part;
   double* scratch;
@@ -406,20 +399,20 @@ hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int*
 // the partial sums of the steps k .. k + nd - 1 (places 0 .. nd - 1): level 1
 // over nl1 blocks (owner1/first1), level 2 over the two-level entries listed
 // in owner2
-hipError_t kpm_group_sums(bool fp32, int B, const KpmSumEntry* sums, int k, int nd,
+hipError_t kpm_group_sums(int B, const KpmSumEntry* sums, int k, int nd,
                           const int* owner1, const int* first1, int nl1, const int* owner2,
                           int nl2, hipStream_t st);
 
-// out[d*W + c] = sum_b part[(d*nblk + b)*W + c] over nblk row blocks, in a
+// out[d*B + c] = sum_b part[(d*nblk + b)*B + c] over nblk row blocks, in a
 // fixed order, for nd consecutive degrees d in one launch; uses scratch (nd *
 // kSumScratch doubles) for a first level when nblk is large
-constexpr int kSumScratch = 256 * 64;
-// first-level blocks of sum_block_partials for (nblk, W): 1 when it sums
+constexpr int kSumScratch = 256 * 32;
+// first-level blocks of sum_block_partials for (nblk, B): 1 when it sums
 // directly, else 256
-inline int sum_levels_blocks(int nblk, int W) {
-  return ((size_t)nblk * W <= 16384) ? 1 : 256;
+inline int sum_levels_blocks(int nblk, int B) {
+  return ((size_t)nblk * B <= 16384) ? 1 : 256;
 }
-hipError_t sum_block_partials(const double* part, int nblk, int W, int nd, double* out,
+hipError_t sum_block_partials(const double* part, int nblk, int B, int nd, double* out,
                               double* scratch, hipStream_t st);
 
 // Fixed-grid reductions: partial buffers hold kRedBlocks entries.

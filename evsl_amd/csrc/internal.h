@@ -373,9 +373,8 @@ struct GroupedWork {
 int grouped_filter(const std::vector<GroupedCols>& parts, GroupedWork& W);
 
 // raw[k] (k >= 1) += the B columns' v^T T_k v from the dots of a series in the
-// order sum_block_partials leaves them (row j: the W = kpm_dots values of
-// step j - 1)
-void kpm_add_dots(int Mdeg, bool f32, int B, const double* dots, double* raw);
+// order sum_block_partials leaves them (row k: degree k)
+void kpm_add_dots(int Mdeg, int B, const double* dots, double* raw);
 // KPM moments and eigenvalue count from raw[k] = sum over the nvec vectors of
 // v^T T_k(A~) v (k >= 1), as kpmdos finishes them
 void kpm_moments(int Mdeg, int damping, int nvec, const double* intv, int n, const double* raw,

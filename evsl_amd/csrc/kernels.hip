@@ -1298,29 +1298,28 @@ hipError_t kpm_group_step(bool fp32, int B, const KpmGroupEntry* tab, const int*
   return hipGetLastError();
 }
 
-hipError_t kpm_group_sums(bool fp32, int B, const KpmSumEntry* sums, int k, int nd,
+hipError_t kpm_group_sums(int B, const KpmSumEntry* sums, int k, int nd,
                           const int* owner1, const int* first1, int nl1, const int* owner2,
                           int nl2, hipStream_t st) {
   if (nl1 <= 0 || nd <= 0) return hipErrorInvalidValue;
-  const int W = kpm_dots(B, fp32);
-  hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl1, nd), dim3(kWG), 0, st, sums, owner1, first1, W,
+  hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl1, nd), dim3(kWG), 0, st, sums, owner1, first1, B,
                      k, 1);
   if (nl2 > 0)
     hipLaunchKernelGGL(k_kpm_group_sums, dim3(nl2, nd), dim3(kWG), 0, st, sums, owner2,
-                       (const int*)nullptr, W, k, 2);
+                       (const int*)nullptr, B, k, 2);
   return hipGetLastError();
 }
 
-hipError_t sum_block_partials(const double* part, int nblk, int W, int nd, double* out,
+hipError_t sum_block_partials(const double* part, int nblk, int B, int nd, double* out,
                               double* scratch, hipStream_t st) {
-  if (W < 1 || W > 64 || nd < 1) return hipErrorInvalidValue;
-  const int G = sum_levels_blocks(nblk, W);
+  if (B < 1 || B > 32 || nd < 1) return hipErrorInvalidValue;
+  const int G = sum_levels_blocks(nblk, B);
   if (G > 1 && !scratch) return hipErrorInvalidValue;
   double* first = G > 1 ? scratch : out;
-  hipLaunchKernelGGL(k_sum_block_partials, dim3(G, nd), dim3(kWG), 0, st, part, nblk, W, first);
+  hipLaunchKernelGGL(k_sum_block_partials, dim3(G, nd), dim3(kWG), 0, st, part, nblk, B, first);
   if (G > 1)
     hipLaunchKernelGGL(k_sum_block_partials, dim3(1, nd), dim3(kWG), 0, st,
-                       (const double*)first, G, W, out);
+                       (const double*)first, G, B, out);
   return hipGetLastError();
 }
 

@@ -45,21 +45,9 @@ void kpm_moments(int Mdeg, int damping, int nvec, const double* intv, int n, con
   *ecnt = tcnt * t * (double)n;
 }
 
-void kpm_add_dots(int Mdeg, bool f32, int B, const double* dots, double* raw) {
-  const int W = evsl_dev::kpm_dots(B, f32);
-  const double* d1 = dots + W;  // the first step's: v.T_1 v behind T_1 v.T_1 v
-  for (int j = 1; j <= evsl_dev::kpm_steps(Mdeg, f32); ++j) {
-    const double* d = dots + (size_t)j * W;
-    for (int col = 0; col < B; ++col) {
-      if (f32) {
-        raw[j] += d[col];
-        continue;
-      }
-      // unit vectors: v.v = 1
-      raw[2 * j - 1] += j == 1 ? d[B + col] : 2.0 * d[B + col] - d1[B + col];
-      if (2 * j <= Mdeg) raw[2 * j] += 2.0 * d[col] - 1.0;
-    }
-  }
+void kpm_add_dots(int Mdeg, int B, const double* dots, double* raw) {
+  for (int k = 1; k <= Mdeg; ++k)
+    for (int col = 0; col < B; ++col) raw[k] += dots[(size_t)k * B + col];
 }
 
 namespace {
@@ -75,14 +63,10 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
   const double ctr = (intv[3] + intv[2]) / 2.0, wid = (intv[3] - intv[2]) / 2.0;
   std::vector<double> raw(Mdeg + 1, 0.0);  // raw[k] = sum_m v_m . T_k v_m
   const int Bmax = c.op == 1 ? evsl_dev::kpm_max_width(n, c.A.regular) : 32;
-  // FP64 on a CSR matrix: two moments a step (kpm_dots); a user operator's
-  // series takes v.T_k v at every step
-  const bool pairs = c.op == 1;
-  const int steps = evsl_dev::kpm_steps(Mdeg, !pairs);
   DevBuf X0, X, dots, part, scratch;
   EVSL_HIP(X0.alloc((size_t)n * Bmax * sizeof(double)));
   EVSL_HIP(X.alloc((size_t)3 * n * Bmax * sizeof(double)));
-  EVSL_HIP(dots.alloc((size_t)(steps + 1) * evsl_dev::kpm_dots(Bmax, !pairs) * sizeof(double)));
+  EVSL_HIP(dots.alloc((size_t)(Mdeg + 1) * Bmax * sizeof(double)));
   std::vector<double> hbuf, hcol, hdots;
   const evsl_dev::Csr A = c.A.view();
   int done = 0;
@@ -111,13 +95,12 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
     if (c.op == 1) {
       const int nblk_kpm = evsl_dev::cheb_spmm_nblk(A, B, false, evsl_dev::kKpm);
       if (nblk_kpm < 0) return EVSL_ERR_ARG;
-      const int W = evsl_dev::kpm_dots(B, false);
-      const size_t pv = (size_t)nblk_kpm * W;
-      const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
+      const size_t pv = (size_t)nblk_kpm * B;
+      const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), Mdeg));
       EVSL_HIP(part.alloc(nd * pv * sizeof(double)));
-      if (evsl_dev::sum_levels_blocks(nblk_kpm, W) > 1)
+      if (evsl_dev::sum_levels_blocks(nblk_kpm, B) > 1)
         EVSL_HIP(scratch.alloc((size_t)nd * evsl_dev::kSumScratch * sizeof(double)));
-      for (int k = 0; k < steps; ++k) {
+      for (int k = 0; k < Mdeg; ++k) {
         const double sc = (k == 0 ? 1.0 : 2.0) / wid;
         void* xkp1 = buf[k % 3];
         const void* xk = (k == 0) ? x0 : buf[(k - 1) % 3];
@@ -125,17 +108,17 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
         EVSL_HIP(evsl_dev::cheb_spmm(A, B, false, evsl_dev::kKpm, xk, xkm1, xkp1, nullptr, x0,
                                      nullptr, nullptr, sc, ctr, false, 0,
                                      part.as<double>() + (k % nd) * pv, c.stream));
-        if ((k + 1) % nd == 0 || k + 1 == steps) {
+        if ((k + 1) % nd == 0 || k + 1 == Mdeg) {
           const int have = k % nd + 1;
-          EVSL_HIP(evsl_dev::sum_block_partials(part.as<double>(), nblk_kpm, W, have,
-                                                dots.as<double>() + (size_t)(k + 2 - have) * W,
+          EVSL_HIP(evsl_dev::sum_block_partials(part.as<double>(), nblk_kpm, B, have,
+                                                dots.as<double>() + (size_t)(k + 2 - have) * B,
                                                 scratch.as<double>(), c.stream));
         }
         c.astats.filter_bytes += c.A.mat_bytes(8, B) +
-                                 (double)(k == 0 ? 2 : 3) * nb * sizeof(double);
+                                 (double)(k == 0 ? 3 : 4) * nb * sizeof(double);
       }
-      c.astats.n_filter_steps += steps;
-      c.astats.n_filter_cols += (size_t)steps * B;
+      c.astats.n_filter_steps += Mdeg;
+      c.astats.n_filter_cols += (size_t)Mdeg * B;
     } else {
       // user operator: one column at a time through the callback
       DevBuf col;
@@ -167,10 +150,10 @@ int kpm_impl(int Mdeg, int damping, int nvec, const double* intv, int kind,
       }
       EVSL_HIP(hipMemcpy(dots.p, dh.data(), dh.size() * sizeof(double), hipMemcpyHostToDevice));
     }
-    hdots.resize((size_t)(steps + 1) * evsl_dev::kpm_dots(B, !pairs));
+    hdots.resize((size_t)(Mdeg + 1) * B);
     EVSL_HIP(hipMemcpy(hdots.data(), dots.p, hdots.size() * sizeof(double),
                        hipMemcpyDeviceToHost));
-    kpm_add_dots(Mdeg, !pairs, B, hdots.data(), raw.data());
+    kpm_add_dots(Mdeg, B, hdots.data(), raw.data());
     done += B;
   }
   kpm_moments(Mdeg, damping, nvec, intv, n, raw.data(), mu, ecnt);
@@ -382,12 +365,12 @@ int evsl_amd_bench_filter(int B, int prec, int mode, int nsteps, double cc, doub
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *ms_per_step = ms / nsteps;
-  // per launch: KPM xk (gathered once), xkm1 in, xkp1 out; ChebAv xk,
+  // per launch: KPM xk (gathered once), xkm1, v0 in, xkp1 out; ChebAv xk,
   // xkm1 in, xkp1 out, plus the FP64 y in and out on a flush; the residual
   // recurrence adds the residual block R
   double vbytes;
   if (mode == 2)
-    vbytes = 3.0 * vs;
+    vbytes = 4.0 * vs;
   else
     vbytes = 3.0 * vs + 16.0 * flushes / nsteps + (mode == 3 ? vs : 0.0);
   *bytes_per_step = c.A.mat_bytes((int)vs, B) + vbytes * nb;

@@ -225,23 +225,21 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
       if (V <= 0 || R <= 0) return EVSL_ERR_ARG;
       const int lanes = B / V / R;
-      // values per block partial, steps, and the degrees summed by one launch
-      const int W = evsl_dev::kpm_dots(B, f32), steps = evsl_dev::kpm_steps(Mdeg, f32);
       size_t pv = 0;
       int maxn = 0, total = 0;
       std::vector<int> nblk(nr), G(nr), owner, owner1, first1(nr), owner2;
       for (int r = 0; r < nr; ++r) {
         BatchMatrix& m = *reqs[r]->mat;
         nblk[r] = (int)(m.row_blocks(lanes).size() / 2) - 1;
-        G[r] = evsl_dev::sum_levels_blocks(nblk[r], W);
-        pv = std::max(pv, (size_t)nblk[r] * W);
+        G[r] = evsl_dev::sum_levels_blocks(nblk[r], B);
+        pv = std::max(pv, (size_t)nblk[r] * B);
         maxn = std::max(maxn, m.n);
         owner.insert(owner.end(), nblk[r], r);
         first1[r] = (int)owner1.size();
         owner1.insert(owner1.end(), G[r], r);
         if (G[r] > 1) owner2.push_back(r);
       }
-      const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), steps));
+      const int nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees(pv), Mdeg));
       // what the host fills in comes first and goes over in one copy
       Places p;
       const size_t tab_at = p.take(nr * sizeof(evsl_dev::KpmGroupEntry));
@@ -255,7 +253,7 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       for (int r = 0; r < nr; ++r)
         if (!rbp_at.count(reqs[r]->mat))
           rbp_at[reqs[r]->mat] = p.take(reqs[r]->mat->row_blocks(lanes).size() * sizeof(int));
-      const size_t up_bytes = p.end, dots1 = (size_t)(steps + 1) * W;
+      const size_t up_bytes = p.end, dots1 = (size_t)(Mdeg + 1) * B;
       const size_t dots_at = p.take(nr * dots1 * sizeof(double));
       struct At {
         size_t x0, ring, part, scratch, npart, nrm2;
@@ -265,8 +263,8 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
         const size_t n = reqs[r]->mat->n, nb = n * B;
         at[r].x0 = p.take(nb * vs);
         at[r].ring = p.take(3 * nb * vs);
-        at[r].part = p.take((size_t)nd * nblk[r] * W * sizeof(double));
-        at[r].scratch = p.take(G[r] > 1 ? (size_t)nd * G[r] * W * sizeof(double) : 0);
+        at[r].part = p.take((size_t)nd * nblk[r] * B * sizeof(double));
+        at[r].scratch = p.take(G[r] > 1 ? (size_t)nd * G[r] * B * sizeof(double) : 0);
         at[r].npart = p.take((size_t)evsl_dev::kpm_start_blocks(n, B) * B * sizeof(double));
         at[r].nrm2 = p.take(B * sizeof(double));
       }
@@ -302,7 +300,7 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
         e.n = m.n;
         e.blk0 = total;
         e.k0 = 0;
-        e.part_step = nblk[r] * W;
+        e.part_step = nblk[r] * B;
         total += nblk[r];
         evsl_dev::KpmSumEntry& s = sums[r];
         s.part = e.part;
@@ -328,28 +326,28 @@ int kpmdos_batch(int nreq, csrMat* const* mats, const double* intvs, int Mdeg, i
       double step_bytes = 0.0;
       for (int r = 0; r < nr; ++r)
         step_bytes += (double)reqs[r]->mat->nnz * (vs + 4) + 4.0 * (reqs[r]->mat->n + 1) +
-                      (f32 ? 4.0 : 3.0) * reqs[r]->mat->n * B * vs;
+                      4.0 * reqs[r]->mat->n * B * vs;
       auto ints = [&](size_t from) { return reinterpret_cast<const int*>(d + from); };
-      for (int k = 0; k < steps; ++k) {
+      for (int k = 0; k < Mdeg; ++k) {
         EVSL_HIP(evsl_dev::kpm_group_step(
             f32, B, reinterpret_cast<const evsl_dev::KpmGroupEntry*>(d + tab_at), ints(owner_at),
             total, k, k % nd, c.stream));
-        if ((k + 1) % nd == 0 || k + 1 == steps) {
+        if ((k + 1) % nd == 0 || k + 1 == Mdeg) {
           const int have = k % nd + 1;
           EVSL_HIP(evsl_dev::kpm_group_sums(
-              f32, B, reinterpret_cast<const evsl_dev::KpmSumEntry*>(d + sums_at), k + 1 - have,
+              B, reinterpret_cast<const evsl_dev::KpmSumEntry*>(d + sums_at), k + 1 - have,
               have, ints(owner1_at), ints(first1_at), (int)owner1.size(), ints(owner2_at),
               (int)owner2.size(), c.stream));
         }
         c.astats.filter_bytes += step_bytes;
       }
-      c.astats.n_filter_steps += steps;
-      c.astats.n_filter_cols += (size_t)steps * B * nr;
+      c.astats.n_filter_steps += Mdeg;
+      c.astats.n_filter_cols += (size_t)Mdeg * B * nr;
       hdots.resize(nr * dots1);
       EVSL_HIP(hipMemcpy(hdots.data(), d + dots_at, hdots.size() * sizeof(double),
                          hipMemcpyDeviceToHost));
       for (int r = 0; r < nr; ++r)
-        kpm_add_dots(Mdeg, f32, B, hdots.data() + r * dots1, reqs[r]->raw.data());
+        kpm_add_dots(Mdeg, B, hdots.data() + r * dots1, reqs[r]->raw.data());
       done += B;
     }
   }

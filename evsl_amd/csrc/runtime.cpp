@@ -431,7 +431,7 @@ int build_device_matrix(int n, int nnz, int* ia_d, int* ja_d, double* a_d, const
     }
     EVSL_HIP(hipMalloc((void**)&M.rb[w], rbp.size() * sizeof(int)));
     EVSL_HIP(hipMemcpy(M.rb[w], rbp.data(), rbp.size() * sizeof(int), hipMemcpyHostToDevice));
-    need = std::max(need, (size_t)(M.nblk[w] + 1) * 2 * B);  // kpm_dots in FP64
+    need = std::max(need, (size_t)(M.nblk[w] + 1) * B);
   }
   // reduction scratch: the largest per-row-block partial buffer and a Lanczos
   // step's partials

@@ -80,7 +80,7 @@ struct SrvRequest {
   int Mdeg = 0, damping = 0, nvec = 0, vec_kind = 0;
   unsigned long long seed = 0;
   int done_vec = 0, B = 0, k = 0, nblk = 0, G = 1;
-  int steps = 0, nd = 1;  // steps of a column block; degrees its partials hold
+  int nd = 1;  // degrees its partials hold
   double t0 = 0, t = 0, cc = 0;
   const float* a32 = nullptr;
   DevBuf x0, ring, part, dots, scratch;
@@ -144,17 +144,15 @@ int dos_round(evslAmdServer* s, SrvRequest& q) {
   const int slot = evsl_dev::width_slot(B / V / R);
   if (slot < 0) return EVSL_ERR_ARG;
   q.nblk = m.M.nblk[slot];
-  const int W = evsl_dev::kpm_dots(B, f32);
-  q.steps = evsl_dev::kpm_steps(q.Mdeg, f32);
-  q.nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees((size_t)q.nblk * W), q.steps));
-  q.G = evsl_dev::sum_levels_blocks(q.nblk, W);
+  q.nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees((size_t)q.nblk * B), q.Mdeg));
+  q.G = evsl_dev::sum_levels_blocks(q.nblk, B);
   const int n = m.M.n;
   const size_t nb = (size_t)n * B;
   EVSL_HIP(q.x0.alloc(nb * vs));
   EVSL_HIP(q.ring.alloc(3 * nb * vs));
-  EVSL_HIP(q.part.alloc((size_t)q.nd * std::max(q.nblk, 1) * W * sizeof(double)));
-  EVSL_HIP(q.dots.alloc((size_t)(q.steps + 1) * W * sizeof(double)));
-  if (q.G > 1) EVSL_HIP(q.scratch.alloc((size_t)q.nd * q.G * W * sizeof(double)));
+  EVSL_HIP(q.part.alloc((size_t)q.nd * std::max(q.nblk, 1) * B * sizeof(double)));
+  EVSL_HIP(q.dots.alloc((size_t)(q.Mdeg + 1) * B * sizeof(double)));
+  if (q.G > 1) EVSL_HIP(q.scratch.alloc((size_t)q.nd * q.G * B * sizeof(double)));
   EVSL_HIP(s->x64.alloc(nb * sizeof(double)));
   EVSL_HIP(s->nrm_part.alloc((size_t)1024 * 32 * sizeof(double)));
   EVSL_HIP(s->nrm2.alloc(32 * sizeof(double)));
@@ -294,7 +292,7 @@ int dos_steps(evslAmdServer* s) {
     std::vector<int> ids;
     int B = 0;
     for (auto& r : s->reqs)
-      if (r->kind == 1 && r->state == 1 && r->k < r->steps && (B == 0 || r->B == B)) {
+      if (r->kind == 1 && r->state == 1 && r->k < r->Mdeg && (B == 0 || r->B == B)) {
         B = r->B;
         ids.push_back(r->id);
       }
@@ -324,7 +322,7 @@ int dos_steps(evslAmdServer* s) {
       e.n = m.M.n;
       e.blk0 = total;
       e.k0 = (int)(s->kg - q.k);
-      e.part_step = q.nblk * evsl_dev::kpm_dots(B, f32);
+      e.part_step = q.nblk * B;
       owner.insert(owner.end(), q.nblk, i);
       total += q.nblk;
       evsl_dev::KpmSumEntry& se = sums[i];
@@ -348,7 +346,7 @@ int dos_steps(evslAmdServer* s) {
     // launches while the membership stays the same
     int run = budget, nd = evsl_dev::kKpmSumDegrees;
     for (int id : ids) {
-      run = std::min(run, s->reqs[id]->steps - s->reqs[id]->k);
+      run = std::min(run, s->reqs[id]->Mdeg - s->reqs[id]->k);
       nd = std::min(nd, s->reqs[id]->nd);
     }
     for (int j = 0; j < run; ++j) {
@@ -357,7 +355,7 @@ int dos_steps(evslAmdServer* s) {
                                         ctx().stream));
       if ((j + 1) % nd == 0 || j + 1 == run) {
         const int have = j % nd + 1;
-        EVSL_HIP(evsl_dev::kpm_group_sums(f32, B, s->d_sums.as<evsl_dev::KpmSumEntry>(),
+        EVSL_HIP(evsl_dev::kpm_group_sums(B, s->d_sums.as<evsl_dev::KpmSumEntry>(),
                                           (int)s->kg + 1 - have, have, s->d_owner1.as<int>(),
                                           s->d_first1.as<int>(), (int)owner1.size(),
                                           s->d_owner2.as<int>(), (int)owner2.size(),
@@ -370,10 +368,10 @@ int dos_steps(evslAmdServer* s) {
     // requests whose column block is through: moments, next block or done
     for (int id : ids) {
       SrvRequest& q = *s->reqs[id];
-      if (q.k < q.steps) continue;
-      std::vector<double> h((size_t)(q.steps + 1) * evsl_dev::kpm_dots(q.B, f32));
+      if (q.k < q.Mdeg) continue;
+      std::vector<double> h((size_t)(q.Mdeg + 1) * q.B);
       EVSL_HIP(hipMemcpy(h.data(), q.dots.p, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-      kpm_add_dots(q.Mdeg, f32, q.B, h.data(), q.raw.data());
+      kpm_add_dots(q.Mdeg, q.B, h.data(), q.raw.data());
       q.done_vec += q.B;
       if (q.done_vec < q.nvec) {
         if (int e = dos_round(s, q)) return e;

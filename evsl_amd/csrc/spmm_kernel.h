@@ -44,9 +44,6 @@ struct alignas(sizeof(VT) * V) VecT {
 // out of L2; it pays when the launch's working set exceeds the Infinity
 // Cache (chosen per launch, streaming_launch below) and leaves the
 // arithmetic unchanged.
-// a KPM step of this vector type sums the pair (w.w, w.xk) per column
-template <typename VT>
-constexpr bool kKpmPairs = kpm_dots(1, sizeof(VT) == 4) == 2;
 template <typename T, int V>
 struct ExtVec {
   typedef T type __attribute__((ext_vector_type(V)));
@@ -175,12 +172,9 @@ __device__ __forceinline__ void cheb_spmm_block(
   }
   const bool ymode = MODE == kCheb || MODE == kRes;
   const bool need_xr = first || MODE == kKpm || cc_ != 0.0 || (ymode && yflush >= 2);
-  // kKpm dots of this lane's columns: in FP64 dacc = w.w and dacc1 = w.xk
-  // (two moments a degree, see dev.h), in FP32 dacc = w.v0
-  constexpr bool kPairs = MODE == kKpm && kKpmPairs<VT>;
-  double dacc[V], dacc1[V];
+  double dacc[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) dacc[j] = dacc1[j] = 0.0;
+  for (int j = 0; j < V; ++j) dacc[j] = 0.0;
 
   // epilogue operands of a row, loaded ahead of the gathers
   struct Ops {
@@ -223,7 +217,7 @@ __device__ __forceinline__ void cheb_spmm_block(
     if (xkm1) o.km1 = ld_last(xkm1, i);
     if (ymode && yflush > 0 && !first) o.yo = ld_last(y, i);
     if (MODE == kRes) o.rr = ld(v0, i);
-    if (MODE == kKpm && !kPairs) o.v = ld(v0, i);
+    if (MODE == kKpm) o.v = ld(v0, i);
     return o;
   };
   auto epilogue = [&](int r, const VT* acc, const Ops& o) {
@@ -262,14 +256,7 @@ __device__ __forceinline__ void cheb_spmm_block(
       }
     } else if (MODE == kKpm) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) {
-        if (kPairs) {
-          dacc[j] += (double)w.v[j] * (double)w.v[j];
-          dacc1[j] += (double)w.v[j] * (double)o.xr.v[j];
-        } else {
-          dacc[j] += (double)w.v[j] * (double)o.v.v[j];
-        }
-      }
+      for (int j = 0; j < V; ++j) dacc[j] += (double)w.v[j] * (double)o.v.v[j];
     }
   };
 
@@ -472,24 +459,19 @@ __device__ __forceinline__ void cheb_spmm_block(
 
   if (MODE == kKpm) {  // L is a power of two here (NG*L == kWG)
     static_assert(MODE != kKpm || (kWG % L) == 0, "KPM blocks need B/V | 256");
-    constexpr int W = kpm_dots(B, sizeof(VT) == 4);
 #pragma unroll
-    for (int h = 0; h < W / B; ++h) {
-      if (h) __syncthreads();
+    for (int j = 0; j < V; ++j) s_red[tid * V + j] = dacc[j];
+    __syncthreads();
+    for (int st = NG / 2; st > 0; st >>= 1) {
+      if (grp < st) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) s_red[tid * V + j] = h ? dacc1[j] : dacc[j];
+        for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
+      }
       __syncthreads();
-      for (int st = NG / 2; st > 0; st >>= 1) {
-        if (grp < st) {
+    }
+    if (grp == 0) {
 #pragma unroll
-          for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
-        }
-        __syncthreads();
-      }
-      if (grp == 0) {
-#pragma unroll
-        for (int j = 0; j < V; ++j) part[(size_t)blk * W + h * B + c0 + j] = s_red[tid * V + j];
-      }
+      for (int j = 0; j < V; ++j) part[(size_t)blk * B + c0 + j] = s_red[tid * V + j];
     }
   }
 }
@@ -623,10 +605,10 @@ hipError_t launch_variant(const Csr& A, const void* xk, const void* xkm1, void* 
 // little (us a degree of all requests, R = 1 layout -> the one taken, large /
 // small): 4 columns V2R1 46 -> V2R2 35 / 9.2 -> 9.4, 8 V2R1 60 -> V4R2 42 / 10.2
 // -> 10.5, 16 V2R1 87 -> V4R4 57 / 15.0 -> 15.5, 32 V4R1 154 -> V4R8 98 / 24.4 ->
-// 24.2.  The FP64 KPM row was swept for its two dots a step in both kernels that share
-// it (100^3, row-mask / CSR kernel, us): 2 columns V2R1 13.0 / 23.4 against
-// V1R1 16.9 / 24.3, 4 V2R1 19.2 / 33.1 against V1R2 28.0 / 33.9, 8 V2R2 32.8 /
-// 47.4 against V4R1 37.6 / 54.0.
+// 24.2.  The FP64 KPM row was swept in both kernels that share it (100^3, row-mask / CSR
+// kernel, us): 2 columns V2R1 12.6 / 22.2 against V1R1 16.2 / 24.4, 4 V2R1 19.7 /
+// 34.1 against V1R2 28.2 / 34.1, 8 V2R2 45.1 / 67.3 against V4R1 45.1 / 68.2 (75^3
+// 18.4 / 24.7 against 18.7 / 25.5).
 //                                    B =  2   4   6   8  16  32
 constexpr int kSpmmLayout[2][3][6] = {{{21, 22, 21, 22, 44, 44},    // FP32 ChebAv
                                        {21, 22, 21, 42, 44, 48},    // FP32 KPM

@@ -62,10 +62,9 @@ __global__ __launch_bounds__(kWG) void k_cheb_mask(
   const int grp = tid / L, c0 = (tid % L) * V;
   const VT t = (VT)t_, cc = (VT)cc_;
   constexpr bool kY = MODE == kCheb || MODE == kRes;
-  constexpr bool kPairs = MODE == kKpm && kKpmPairs<VT>;
-  double dacc[V], dacc1[V];
+  double dacc[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) dacc[j] = dacc1[j] = 0.0;
+  for (int j = 0; j < V; ++j) dacc[j] = 0.0;
   auto ld = [](const VT* p) { return *reinterpret_cast<const Vec*>(p); };
   auto ld_last = [](const auto* p) {
     using ET = typename std::remove_cv<typename std::remove_reference<decltype(*p)>::type>::type;
@@ -108,7 +107,7 @@ __global__ __launch_bounds__(kWG) void k_cheb_mask(
     VecY yo{};
     if (MODE != kPlain && xkm1) km1 = ld_last(xkm1 + base + li);
     if (kY && yflush > 0 && !first) yo = ld_last(y + base + li);
-    if (MODE == kRes || (MODE == kKpm && !kPairs)) rr = ld(v0 + base + li);
+    if (MODE == kRes || MODE == kKpm) rr = ld(v0 + base + li);
     VT acc[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] = 0;
@@ -173,14 +172,7 @@ __global__ __launch_bounds__(kWG) void k_cheb_mask(
     }
     if (MODE == kKpm) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) {
-        if (kPairs) {
-          dacc[j] = fma_((double)w.v[j], (double)w.v[j], dacc[j]);
-          dacc1[j] = fma_((double)w.v[j], (double)xr.v[j], dacc1[j]);
-        } else {
-          dacc[j] = fma_((double)w.v[j], (double)rr.v[j], dacc[j]);
-        }
-      }
+      for (int j = 0; j < V; ++j) dacc[j] = fma_((double)w.v[j], (double)rr.v[j], dacc[j]);
     }
   }
   if constexpr (MODE == kKpm) {
@@ -188,24 +180,19 @@ __global__ __launch_bounds__(kWG) void k_cheb_mask(
     // and lane, see mask_launch), so the moments have the CSR kernel's bits
     static_assert(kWG % L == 0, "KPM blocks need B/V | 256");
     __shared__ double s_red[kWG * V];
-    constexpr int W = kpm_dots(B, sizeof(VT) == 4);
 #pragma unroll
-    for (int h = 0; h < W / B; ++h) {
-      if (h) __syncthreads();
+    for (int j = 0; j < V; ++j) s_red[tid * V + j] = dacc[j];
+    __syncthreads();
+    for (int st = NG / 2; st > 0; st >>= 1) {
+      if (grp < st) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) s_red[tid * V + j] = h ? dacc1[j] : dacc[j];
+        for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
+      }
       __syncthreads();
-      for (int st = NG / 2; st > 0; st >>= 1) {
-        if (grp < st) {
+    }
+    if (grp == 0) {
 #pragma unroll
-          for (int j = 0; j < V; ++j) s_red[tid * V + j] += s_red[(tid + st * L) * V + j];
-        }
-        __syncthreads();
-      }
-      if (grp == 0) {
-#pragma unroll
-        for (int j = 0; j < V; ++j) part[(size_t)blk * W + h * B + c0 + j] = s_red[tid * V + j];
-      }
+      for (int j = 0; j < V; ++j) part[(size_t)blk * B + c0 + j] = s_red[tid * V + j];
     }
   }
 }
