@@ -269,7 +269,8 @@ namespace {
 // LanDos), enqueued without waiting: step j forms V(:, j+1) from V(:, 0..j) and
 // leaves alpha_j, ||w||^2 and ||w|| in device arrays.  The host looks at them
 // after the steps it asked for; a step past one where the recurrence ended has
-// computed nothing that is used.  Up to `slots` runs from different vectors
+// computed nothing that is used (a user's operator is asked for a step at a time,
+// since it would be called with what that step divides by).  Up to `slots` runs from different vectors
 // advance together, a column each of the step's launches, A applied to all of
 // them as one interleaved block; the bits of a run do not depend on the others.
 struct MgsChain {
@@ -663,11 +664,18 @@ int LanBounds(int msteps, double* vin, double* lmin, double* lmax) {
   double nv;
   if (int e = nrm2_dev(n, v, &nv)) return e;
   EVSL_HIP(evsl_dev::scal_copy(n, 1.0 / nv, v, ch.col(0, 0), c.stream));
-  if (int e = ch.run(0, msteps)) return e;
-  if (int e = ch.read(sc, 0)) return e;
+  const bool ahead = c.op == 1;
+  if (ahead) {
+    if (int e = ch.run(0, msteps)) return e;
+    if (int e = ch.read(sc, 0)) return e;
+  }
   const int m0 = msteps;
   double wn = 0.0;
   for (int j = 0; j < msteps; ++j) {
+    if (!ahead) {
+      if (int e = ch.run(j, j + 1)) return e;
+      if (int e = ch.read(sc, 0)) return e;
+    }
     alp[j] = sc[j];
     bet[j] = sc[m0 + j];
     wn += alp[j] * alp[j];
@@ -729,6 +737,7 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
   MgsChain ch;
   if (int e = ch.init(n, msteps, slots)) return e;
   const int m0 = msteps;
+  const bool ahead = c.op == 1;
   int have = 0, next = 0, group = 1;  // runs of the current group, the next one to look at
   for (int m = 0; m < nvec; ++m) {
     if (next == have) {
@@ -746,16 +755,22 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
                            hipMemcpyHostToDevice));
       drawn.erase(drawn.begin(), drawn.begin() + have);
       if (int e = ch.start(0, have)) return e;
-      if (int e = ch.run(0, msteps, 0, have)) return e;
-      // the next group's draws while the device runs this one
-      const int left = nvec - m - have;
-      if (left > 0) draw(size_of(left));
+      if (ahead) {
+        if (int e = ch.run(0, msteps, 0, have)) return e;
+        // the next group's draws while the device runs this one
+        const int left = nvec - m - have;
+        if (left > 0) draw(size_of(left));
+      }
       if (int e = ch.read(sc, 0, have)) return e;
     }
     const int s = next++;
     const double* scs = sc.data() + s * ch.nscal();
     double wn = 0.0;
     for (int j = 0; j < msteps; ++j) {
+      if (!ahead) {
+        if (int e = ch.run(j, j + 1, s)) return e;
+        if (int e = ch.read(sc, s)) return e;
+      }
       alp[j] = scs[j];
       bet[j] = scs[m0 + j];
       wn += alp[j] * alp[j];
@@ -788,8 +803,10 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
         bet[j] = 0;
         const double zero = 0.0;
         EVSL_HIP(hipMemcpy(ch.b(j, s), &zero, sizeof(double), hipMemcpyHostToDevice));
-        if (int e = ch.run(j + 1, msteps, s)) return e;
-        if (int e = ch.read(sc, s)) return e;
+        if (ahead) {
+          if (int e = ch.run(j + 1, msteps, s)) return e;
+          if (int e = ch.read(sc, s)) return e;
+        }
       }
     }
     if (tridiag_eig_host(msteps, alp.data(), bet.data(), ritz.data(), S.data()))
