@@ -543,12 +543,14 @@ hipError_t gather_cols(size_t nrow, int m, const double* src, size_t lds, const 
 // Zsel (k x m, column-major) = the columns cols[0..m) of Z = I * rotations.
 // Sweep s covers rotation indices i = top[s], top[s]-1, ..., top[s]-cnt[s]+1;
 // cs holds the nrot (cosine, sine) pairs of all sweeps one after the other.
-// rotations_rows: rows of Z a block holds in LDS, 0 where one does not fit
-// (k > 6144; the caller then replays on the host).
+// rotations_rows: rows of Z a block holds in LDS; 0 for larger k, whose rotations
+// apply_rotations replays on Z itself (k x k; the caller then gathers the columns).
 int rotations_rows(int k);
 hipError_t replay_rotations(int k, int nsweep, const int* top, const int* cnt, int nrot,
                             const double* cs, int m, const int* cols, double* Zsel,
                             hipStream_t st);
+hipError_t apply_rotations(int k, double* Z, int nsweep, const int* top, const int* cnt,
+                           const double* cs, hipStream_t st);
 
 // block (row-major, B columns) helpers
 // out[c] = ||X(:,c)||^2 partials -> finalised into out (B values)

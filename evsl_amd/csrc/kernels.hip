@@ -632,7 +632,12 @@ __global__ void k_gather_cols(size_t nrow, const double* __restrict__ src, size_
 // ---------------------------------------------------------------------
 constexpr int kRotChunk = 256;                // rotations staged at a time
 constexpr int kRotUnroll = 8;
-constexpr size_t kRotRowBytes = 48u << 10;    // LDS of a block's rows
+// LDS of a block's rows, two of them at least: the blocks of larger k go through
+// the device in rounds, and Z in global memory is faster (a random tridiagonal
+// matrix, LDS / global, ms: k = 331 3.2 / 7.8, 1000 26 / 99, 2000 128 / 389, 3072
+// 807 / 996; with one row a block 3073 1166 / 935, 4200 3236 / 1791, 6144 12203 /
+// 4833).
+constexpr size_t kRotRowBytes = 48u << 10;
 
 template <int RW>
 __global__ __launch_bounds__(64) void k_replay_rotations(
@@ -715,6 +720,49 @@ __global__ __launch_bounds__(64) void k_replay_rotations(
   __syncthreads();
   if (act)
     for (int j = 0; j < m; ++j) Zsel[(size_t)j * k + row] = s_z[(size_t)cols[j] * RW + lane];
+}
+
+// The replay of larger Z: a thread a row, Z (k x k, column-major) in global memory,
+// one sweep at a time.  The rotated pair shares column i with the next rotation, so
+// that value is carried in a register and a rotation costs one load and one store.
+// Bound: that latency, four rotations' loads in flight (k = 7000, 51 million
+// rotations: 6.8 s).
+__global__ __launch_bounds__(kWG) void k_apply_rotations(int k, double* __restrict__ Z,
+                                                         int nsweep, const int* __restrict__ top,
+                                                         const int* __restrict__ cnt,
+                                                         const double2* __restrict__ cs) {
+  const int r = blockIdx.x * kWG + threadIdx.x;
+  if (r >= k) return;
+  const size_t ldz = (size_t)k;
+  const double2* rot = cs;
+  for (int sw = 0; sw < nsweep; ++sw) {
+    const int c = cnt[sw];
+    double* z = Z + (size_t)(top[sw] + 1) * ldz + r;  // column i + 1 of the next rotation
+    double carry = *z;
+    auto one = [&](const double2& q, double zi) {
+      *z = __builtin_fma(q.x, carry, q.y * zi);
+      carry = __builtin_fma(q.x, zi, -(q.y * carry));
+      z -= ldz;
+    };
+    int j = 0;
+    for (; j + 4 <= c; j += 4) {
+      const double z0 = *(z - ldz), z1 = *(z - 2 * ldz), z2 = *(z - 3 * ldz), z3 = *(z - 4 * ldz);
+      one(rot[j], z0);
+      one(rot[j + 1], z1);
+      one(rot[j + 2], z2);
+      one(rot[j + 3], z3);
+    }
+    for (; j < c; ++j) one(rot[j], *(z - ldz));
+    *z = carry;
+    rot += c;
+  }
+}
+
+__global__ void k_set_identity(int k, double* __restrict__ Z) {
+  const size_t tot = (size_t)k * k;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
+       i += (size_t)gridDim.x * blockDim.x)
+    Z[i] = (i % (size_t)(k + 1) == 0) ? 1.0 : 0.0;
 }
 
 // ---------------------------------------------------------------------
@@ -1493,9 +1541,20 @@ hipError_t gather_cols(size_t nrow, int m, const double* src, size_t lds, const 
 }
 
 int rotations_rows(int k) {
-  for (int rw = 16; rw > 0; rw >>= 1)
+  for (int rw = 16; rw > 1; rw >>= 1)
     if ((size_t)rw * k * sizeof(double) <= kRotRowBytes) return rw;
   return 0;
+}
+
+hipError_t apply_rotations(int k, double* Z, int nsweep, const int* top, const int* cnt,
+                           const double* cs, hipStream_t st) {
+  if (k <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_set_identity, dim3(grid_for((size_t)k * k, kWG, 4096)), dim3(kWG), 0, st, k,
+                     Z);
+  if (nsweep > 0)
+    hipLaunchKernelGGL(k_apply_rotations, dim3((k + kWG - 1) / kWG), dim3(kWG), 0, st, k, Z,
+                       nsweep, top, cnt, (const double2*)cs);
+  return hipGetLastError();
 }
 
 hipError_t replay_rotations(int k, int nsweep, const int* top, const int* cnt, int nrot,
@@ -1515,7 +1574,6 @@ hipError_t replay_rotations(int k, int nsweep, const int* top, const int* cnt, i
     EVSL_ROT(8)
     EVSL_ROT(4)
     EVSL_ROT(2)
-    EVSL_ROT(1)
     default:
       return hipErrorInvalidValue;
   }

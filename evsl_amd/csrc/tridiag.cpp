@@ -216,23 +216,7 @@ int tridiag_rotations_to_device(int kdim, const RotationLog& rec, const std::vec
   if (m == 0) return 0;
   std::vector<int> cols(m);
   for (int j = 0; j < m; ++j) cols[j] = rec.perm[sel[j]];
-  if (evsl_dev::rotations_rows(kdim) == 0) {  // a row of Z outgrows a block's LDS
-    std::vector<double> Z((size_t)kdim * m);
-#pragma omp parallel
-    {
-      std::vector<double> z(kdim);
-#pragma omp for schedule(static)
-      for (int r = 0; r < kdim; ++r) {
-        std::fill(z.begin(), z.end(), 0.0);
-        z[r] = 1.0;
-        replay_row(rec, z.data());
-        for (int j = 0; j < m; ++j) Z[(size_t)j * kdim + r] = z[cols[j]];
-      }
-    }
-    EVSL_HIP(hipMemcpy(Zsel_d, Z.data(), Z.size() * sizeof(double), hipMemcpyHostToDevice));
-    return 0;
-  }
-  DevBuf sweeps, cs;
+  DevBuf sweeps, cs, Z;
   const int nrot = (int)(rec.cs.size() / 2);
   std::vector<int> h;  // tops, counts, columns
   h.insert(h.end(), rec.top.begin(), rec.top.end());
@@ -245,8 +229,16 @@ int tridiag_rotations_to_device(int kdim, const RotationLog& rec, const std::vec
     EVSL_HIP(hipMemcpy(cs.p, rec.cs.data(), rec.cs.size() * sizeof(double),
                        hipMemcpyHostToDevice));
   const int* d = sweeps.as<int>();
-  EVSL_HIP(evsl_dev::replay_rotations(kdim, nsw, d, d + nsw, nrot, cs.as<double>(), m, d + 2 * nsw,
-                                      Zsel_d, c.stream));
+  if (evsl_dev::rotations_rows(kdim) > 0) {
+    EVSL_HIP(evsl_dev::replay_rotations(kdim, nsw, d, d + nsw, nrot, cs.as<double>(), m,
+                                        d + 2 * nsw, Zsel_d, c.stream));
+  } else {
+    EVSL_HIP(Z.alloc((size_t)kdim * kdim * sizeof(double)));
+    EVSL_HIP(evsl_dev::apply_rotations(kdim, Z.as<double>(), nsw, d, d + nsw, cs.as<double>(),
+                                       c.stream));
+    EVSL_HIP(evsl_dev::gather_cols(kdim, m, Z.as<double>(), kdim, d + 2 * nsw, Zsel_d, kdim,
+                                   c.stream));
+  }
   EVSL_HIP(hipStreamSynchronize(c.stream));
   return 0;
 }
