@@ -123,9 +123,42 @@ int upload(DevBuf& d, const void* src, size_t bytes) {
   return 0;
 }
 
-size_t dos_mem(const SrvMatrix& m, bool f32) {
-  const size_t vs = f32 ? 4 : 8;
-  return (size_t)m.M.n * 32 * (4 * vs + 8) + (size_t)m.M.n * 8;
+// A density's column block of B columns: its row blocks, the degrees its partials
+// hold, the blocks of the first level of their sums
+struct DosBlock {
+  int nblk = 0, nd = 1, G = 1;
+};
+int dos_block(const DevMatrix& M, bool f32, int B, int Mdeg, DosBlock* d) {
+  const int V = evsl_dev::cheb_spmm_vec(B, f32, evsl_dev::kKpm);
+  const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
+  const int slot = V > 0 && R > 0 ? evsl_dev::width_slot(B / V / R) : -1;
+  if (slot < 0) return EVSL_ERR_ARG;
+  d->nblk = M.nblk[slot];
+  d->nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees((size_t)d->nblk * B), Mdeg));
+  d->G = evsl_dev::sum_levels_blocks(d->nblk, B);
+  return 0;
+}
+
+// columns of the next block of a density of which `left` vectors are to come
+int dos_width(const DevMatrix& M, bool f32, int left) {
+  int B = evsl_dev::kpm_max_width(M.n, !f32 && M.regular);
+  while (B > left) B >>= 1;
+  return B;
+}
+
+// device memory of a density: its vector blocks, a share of x64, the dots, and the
+// partials and their sums, which a later, narrower block may have more of
+size_t dos_mem(const DevMatrix& M, bool f32, int Mdeg, int nvec) {
+  const size_t n = M.n, vs = f32 ? 4 : 8;
+  size_t part = 0, scratch = 0, first = 0;
+  for (int B = dos_width(M, f32, nvec); B > 0; B >>= 1) {
+    DosBlock d;
+    if (dos_block(M, f32, B, Mdeg, &d)) continue;
+    first = std::max(first, (size_t)B);
+    part = std::max(part, (size_t)d.nd * std::max(d.nblk, 1) * B);
+    if (d.G > 1) scratch = std::max(scratch, (size_t)d.nd * d.G * B);
+  }
+  return first * n * (4 * vs + 8) + (part + scratch + first * (Mdeg + 1)) * sizeof(double);
 }
 
 // starts the next column block of a DOS request: seeded start vectors
@@ -135,17 +168,14 @@ int dos_round(evslAmdServer* s, SrvRequest& q) {
   SrvMatrix& m = *s->mats[q.mat];
   const bool f32 = s->mixed;
   const size_t vs = f32 ? 4 : 8;
-  int B = evsl_dev::kpm_max_width(m.M.n, !f32 && m.M.regular);
-  while (B > q.nvec - q.done_vec) B >>= 1;
+  const int B = dos_width(m.M, f32, q.nvec - q.done_vec);
+  DosBlock d;
+  if (int e = dos_block(m.M, f32, B, q.Mdeg, &d)) return e;
   q.B = B;
   q.k = 0;
-  const int V = evsl_dev::cheb_spmm_vec(B, f32, evsl_dev::kKpm);
-  const int R = evsl_dev::cheb_spmm_rows(B, f32, evsl_dev::kKpm);
-  const int slot = evsl_dev::width_slot(B / V / R);
-  if (slot < 0) return EVSL_ERR_ARG;
-  q.nblk = m.M.nblk[slot];
-  q.nd = std::max(1, std::min(evsl_dev::kpm_sum_degrees((size_t)q.nblk * B), q.Mdeg));
-  q.G = evsl_dev::sum_levels_blocks(q.nblk, B);
+  q.nblk = d.nblk;
+  q.nd = d.nd;
+  q.G = d.G;
   const int n = m.M.n;
   const size_t nb = (size_t)n * B;
   EVSL_HIP(q.x0.alloc(nb * vs));
@@ -509,7 +539,7 @@ int evsl_amd_server_submit_dos(evslAmdServer* s, int mat, double a, double b, in
   q->nvec = nvec;
   q->vec_kind = vec_kind;
   q->seed = seed;
-  q->mem = dos_mem(*s->mats[mat], s->mixed);
+  q->mem = dos_mem(s->mats[mat]->M, s->mixed, Mdeg, nvec);
   s->queue.push_back(q->id);
   s->reqs.push_back(std::move(q));
   return s->reqs.back()->id;
