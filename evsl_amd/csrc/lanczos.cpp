@@ -304,6 +304,9 @@ struct MgsChain {
     }
     return 0;
   }
+  void release() {
+    for (DevBuf* d : {&V, &scal, &G, &h, &gt, &part, &xi, &wi}) d->release();
+  }
   // step j of the runs s0 .. s0 + cnt - 1
   evsl_dev::LanCols cols(int j, int s0, int cnt) const {
     evsl_dev::LanCols c{};
@@ -735,7 +738,14 @@ int LanDos(const int nvec, int msteps, int npts, double* xdos, double* ydos, dou
     }
   };
   MgsChain ch;
-  if (int e = ch.init(n, msteps, slots)) return e;
+  // as many runs as there is memory for (the bits of a run do not depend on it)
+  while (int e = ch.init(n, msteps, slots)) {
+    if (slots == 1) return e;
+    slots /= 2;
+    ch.release();
+    (void)hipGetLastError();
+    clear_error();
+  }
   const int m0 = msteps;
   const bool ahead = c.op == 1;
   int have = 0, next = 0, group = 1;  // runs of the current group, the next one to look at
