@@ -292,19 +292,22 @@ bool cheb_spmm_streaming(const Csr& A, int B, bool fp32, Mode mode);
 // instead of 2.1e-16 on a 64 x 60 grid, 3.8e-16 instead of 1.0e-16 on 5,000 random
 // rows, and with exact dots still more than v.T_k v.
 
-// Columns of a KPM block: 32, or fewer where the four FP64 vector blocks of a step
-// at 32 columns outgrow 256 MB, the Infinity Cache (n > 250,000), and the rows are
-// regular (a row has its neighbour's column offsets, so a gather reads contiguous
-// segments and the matrix is a small part of a step): 16 while that keeps them
-// under it, else 8.  The blocks then stay there from step to step (us per column
-// and step at 32 / 16 / 8 columns, row-mask kernel, CSR kernel: 58^3 1.0 / 1.1 /
-// 1.3, 1.1 / 1.4 / 1.8; 68^3 2.3 / 1.6 / 1.9, 2.5 / 2.0 / 2.5; 90^3 5.5 / 5.6 /
-// 3.5, 5.8 / 6.2 / 4.6; 100^3 7.4 / 7.5 / 5.6, 7.9 / 8.3 / 8.4); irregular rows pay
-// for their gathers by the segment, so wider is better (131,072 random rows of
-// 3-70: 5.4 / 5.1 / 7.1).  One rule for every KPM path: moments depend on the width.
+// Columns of a KPM block.  Regular rows (a row has its neighbour's column offsets, so
+// a gather reads contiguous segments and the matrix is a small part of a step): the
+// most of 32, 16 and 8 whose four FP64 vector blocks fit the 256 MB Infinity Cache,
+// where they then stay from step to step, and 16 where none does (60 moments of 32
+// vectors, ms, at 32 / 16 / 8 columns, row-mask kernel, CSR kernel: 58^3 3.0 / 2.9 /
+// 3.0, 3.2 / 3.5 / 4.0; 68^3 5.4 / 3.9 / 4.9, 5.7 / 4.7 / 6.0; 90^3 11.6 / 11.5 / 8.4,
+// 12.2 / 12.6 / 10.4; 100^3 15.4 / 15.5 / 12.6, 16.4 / 16.9 / 17.5; 107^3 19.0 / 18.9 /
+// 18.8, 19.9 / 20.8 / 22.6; 126^3 30.7 / 29.9 / 29.3, 32.2 / 32.8 / 34.7; 160^3 72.4 /
+// 60.0 / 59.6, 75.7 / 65.7 / 69.7).  Irregular rows pay for their gathers by the
+// segment: 32 (131,072 random rows of 3-70, us a column and step 5.4 / 5.1 / 7.1).
+// One rule for every KPM path: moments depend on the width.
 inline int kpm_max_width(int n, bool regular) {
-  if (!regular || 32.0 * n * 32 <= 256e6) return 32;
-  return 32.0 * n * 16 <= 256e6 ? 16 : 8;
+  if (!regular) return 32;
+  for (int B : {32, 16, 8})
+    if (32.0 * n * B <= 256e6) return B;
+  return 16;
 }
 
 // degrees whose block partials are kept and then summed by one launch: the
