@@ -39,14 +39,15 @@ def profiled_traffic(kname):
     summary (rocprofv3 FETCH_SIZE and WRITE_SIZE, scaled by the factors a
     copy kernel of known size gives), or None if it was not profiled."""
     import re
-    path = os.path.join(ROOT, "profiles", "k_cheb_spmm_pmc_lap3d100.md")
-    if not os.path.exists(path):
-        return None
     pat = re.compile(r"^\|\s*`([^`]+)`\s*\|\s*([\d.]+)\s*\|\s*([\d.]+)\s*\|\s*([\d.]+)\s*\|")
-    for line in open(path):
-        m = pat.match(line)
-        if m and m.group(1).strip() == kname:
-            return float(m.group(4))
+    for name in ("filter_pmc.md", "k_cheb_spmm_pmc_lap3d100.md"):
+        path = os.path.join(ROOT, "profiles", name)
+        if not os.path.exists(path):
+            continue
+        for line in open(path):
+            m = pat.match(line)
+            if m and m.group(1).strip() == kname:
+                return float(m.group(4))
     return None
 
 
@@ -817,8 +818,9 @@ def main():
                         if (b, pr, md) != (B, prec, 1):
                             assert ev.set_spmm_layout(b, pr, md, 0) == 0
         out = {}
-        for tag, (b, pr, mode) in {"filter": (B, prec, 1), "refine": (32, prec, 3),
-                                   "kpm": (32, PREC_FP64, 2)}.items():
+        for tag, (b, pr, mode) in {"filter": (B, prec, 1), "refine": (8, prec, 3),
+                                   "kpm": (8, PREC_FP64, 2),
+                                   "plain": (1, PREC_FP64, 1)}.items():
             err, ms, by = ev.bench_filter(b, pr, mode, 50, cc, dd)
             out[tag] = {"kernel": ev.spmm_kernel_name(b, pr, mode),
                         "launch_ms": ms, "bytes_per_launch": by,
