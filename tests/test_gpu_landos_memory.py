@@ -34,12 +34,14 @@ def test_fewer_runs_where_memory_is_short(ev, libc):
         return x, y, cnt
 
     ref = run()
-    held = []
+    held, piece = [], 16 * GB
     try:
-        while (room := free_bytes(ev) - 3 * one) > GB // 4:
-            p = ev.lib._evsl_Malloc_device(min(room, 16 * GB))
-            assert p, ev.last_error()
-            held.append(p)
+        while (room := free_bytes(ev) - 3 * one) > GB // 4 and piece > GB // 16:
+            p = ev.lib._evsl_Malloc_device(min(room, piece))
+            if p:
+                held.append(p)
+            else:
+                piece //= 2
         got = run()
     finally:
         for p in held:
