@@ -41,6 +41,7 @@ def test_fewer_runs_where_memory_is_short(ev, libc):
             if p:
                 held.append(p)
             else:
+                ev.lib.hipGetLastError()
                 piece //= 2
         got = run()
     finally:
