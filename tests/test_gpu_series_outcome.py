@@ -71,6 +71,27 @@ def test_series_run_and_fail(series, n, offsets):
         ev.free_pol(p)
 
 
+@pytest.mark.parametrize("L", [5, 16, 31, 40])
+def test_series_run_on_lattices(series, L):
+    # rows of six entries out of twelve pairs; columns that take turns on an XCD
+    ev = series
+    A = M.anderson(L, 16.5, seed=L)
+    assert ev.set_matrix(A) == 0, ev.last_error()
+    pols = filters(ev, A, 33)
+    X = np.random.default_rng(5).uniform(-1.0, 1.0, (A.n, 33))
+    for prec in (PREC_FP64, PREC_MIXED):
+        ref, _, _ = run(ev, pols, X, prec, 0)
+        for cols in (1, 16, 33):
+            Y, launched, failed = run(ev, pols[:cols], X[:, :cols], prec)
+            assert (launched, failed) == (-(-cols // 16), 0)
+            assert np.array_equal(Y, ref[:, :cols])
+        if L > 5:
+            Y, launched, failed = run(ev, pols, X, prec, 1)
+            assert launched == 3 and failed > 0 and np.array_equal(Y, ref)
+    for p in pols:
+        ev.free_pol(p)
+
+
 def test_a_failure_lasts_until_the_next_start(series):
     ev = series
     A = sym_band(5000, [1, 70], seed=1)
